@@ -105,17 +105,19 @@ HostOps fr_operators() {
     return o;
 }
 
-double cfl_dt_from_state(const double* h, int64_t NP, double dx, double dy, double dz, double cfl) {
+od_status cfl_dt_of_state(const void* u, int u_real, int64_t E, double dx, double dy, double dz, double cfl,
+                          double* partial, hipStream_t stream, double* dt_out) {
+    const int rc = u_real == OD_F32 ? od::launch_cfl<float>((const float*)u, partial, E, dx, dy, dz, stream)
+                                    : od::launch_cfl<double>((const double*)u, partial, E, dx, dy, dz, stream);
+    if (rc) return fail(OD_ERR_HIP, "od_cfl_kernel launch failed");
+    double h[od::kCflGroups];
+    const int groups = od::cfl_groups(E);
+    HIP_TRY(hipMemcpyAsync(h, partial, groups * sizeof(double), hipMemcpyDeviceToHost, stream));
+    HIP_TRY(hipStreamSynchronize(stream));
     double lam = 0.0;
-    for (int64_t q = 0; q < NP; ++q) {
-        double r = h[q], ru = h[NP + q], rv = h[2 * NP + q], rw = h[3 * NP + q], e = h[4 * NP + q];
-        double ke = 0.5 * (ru * ru + rv * rv + rw * rw) / r;
-        double pp = std::fmax(1e-7, 0.4 * (e - ke));
-        double cs = std::sqrt(1.4 * pp / r);
-        double l = (std::fabs(ru / r) + cs) / dx + (std::fabs(rv / r) + cs) / dy + (std::fabs(rw / r) + cs) / dz;
-        lam = std::fmax(lam, l);
-    }
-    return (double)(float)(cfl / (7.0 * lam));
+    for (int q = 0; q < groups; ++q) lam = std::fmax(lam, h[q]);
+    *dt_out = (double)(float)(cfl / (7.0 * lam));
+    return OD_OK;
 }
 
 }  // namespace od::host
@@ -124,11 +126,15 @@ using namespace od::host;
 
 namespace {
 
+constexpr double kTableDt = 0.0;  // no dt of its own: c * dt from od_ctx::dt_table
+
 template <class UT, class CT>
 od::StageArgs<UT, CT> stage_args(od_ctx* c, int stage, double dt) {
     od::StageArgs<UT, CT> a = make_stage_args<UT, CT>(c->p, c->p.nx, c->p.ny, c->p.nz, c->p.lx, c->p.ly, c->p.lz,
                                                       c->u, c->tr, c->fv, c->dbg, stage, dt);
     a.mu_t = c->mu_t_on ? (const CT*)c->mu_t : nullptr;
+    // a captured step (dt 0) reads c * dt from the context's table
+    if (dt == kTableDt) a.dt = (const od::StageDt<UT, CT>*)c->dt_table + stage;
     return a;
 }
 
@@ -185,11 +191,11 @@ od_status enqueue_step(od_ctx* c, double dt) {
 // 8-step graph plus n % 8 of the one-step graph (same kernels, same order).
 constexpr uint32_t kStepsPerGraph = 8;
 
-od_status capture_steps(od_ctx* c, double dt, uint32_t steps, hipGraphExec_t* out) {
+od_status capture_steps(od_ctx* c, uint32_t steps, hipGraphExec_t* out) {
     hipGraph_t g = nullptr;
     HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     od_status s = OD_OK;
-    for (uint32_t q = 0; q < steps && s == OD_OK; ++q) s = enqueue_step(c, dt);
+    for (uint32_t q = 0; q < steps && s == OD_OK; ++q) s = enqueue_step(c, kTableDt);
     hipError_t e = hipStreamEndCapture(c->stream, &g);
     if (s != OD_OK) {
         if (g) (void)hipGraphDestroy(g);
@@ -206,24 +212,52 @@ od_status capture_steps(od_ctx* c, double dt, uint32_t steps, hipGraphExec_t* ou
     return OD_OK;
 }
 
-od_status ensure_graph(od_ctx* c, double dt) {
-    if (c->graph && c->graph_k && c->graph_dt == dt && c->graph_mu_t == c->mu_t_on) return OD_OK;
-    for (hipGraphExec_t* gx : {&c->graph, &c->graph_k}) {
-        if (*gx) {
-            HIP_TRY(hipGraphExecDestroy(*gx));
-            *gx = nullptr;
-        }
+template <class UT, class CT>
+int write_dt(od_ctx* c, double dt) {
+    od::StageDt<UT, CT> v[3];
+    for (int s = 0; s < 3; ++s) {
+        v[s].cc = stage_dt_coef<CT>(s, dt);
+        v[s].uc = stage_dt_coef<UT>(s, dt);
     }
-    od_status s = capture_steps(c, dt, 1, &c->graph);
-    if (s == OD_OK) s = capture_steps(c, dt, kStepsPerGraph, &c->graph_k);
-    if (s != OD_OK) return s;
-    c->graph_dt = dt;
-    c->graph_mu_t = c->mu_t_on;
+    return od::launch_set_dt<UT, CT>((od::StageDt<UT, CT>*)c->dt_table, v, c->stream);
+}
+
+// The dt of the steps enqueued from here on, written in stream order (steps
+// already enqueued keep theirs).
+od_status set_dt(od_ctx* c, double dt) {
+    if (c->table_dt == dt) return OD_OK;
+    const bool uf = c->p.u_real == OD_F32, cf = c->p.compute_real == OD_F32;
+    const int rc = uf ? (cf ? write_dt<float, float>(c, dt) : write_dt<float, double>(c, dt))
+                      : (cf ? write_dt<double, float>(c, dt) : write_dt<double, double>(c, dt));
+    if (rc) {
+        c->table_dt = 0.0;
+        return fail(OD_ERR_HIP, "od_set_dt_kernel launch failed");
+    }
+    c->table_dt = dt;
     return OD_OK;
 }
 
-// Enqueue n steps of the captured graphs on the library stream.
-od_status launch_steps(od_ctx* c, uint32_t n) {
+// The one-step graph or the kStepsPerGraph-step one, captured when first needed.
+od_status ensure_graph(od_ctx* c, bool multi) {
+    if (c->graph_mu_t != c->mu_t_on) {
+        for (hipGraphExec_t* gx : {&c->graph, &c->graph_k}) {
+            if (*gx) {
+                HIP_TRY(hipGraphExecDestroy(*gx));
+                *gx = nullptr;
+            }
+        }
+        c->graph_mu_t = c->mu_t_on;
+    }
+    hipGraphExec_t* gx = multi ? &c->graph_k : &c->graph;
+    return *gx ? OD_OK : capture_steps(c, multi ? kStepsPerGraph : 1, gx);
+}
+
+// Enqueue n steps of size dt of the captured graphs on the library stream.
+od_status launch_steps(od_ctx* c, double dt, uint32_t n) {
+    od_status s = set_dt(c, dt);
+    if (s == OD_OK && n >= kStepsPerGraph) s = ensure_graph(c, true);
+    if (s == OD_OK && n % kStepsPerGraph) s = ensure_graph(c, false);
+    if (s != OD_OK) return s;
     uint32_t q = 0;
     for (; q + kStepsPerGraph <= n; q += kStepsPerGraph) HIP_TRY(hipGraphLaunch(c->graph_k, c->stream));
     for (; q < n; ++q) HIP_TRY(hipGraphLaunch(c->graph, c->stream));
@@ -311,7 +345,9 @@ od_status od_create(const od_params* p, int device, od_ctx** out) {
     for (int q = 0; q < 3 && ok; ++q) ok = dmalloc(&c->tr[q], tr_bytes);
     ok = ok && (!p->viscous || dmalloc(&c->fv, fv_bytes));
     ok = ok && dmalloc((void**)&c->sums_partial, (size_t)5 * E * sizeof(double)) &&
-         dmalloc((void**)&c->sums_out, 8 * sizeof(double));
+         dmalloc((void**)&c->sums_out, 8 * sizeof(double)) &&
+         dmalloc((void**)&c->cfl_partial, od::kCflGroups * sizeof(double)) &&
+         dmalloc(&c->dt_table, 3 * sizeof(od::StageDt<double, double>));
     if (!ok) return cleanup(fail(OD_ERR_NOMEM, "device allocation failed"));
     for (int q = 0; q < 3; ++q)
         if (hipHostMalloc(&c->pinned[q], state_bytes, hipHostMallocDefault) != hipSuccess ||
@@ -336,6 +372,8 @@ void od_destroy(od_ctx* c) {
     if (c->dbg) (void)hipFree(c->dbg);
     if (c->sums_partial) (void)hipFree(c->sums_partial);
     if (c->sums_out) (void)hipFree(c->sums_out);
+    if (c->cfl_partial) (void)hipFree(c->cfl_partial);
+    if (c->dt_table) (void)hipFree(c->dt_table);
     od_closure_release_internal(c);
     for (int q = 0; q < 3; ++q) {
         if (c->pinned[q]) (void)hipHostFree(c->pinned[q]);
@@ -453,13 +491,13 @@ od_status od_step(od_ctx* c, double dt, uint32_t n_steps) {
     if (!c->state_set) return fail(OD_ERR_STATE, "od_step: state not set");
     if (!(dt > 0.0) || !std::isfinite(dt)) return fail(OD_ERR_INVALID, "od_step: dt must be positive and finite");
     HIP_TRY(hipSetDevice(c->device));
-    od_status s = ensure_graph(c, dt);
-    if (s != OD_OK) return s;
+    od_status s = OD_OK;
     if (!c->mlp) {
-        s = launch_steps(c, n_steps);
+        s = launch_steps(c, dt, n_steps);
         if (s == OD_OK) c->steps_done += n_steps;
         return s;
     }
+    if ((s = set_dt(c, dt)) != OD_OK || (s = ensure_graph(c, false)) != OD_OK) return s;
     for (uint32_t q = 0; q < n_steps; ++q) {  // the closure refreshes mu_t between steps
         if (c->steps_done % (uint64_t)c->closure.update_interval == 0) {
             s = od_closure_update_internal(c, dt * c->closure.update_interval);
@@ -516,25 +554,24 @@ od_status od_conservation_sums(od_ctx* c, double out[5]) {
 od_status od_cfl_dt(od_ctx* c, double cfl, double* dt_out) {
     if (!c || !dt_out) return fail(OD_ERR_INVALID, "od_cfl_dt: null argument");
     if (!(cfl > 0.0)) return fail(OD_ERR_INVALID, "od_cfl_dt: cfl must be positive");
-    const size_t n = (size_t)5 * c->NP;
-    std::vector<double> h(n);
-    od_status s = od_get_state(c, h.data(), n, OD_F64);
-    if (s != OD_OK) return s;
-    *dt_out = cfl_dt_from_state(h.data(), c->NP, c->p.lx / c->p.nx, c->p.ly / c->p.ny, c->p.lz / c->p.nz, cfl);
-    return OD_OK;
+    HIP_TRY(hipSetDevice(c->device));
+    return cfl_dt_of_state(c->u[0], c->p.u_real, c->E, c->p.lx / c->p.nx, c->p.ly / c->p.ny, c->p.lz / c->p.nz, cfl,
+                           c->cfl_partial, c->stream, dt_out);
 }
 
 od_status od_time_steps(od_ctx* c, double dt, uint32_t n_steps, double* ms_total) {
     if (!c || !ms_total) return fail(OD_ERR_INVALID, "od_time_steps: null argument");
     if (!c->state_set) return fail(OD_ERR_STATE, "od_time_steps: state not set");
     HIP_TRY(hipSetDevice(c->device));
-    od_status s = ensure_graph(c, dt);
+    od_status s = launch_steps(c, dt, 0);  // its dt, before the clock starts
+    if (s == OD_OK && n_steps >= kStepsPerGraph) s = ensure_graph(c, true);
+    if (s == OD_OK && n_steps % kStepsPerGraph) s = ensure_graph(c, false);
     if (s != OD_OK) return s;
     hipEvent_t a, b;
     HIP_TRY(hipEventCreate(&a));
     HIP_TRY(hipEventCreate(&b));
     HIP_TRY(hipEventRecord(a, c->stream));
-    s = launch_steps(c, n_steps);
+    s = launch_steps(c, dt, n_steps);
     if (s != OD_OK) {
         (void)hipEventDestroy(a);
         (void)hipEventDestroy(b);

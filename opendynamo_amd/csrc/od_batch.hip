@@ -36,6 +36,7 @@ struct od_batch {
     size_t table_bytes = 0;
     double* sums_partial = nullptr;
     double* sums_out = nullptr;
+    double* cfl_partial = nullptr;  // od::kCflGroups doubles
     HostOps ops;
     std::vector<char> state_set;
     od_schedule sched{0, 1, 0, 0};
@@ -468,7 +469,8 @@ od_status od_batch_create(const od_params* p, const od_box* boxes, int32_t n_box
     b->table_bytes = (size_t)n_boxes * sizeof(od::BoxDev<double, double>);
     ok = ok && dmalloc(&b->table, b->table_bytes);
     ok = ok && dmalloc((void**)&b->sums_partial, (size_t)5 * max_box * sizeof(double)) &&
-         dmalloc((void**)&b->sums_out, 8 * sizeof(double));
+         dmalloc((void**)&b->sums_out, 8 * sizeof(double)) &&
+         dmalloc((void**)&b->cfl_partial, od::kCflGroups * sizeof(double));
     if (!ok) return cleanup(fail(OD_ERR_NOMEM, "device allocation failed"));
     *out = b;
     return OD_OK;
@@ -487,6 +489,7 @@ void od_batch_destroy(od_batch* b) {
     if (b->table) (void)hipFree(b->table);
     if (b->sums_partial) (void)hipFree(b->sums_partial);
     if (b->sums_out) (void)hipFree(b->sums_out);
+    if (b->cfl_partial) (void)hipFree(b->cfl_partial);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
 }
@@ -566,13 +569,13 @@ od_status od_batch_synchronize(od_batch* b) {
 od_status od_batch_cfl_dt(od_batch* b, double cfl, double* dt_out) {
     if (!b || !dt_out) return fail(OD_ERR_INVALID, "od_batch_cfl_dt: null argument");
     if (!(cfl > 0.0)) return fail(OD_ERR_INVALID, "od_batch_cfl_dt: cfl must be positive");
+    HIP_TRY(hipSetDevice(b->device));
     for (size_t i = 0; i < b->boxes.size(); ++i) {
         const od_box& x = b->boxes[i];
-        const int64_t NP = (int64_t)64 * x.nx * x.ny * x.nz;
-        std::vector<double> h((size_t)5 * NP);
-        od_status s = od_batch_get_state(b, (int32_t)i, h.data(), h.size(), OD_F64);
+        const unsigned char* u = (const unsigned char*)b->u[0] + (size_t)320 * b->e_off[i] * b->ubytes;
+        od_status s = cfl_dt_of_state(u, b->p.u_real, (int64_t)x.nx * x.ny * x.nz, x.lx / x.nx, x.ly / x.ny,
+                                      x.lz / x.nz, cfl, b->cfl_partial, b->stream, dt_out + i);
         if (s != OD_OK) return s;
-        dt_out[i] = cfl_dt_from_state(h.data(), NP, x.lx / x.nx, x.ly / x.ny, x.lz / x.nz, cfl);
     }
     return OD_OK;
 }

@@ -19,13 +19,15 @@ struct od_ctx {
     void* dbg = nullptr;
     double* sums_partial = nullptr;
     double* sums_out = nullptr;
+    double* cfl_partial = nullptr;  // od::kCflGroups doubles
     od::host::HostOps ops;
     bool state_set = false;
     bool blocks = false;               // step kernels on 2x2x2-element blocks (fast f32, even dims),
                                        // which store the traces of the blocks' external faces only
     hipGraphExec_t graph = nullptr;    // one RK3 step
     hipGraphExec_t graph_k = nullptr;  // kStepsPerGraph RK3 steps
-    double graph_dt = 0.0;
+    void* dt_table = nullptr;          // StageDt[3] that the graphs' kernels read
+    double table_dt = 0.0;             // the dt it holds (in stream order), 0: none yet
     void* pinned[3] = {nullptr, nullptr, nullptr};
     hipEvent_t slot_done[3] = {nullptr, nullptr, nullptr};
     // Device copies of the snapshots (allocated at the first snapshot): the

@@ -114,8 +114,10 @@ od::StageArgs<UT, CT> make_stage_args(const od_params& p, int nx, int ny, int nz
     return a;
 }
 
-// dt = cfl / ((2P+1) max_points sum_d (|u_d| + c) / dx_d), rounded to f32,
-// from an f64 state [5][NP].
-double cfl_dt_from_state(const double* h, int64_t NP, double dx, double dy, double dz, double cfl);
+// dt = cfl / ((2P+1) max_points sum_d (|u_d| + c) / dx_d), rounded to f32, of a
+// state [5][64 E] on the device; partial: od::kCflGroups doubles there.  Waits
+// for the stream.
+od_status cfl_dt_of_state(const void* u, int u_real, int64_t E, double dx, double dy, double dz, double cfl,
+                          double* partial, hipStream_t stream, double* dt_out);
 
 }  // namespace od::host

@@ -38,6 +38,15 @@ struct Ops {
     C gR[4];   // g_right'(x_i)
 };
 
+// c * dt of one stage in the compute and the state type.  A captured step
+// graph reads it from device memory, so that a new dt leaves the graph valid
+// (capturing and instantiating it again takes milliseconds).
+template <class UT, class CT>
+struct StageDt {
+    CT cc;
+    UT uc;
+};
+
 template <class UT, class CT>
 struct StageArgs {
     const UT* uin;     // state the stage differentiates
@@ -54,6 +63,7 @@ struct StageArgs {
     CT mu, mu_ref, t_ref, s_suth, bf;
     CT ca, cb, cc;     // blend coefficients in the compute type
     UT ua, ub, uc;     // blend coefficients in the state type
+    const StageDt<UT, CT>* dt;  // cc and uc from here (null: as given above)
 };
 
 // Copy the FR operators to the kernels' constant memory on the current
@@ -113,6 +123,15 @@ int launch_batch_update(const StageArgs<UT, CT>& a, const BatchArgs<UT, CT>& b, 
 // Resident work-groups per CU of a batch kernel (kind 0 visc, 1 update).
 template <class UT, class CT>
 int batch_occupancy(int kind, int pairs, bool visc, int* groups_per_cu);
+// The three stages' c * dt -> table, in stream order.
+template <class UT, class CT>
+int launch_set_dt(StageDt<UT, CT>* table, const StageDt<UT, CT> v[3], void* stream);
+// Largest sum over d of (|u_d| + c) / dx_d of the points of each work-group, in
+// f64, -> partial[groups] (host: their maximum); groups = cfl_groups(n_elem).
+constexpr int kCflGroups = 1024;
+inline int cfl_groups(int64_t n_elem) { return (int)(n_elem < 4 * kCflGroups ? (n_elem + 3) / 4 : kCflGroups); }
+template <class UT>
+int launch_cfl(const UT* u, double* partial, int64_t n_elem, double dx, double dy, double dz, void* stream);
 template <class UT>
 int launch_sums(const UT* u, double* partial, double* out, int64_t n_elem, const double w3[64],
                 double jac, void* stream);

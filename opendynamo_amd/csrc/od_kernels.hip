@@ -1008,6 +1008,15 @@ __device__ __forceinline__ T stream_load(const T* p) { return __builtin_nontempo
 template <class T>
 __device__ __forceinline__ void stream_store(T v, T* p) { __builtin_nontemporal_store(v, p); }
 
+// c * dt of the stage, from device memory where it is given there.  The update
+// kernels read it before the FR correction, whose arithmetic covers the load:
+// at the kernel's start it held up the first loads of the state, 0.1 us a
+// launch, and after the first barrier it took registers for the whole kernel.
+template <class UT, class CT>
+__device__ __forceinline__ StageDt<UT, CT> stage_dt(const StageArgs<UT, CT>& a) {
+    return a.dt ? *a.dt : StageDt<UT, CT>{a.cc, a.uc};
+}
+
 // Face traces of one element (its state tile sUe in LDS) -> dst, the
 // element's kTraceStride block of tr_out.  The element's own wave writes
 // them: 16 lanes per face, 4 faces per pass.  Without BR1 (Euler) the strict
@@ -1326,6 +1335,7 @@ __device__ __forceinline__ void update_body(const StageArgs<UT, CT>& a, const Ti
     __syncthreads();
 
     // FR correction and stage update (rk.cu:12-25, 63-82).
+    const StageDt<UT, CT> cdt = stage_dt(a);
     const CoefTable<CT>& o = coef_lds<CT>();
 #if OD_FAST
     // correction slopes with the Jacobian folded in
@@ -1379,7 +1389,7 @@ __device__ __forceinline__ void update_body(const StageArgs<UT, CT>& a, const Ti
         // in their coefficients, chosen once; uniform branch on the stage
         const CT kA = a.accum_state ? a.ua : a.ca;
         const CT kB = a.accum_state ? a.ub : a.cb;
-        const CT kC = a.accum_state ? a.uc : a.cc;
+        const CT kC = a.accum_state ? cdt.uc : cdt.cc;
         if (a.stage1) {
 #pragma unroll
             for (int v = 0; v < 5; ++v) unew[v] = rk_blend1(kA, kC, uprv[v], rts[v]);
@@ -1393,12 +1403,12 @@ __device__ __forceinline__ void update_body(const StageArgs<UT, CT>& a, const Ti
             const CT rt = rts[v];
             if (!a.accum_state) {
                 CT up = (CT)uprv[v], uc = (CT)ucr[v];
-                CT val = a.stage1 ? (a.ca * up + a.cc * rt) : (a.ca * up + a.cb * uc + a.cc * rt);
+                CT val = a.stage1 ? (a.ca * up + cdt.cc * rt) : (a.ca * up + a.cb * uc + cdt.cc * rt);
                 unew[v] = (UT)val;
             } else {
                 UT rr = (UT)rt;
                 unew[v] =
-                    a.stage1 ? (UT)(a.ua * uprv[v] + a.uc * rr) : (UT)(a.ua * uprv[v] + a.ub * ucr[v] + a.uc * rr);
+                    a.stage1 ? (UT)(a.ua * uprv[v] + cdt.uc * rr) : (UT)(a.ua * uprv[v] + a.ub * ucr[v] + cdt.uc * rr);
             }
         }
     }
@@ -1734,6 +1744,7 @@ __device__ __forceinline__ void update_block_body(const StageArgs<float, float>&
 
     // FR correction and stage update of the wave's element (rk.cu:12-25,
     // 63-82; update_body's fast f32 path).
+    const StageDt<float, float> cdt = stage_dt(a);
     const CoefTable<float>& o = coef_lds<float>();
     const float gLi = o.g[i][0] * a.jx, gRi = o.g[i][1] * a.jx;
     const float gLj = o.g[j][0] * a.jy, gRj = o.g[j][1] * a.jy;
@@ -1778,7 +1789,7 @@ __device__ __forceinline__ void update_block_body(const StageArgs<float, float>&
     // two differ only in their coefficients, chosen once (scalar selects)
     const float kA = a.accum_state ? a.ua : a.ca;
     const float kB = a.accum_state ? a.ub : a.cb;
-    const float kC = a.accum_state ? a.uc : a.cc;
+    const float kC = a.accum_state ? cdt.uc : cdt.cc;
     float unew[5];
     if (a.stage1) {  // uniform branch: each form computes only its own blend
 #pragma unroll
@@ -2206,6 +2217,17 @@ __global__ __launch_bounds__(128 * PAIRS) __attribute__((amdgpu_waves_per_eu(LOO
     }
 }
 
+#if !OD_FAST
+// Sum over d of (|u_d| + c) / dx_d at a point: the signal speed of the CFL condition.
+__device__ __forceinline__ double cfl_signal(double r, double ru, double rv, double rw, double e, double dx, double dy,
+                                             double dz) {
+    const double ke = 0.5 * (ru * ru + rv * rv + rw * rw) / r;
+    const double pp = fmax(1e-7, 0.4 * (e - ke));
+    const double cs = sqrt(1.4 * pp / r);
+    return (fabs(ru / r) + cs) / dx + (fabs(rv / r) + cs) / dy + (fabs(rw / r) + cs) / dz;
+}
+#endif
+
 // Conservation sums: per-element GL-weighted sums (sequential over points),
 // then one block reduces them in a fixed order -> deterministic.
 struct W3 {
@@ -2240,6 +2262,37 @@ __global__ __launch_bounds__(256) void od_sums_final_kernel(const double* partia
         __syncthreads();
     }
 }
+
+#if !OD_FAST
+template <class UT, class CT>
+struct DtTable {
+    StageDt<UT, CT> s[3];
+};
+template <class UT, class CT>
+__global__ void od_set_dt_kernel(StageDt<UT, CT>* table, DtTable<UT, CT> v) {
+    if (threadIdx.x == 0 && blockIdx.x == 0)
+        for (int s = 0; s < 3; ++s) table[s] = v.s[s];
+}
+
+// The largest signal speed of the CFL condition, in f64 from the state's values
+// (the operations that the host used on its copy of the state, so that the dt is
+// the same to the last bit: a maximum does not depend on its order).
+// Reads the state once.
+template <class UT>
+__global__ __launch_bounds__(256) void od_cfl_kernel(const UT* __restrict__ u, double* __restrict__ partial, int64_t E,
+                                                     double dx, double dy, double dz) {
+    __shared__ double red[4];
+    const int64_t NP = E * 64;
+    double lam = 0.0;
+    for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < NP; q += (int64_t)gridDim.x * 256)
+        lam = fmax(lam, cfl_signal((double)u[q], (double)u[NP + q], (double)u[2 * NP + q], (double)u[3 * NP + q],
+                                   (double)u[4 * NP + q], dx, dy, dz));
+    for (int m = 32; m >= 1; m >>= 1) lam = fmax(lam, __shfl_xor(lam, m, 64));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = lam;
+    __syncthreads();
+    if (threadIdx.x == 0) partial[blockIdx.x] = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+}
+#endif
 
 inline int check_launch() { return hipGetLastError() == hipSuccess ? 0 : 1; }
 
@@ -2381,6 +2434,20 @@ int launch_sums(const UT* u, double* partial, double* out, int64_t n_elem, const
 }
 
 #if !OD_FAST
+template <class UT, class CT>
+int launch_set_dt(StageDt<UT, CT>* table, const StageDt<UT, CT> v[3], void* stream) {
+    DtTable<UT, CT> t;
+    for (int s = 0; s < 3; ++s) t.s[s] = v[s];
+    hipLaunchKernelGGL((od_set_dt_kernel<UT, CT>), dim3(1), dim3(64), 0, (hipStream_t)stream, table, t);
+    return check_launch();
+}
+template <class UT>
+int launch_cfl(const UT* u, double* partial, int64_t n_elem, double dx, double dy, double dz, void* stream) {
+    hipLaunchKernelGGL((od_cfl_kernel<UT>), dim3((unsigned)cfl_groups(n_elem)), dim3(256), 0, (hipStream_t)stream, u,
+                       partial, n_elem, dx, dy, dz);
+    return check_launch();
+}
+
 const char* kernel_name(int kind) {
     switch (kind) {
         case 0: return "od_visc_kernel";
@@ -2410,6 +2477,12 @@ OD_INST(float, double)
 #endif
 #undef OD_INST
 #if !OD_FAST
+template int launch_set_dt<float, float>(StageDt<float, float>*, const StageDt<float, float>*, void*);
+template int launch_set_dt<double, float>(StageDt<double, float>*, const StageDt<double, float>*, void*);
+template int launch_set_dt<double, double>(StageDt<double, double>*, const StageDt<double, double>*, void*);
+template int launch_set_dt<float, double>(StageDt<float, double>*, const StageDt<float, double>*, void*);
+template int launch_cfl<float>(const float*, double*, int64_t, double, double, double, void*);
+template int launch_cfl<double>(const double*, double*, int64_t, double, double, double, void*);
 template int launch_sums<float>(const float*, double*, double*, int64_t, const double*, double, void*);
 template int launch_sums<double>(const double*, double*, double*, int64_t, const double*, double, void*);
 #endif
