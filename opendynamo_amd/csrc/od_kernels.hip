@@ -77,6 +77,51 @@ __device__ __forceinline__ C sq(C x) {
     return sqrt(x);
 }
 
+// A denominator that several quotients share.  In the strict build its
+// reciprocal is formed once, in f64 (v_rcp_f64 to 24 bits, then the cubic
+// iteration y (1 + e + e^2), e = 1 - b y: within 2^-52 of 1 / b), and each
+// quotient is the correctly rounded a / b in three or four more instructions:
+//   f32  a y in f64, rounded to f32.  The quotient of two 24-bit numbers lies
+//        2^-49 of itself or more from the middle between two f32 numbers, a y
+//        within 2^-51.5 of it, so the rounding is that of a / b.
+//   f64  q = a y, then one correction with the residual a - b q, exact in an
+//        FMA (Markstein, IBM J. Res. Dev. 34, 1990: the last steps of the
+//        compiler's own a / b).  v_div_fixup gives zeros, infinities and NaN
+//        their IEEE results; |a| between 0 and 2^-969 may be off by one unit
+//        in the last place.
+// A division takes 46 (f32) and 65 (f64) cycles of a SIMD, a quotient 14 and
+// 20, a reciprocal 37; a point has about 90 quotients by some ten
+// denominators, which were nearly half of the strict kernels' instructions.
+template <class C>
+struct Recip {
+    C b;
+    double y;
+};
+template <class C>
+__device__ __forceinline__ Recip<C> recip(C b) {
+#if OD_FAST
+    return {b, 0.0};  // quot takes v_rcp_f32 as dv does
+#else
+    const double d = (double)b, y0 = __builtin_amdgcn_rcp(d);
+    const double e = __builtin_fma(-d, y0, 1.0);
+    const double y = __builtin_fma(__builtin_fma(e, e, e), y0, y0);
+    if constexpr (sizeof(C) == 8) return {b, y};
+    return {b, e == e ? y : y0};  // b zero or infinite: y0 is infinite or zero, and e NaN
+#endif
+}
+template <class C>
+__device__ __forceinline__ C quot(C a, Recip<C> r) {
+#if OD_FAST
+    return a * __builtin_amdgcn_rcpf(r.b);
+#else
+    if constexpr (sizeof(C) == 8) {
+        const double q = a * r.y;
+        return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-r.b, q, a), r.y, q), r.b, a);
+    }
+    return (C)((double)a * r.y);
+#endif
+}
+
 // Fast build: the arithmetic of the point and interface fluxes may fuse a
 // multiply into an add only within one source expression (as the C standard
 // allows), not across statements.  Fusion across statements is decided per
@@ -134,16 +179,16 @@ template <class C>
 __device__ __forceinline__ C gamma_m1() { return ((C)1.4) - ((C)1.0); }
 
 template <class C>
-__device__ __forceinline__ C pressure(C rho, C ru, C rv, C rw, C e) {  // :1-5
+__device__ __forceinline__ C pressure(Recip<C> ir, C ru, C rv, C rw, C e) {  // :1-5
     OD_CONTRACT_IN_EXPRESSIONS
 #if OD_FAST
     if constexpr (sizeof(C) == 4) {  // fast build: the fusions written out
         const C h = ((C)0.5) * __builtin_fmaf(rw, rw, __builtin_fmaf(rv, rv, ru * ru));
-        const C p = gamma_m1<C>() * __builtin_fmaf(-h, __builtin_amdgcn_rcpf(rho), e);
+        const C p = gamma_m1<C>() * __builtin_fmaf(-h, __builtin_amdgcn_rcpf(ir.b), e);
         return fmax(((C)1e-7), p);
     }
 #endif
-    C ke = dv(((C)0.5) * (ru * ru + rv * rv + rw * rw), rho);
+    C ke = quot(((C)0.5) * (ru * ru + rv * rv + rw * rw), ir);
     C p = gamma_m1<C>() * (e - ke);
     return fmax(((C)1e-7), p);
 }
@@ -151,10 +196,11 @@ __device__ __forceinline__ C pressure(C rho, C ru, C rv, C rw, C e) {  // :1-5
 template <class C>
 __device__ __forceinline__ void euler_flux(int d, const C* s, C* f) {  // :7-21
     OD_CONTRACT_IN_EXPRESSIONS
-    C rho = s[0], e = s[4];
-    C p = pressure(rho, s[1], s[2], s[3], e);
+    C e = s[4];
+    const Recip<C> ir = recip(s[0]);
+    C p = pressure(ir, s[1], s[2], s[3], e);
     C md = sel3(s[1], s[2], s[3], d);
-    C ud = dv(md, rho);
+    C ud = quot(md, ir);
     f[0] = md;
 #pragma unroll
     for (int c = 0; c < 3; ++c) f[1 + c] = (c == d) ? s[1 + c] * ud + p : s[1 + c] * ud;
@@ -174,30 +220,31 @@ struct ViscPoint {
     C q[3];
 };
 template <class C>
-__device__ __forceinline__ C heat_flux(int d, const C* s, const C* g, C mu, C rho, C ke, C p) {
+__device__ __forceinline__ C heat_flux(int d, const C* s, const C* g, C mu, Recip<C> ir, Recip<C> irr, C ke, C p) {
     C gd = sel3(g[0], g[1], g[2], d);
     C gu = sel3(g[3], g[4], g[5], d);
     C gv = sel3(g[6], g[7], g[8], d);
     C gw = sel3(g[9], g[10], g[11], d);
     C ge = sel3(g[12], g[13], g[14], d);
-    C dke = dv(s[1] * gu + s[2] * gv + s[3] * gw, rho) - dv(ke * gd, rho);
+    C dke = quot(s[1] * gu + s[2] * gv + s[3] * gw, ir) - quot(ke * gd, ir);
     C dp = gamma_m1<C>() * (ge - dke);
     C coeff = dv(mu * ((C)1.4), ((C)0.72) * gamma_m1<C>());
-    return -coeff * (dv(dp, rho) - dv(p * gd, rho * rho));
+    return -coeff * (quot(dp, ir) - quot(p * gd, irr));
 }
 // dirs: bit d set = the heat flux along d is needed.
 template <class C>
 __device__ __forceinline__ ViscPoint<C> viscous_point(const C* s, const C* g, C mu, int dirs) {
     ViscPoint<C> vp;
     C rho = s[0];
-    vp.u[0] = dv(s[1], rho);
-    vp.u[1] = dv(s[2], rho);
-    vp.u[2] = dv(s[3], rho);
+    const Recip<C> ir = recip(rho), irr = recip(rho * rho);
+    vp.u[0] = quot(s[1], ir);
+    vp.u[1] = quot(s[2], ir);
+    vp.u[2] = quot(s[3], ir);
     C G[3][3];
 #pragma unroll
     for (int a = 0; a < 3; ++a)
 #pragma unroll
-        for (int b = 0; b < 3; ++b) G[a][b] = dv(g[3 * (a + 1) + b] - vp.u[a] * g[b], rho);
+        for (int b = 0; b < 3; ++b) G[a][b] = quot(g[3 * (a + 1) + b] - vp.u[a] * g[b], ir);
     C div = G[0][0] + G[1][1] + G[2][2];
     const C two = (C)2.0, tt = ((C)2.0) / ((C)3.0);
     vp.t00 = mu * (two * G[0][0] - tt * div);
@@ -206,10 +253,10 @@ __device__ __forceinline__ ViscPoint<C> viscous_point(const C* s, const C* g, C 
     vp.t01 = mu * (G[0][1] + G[1][0]);
     vp.t02 = mu * (G[0][2] + G[2][0]);
     vp.t12 = mu * (G[1][2] + G[2][1]);
-    C ke = dv(((C)0.5) * (s[1] * s[1] + s[2] * s[2] + s[3] * s[3]), rho);
+    C ke = quot(((C)0.5) * (s[1] * s[1] + s[2] * s[2] + s[3] * s[3]), ir);
     C p = gamma_m1<C>() * (s[4] - ke);
 #pragma unroll
-    for (int d = 0; d < 3; ++d) vp.q[d] = (dirs >> d) & 1 ? heat_flux(d, s, g, mu, rho, ke, p) : (C)0;
+    for (int d = 0; d < 3; ++d) vp.q[d] = (dirs >> d) & 1 ? heat_flux(d, s, g, mu, ir, irr, ke, p) : (C)0;
     return vp;
 }
 template <class C>
@@ -227,8 +274,9 @@ __device__ __forceinline__ void viscous_flux(int d, const C* s, const C* g, C mu
 }
 
 template <class C>
-__device__ __forceinline__ C sound_speed(C p, C rho) {
+__device__ __forceinline__ C sound_speed(C p, Recip<C> ir) {
     OD_CONTRACT_IN_EXPRESSIONS
+    const C rho = ir.b;
 #if OD_FAST
     if constexpr (sizeof(C) == 4) {
         // 1 / max(1e-7, rho) as a select: the reciprocal of rho is the one
@@ -237,7 +285,9 @@ __device__ __forceinline__ C sound_speed(C p, C rho) {
         return __builtin_amdgcn_sqrtf(fmax(((C)0.0), (((C)1.4) * p) * inv));
     }
 #endif
-    return sq(fmax(((C)0.0), dv(((C)1.4) * p, fmax(((C)1e-7), rho))));
+    // by max(1e-7, rho): rho's reciprocal, or that of the constant
+    const Recip<C> im = rho >= (C)1e-7 ? ir : Recip<C>{(C)1e-7, 1.0 / (double)(C)1e-7};
+    return sq(fmax(((C)0.0), quot(((C)1.4) * p, im)));
 }
 
 // Normal velocity u . n and momentum flux component m v_n + p n_c for the
@@ -267,13 +317,14 @@ __device__ __forceinline__ C mflux(int c, C a, C b, C p) {
 template <int D, class C>
 __device__ __forceinline__ void rusanov(const C* l, const C* r, C* f) {  // :104-128
     OD_CONTRACT_IN_EXPRESSIONS
-    C ul = dv(l[1], l[0]), vl = dv(l[2], l[0]), wl = dv(l[3], l[0]);
-    C ur = dv(r[1], r[0]), vr = dv(r[2], r[0]), wr = dv(r[3], r[0]);
-    C pl = pressure(l[0], l[1], l[2], l[3], l[4]);
-    C pr = pressure(r[0], r[1], r[2], r[3], r[4]);
+    const Recip<C> il = recip(l[0]), ir = recip(r[0]);
+    C ul = quot(l[1], il), vl = quot(l[2], il), wl = quot(l[3], il);
+    C ur = quot(r[1], ir), vr = quot(r[2], ir), wr = quot(r[3], ir);
+    C pl = pressure(il, l[1], l[2], l[3], l[4]);
+    C pr = pressure(ir, r[1], r[2], r[3], r[4]);
     C vnl = nvel<D>(ul, vl, wl);
     C vnr = nvel<D>(ur, vr, wr);
-    C cl = sound_speed(pl, l[0]), cr = sound_speed(pr, r[0]);
+    C cl = sound_speed(pl, il), cr = sound_speed(pr, ir);
     C lam = fmax(fabs(vnl) + cl, fabs(vnr) + cr);
     C fl[5], fr[5];
     fl[0] = l[0] * vnl;
@@ -292,16 +343,18 @@ __device__ __forceinline__ void rusanov(const C* l, const C* r, C* f) {  // :104
 template <int D, class C>
 __device__ __forceinline__ void ausm_plus(const C* l, const C* r, C* f) {  // :130-188
     OD_CONTRACT_IN_EXPRESSIONS
-    C ul = dv(l[1], l[0]), vl = dv(l[2], l[0]), wl = dv(l[3], l[0]);
-    C ur = dv(r[1], r[0]), vr = dv(r[2], r[0]), wr = dv(r[3], r[0]);
-    C pl = pressure(l[0], l[1], l[2], l[3], l[4]);
-    C pr = pressure(r[0], r[1], r[2], r[3], r[4]);
+    const Recip<C> il = recip(l[0]), ir = recip(r[0]);
+    C ul = quot(l[1], il), vl = quot(l[2], il), wl = quot(l[3], il);
+    C ur = quot(r[1], ir), vr = quot(r[2], ir), wr = quot(r[3], ir);
+    C pl = pressure(il, l[1], l[2], l[3], l[4]);
+    C pr = pressure(ir, r[1], r[2], r[3], r[4]);
     C vnl = nvel<D>(ul, vl, wl);
     C vnr = nvel<D>(ur, vr, wr);
-    C hl = dv(l[4] + pl, l[0]), hr = dv(r[4] + pr, r[0]);
-    C cl = sound_speed(pl, l[0]), cr = sound_speed(pr, r[0]);
+    C hl = quot(l[4] + pl, il), hr = quot(r[4] + pr, ir);
+    C cl = sound_speed(pl, il), cr = sound_speed(pr, ir);
     C cm = fmax(cl, cr);
-    C ml = dv(vnl, cm), mr = dv(vnr, cm);
+    const Recip<C> icm = recip(cm);
+    C ml = quot(vnl, icm), mr = quot(vnr, icm);
     const C one = (C)1.0, q = (C)0.25, alpha = (C)0.1875, beta = (C)0.125, zero = (C)0.0;
     C mp, mm, pp, pm;
     if (fabs(ml) >= one) {
@@ -333,27 +386,29 @@ __device__ __forceinline__ void ausm_plus(const C* l, const C* r, C* f) {  // :1
 template <int D, class C>
 __device__ __forceinline__ void slau2(const C* l, const C* r, C* f) {  // :190-257
     OD_CONTRACT_IN_EXPRESSIONS
-    C ul = dv(l[1], l[0]), vl = dv(l[2], l[0]), wl = dv(l[3], l[0]);
-    C ur = dv(r[1], r[0]), vr = dv(r[2], r[0]), wr = dv(r[3], r[0]);
-    C pl = pressure(l[0], l[1], l[2], l[3], l[4]);
-    C pr = pressure(r[0], r[1], r[2], r[3], r[4]);
+    const Recip<C> il = recip(l[0]), ir = recip(r[0]);
+    C ul = quot(l[1], il), vl = quot(l[2], il), wl = quot(l[3], il);
+    C ur = quot(r[1], ir), vr = quot(r[2], ir), wr = quot(r[3], ir);
+    C pl = pressure(il, l[1], l[2], l[3], l[4]);
+    C pr = pressure(ir, r[1], r[2], r[3], r[4]);
     C vnl = nvel<D>(ul, vl, wl);
     C vnr = nvel<D>(ur, vr, wr);
-    C hl = dv(l[4] + pl, l[0]), hr = dv(r[4] + pr, r[0]);
+    C hl = quot(l[4] + pl, il), hr = quot(r[4] + pr, ir);
     C sql = ul * ul + vl * vl + wl * wl;
     C sqr = ur * ur + vr * vr + wr * wr;
-    C cl = sound_speed(pl, l[0]), cr = sound_speed(pr, r[0]);
+    C cl = sound_speed(pl, il), cr = sound_speed(pr, ir);
     const C half = (C)0.5, one = (C)1.0, zero = (C)0.0;
     C cf = half * (cl + cr);
-    C ml = dv(vnl, cf), mr = dv(vnr, cf);
-    C mt = fmin(one, dv(one, cf) * sq(half * (sql + sqr)));
+    const Recip<C> icf = recip(cf);
+    C ml = quot(vnl, icf), mr = quot(vnr, icf);
+    C mt = fmin(one, quot(one, icf) * sq(half * (sql + sqr)));
     C chi = one - mt;
     chi = chi * chi;
     C g = -fmax(fmin(ml, zero), -one) * fmin(fmax(mr, zero), one);
     C vavg = dv(l[0] * fabs(vnl) + r[0] * fabs(vnr), l[0] + r[0]);
     C val = (one - g) * vavg + g * fabs(vnl);
     C var = (one - g) * vavg + g * fabs(vnr);
-    C mf = half * (l[0] * (vnl + val) + r[0] * (vnr - var) - dv(chi, cf) * (pr - pl));
+    C mf = half * (l[0] * (vnl + val) + r[0] * (vnr - var) - quot(chi, icf) * (pr - pl));
     C bl = (fabs(ml) < one) ? ((C)0.25) * (((C)2.0) - ml) * (ml + one) * (ml + one)
                             : ((ml >= zero) ? one : zero);
     C br = (fabs(mr) < one) ? ((C)0.25) * (((C)2.0) + mr) * (mr - one) * (mr - one)
@@ -383,7 +438,8 @@ __device__ __forceinline__ void interface_flux(int scheme, const C* l, const C* 
 // reference parses the keys but uses a constant mu, constants.cuh:42).
 template <class C>
 __device__ __forceinline__ C sutherland(const C* s, C mu_ref, C t_ref, C s_suth) {
-    C theta = dv(((C)1.4) * pressure(s[0], s[1], s[2], s[3], s[4]), s[0]);
+    const Recip<C> ir = recip(s[0]);
+    C theta = quot(((C)1.4) * pressure(ir, s[1], s[2], s[3], s[4]), ir);
     return dv((mu_ref * (theta * sq(theta))) * (t_ref + s_suth), t_ref * theta + s_suth);
 }
 
