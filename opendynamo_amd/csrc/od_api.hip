@@ -335,7 +335,7 @@ od_status od_create(const od_params* p, int device, od_ctx** out) {
         return cleanup(fail(OD_ERR_HIP, "stream creation failed"));
     const size_t state_bytes = (size_t)5 * c->NP * c->ubytes;
     const size_t tr_bytes = (size_t)E * od::kTraceStride * c->cbytes;
-    const size_t fv_bytes = (size_t)E * od::kFvStride * c->cbytes;
+    const size_t fv_bytes = (size_t)E * od::fv_stride(fast_kernels(*p)) * c->cbytes;
     auto dmalloc = [&](void** ptr, size_t bytes) {
         if (hipMalloc(ptr, bytes) != hipSuccess) return false;
         c->device_bytes += bytes;

@@ -94,7 +94,7 @@ od::StageArgs<UT, CT> box_args(od_batch* b, int i, int stage, double dt) {
     void* u[2] = {(UT*)b->u[0] + 320 * eo, (UT*)b->u[1] + 320 * eo};
     void* tr[3] = {(CT*)b->tr[0] + eo * od::kTraceStride, (CT*)b->tr[1] + eo * od::kTraceStride,
                    (CT*)b->tr[2] + eo * od::kTraceStride};
-    void* fv = b->fv ? (void*)((CT*)b->fv + eo * od::kFvStride) : nullptr;
+    void* fv = b->fv ? (void*)((CT*)b->fv + eo * od::fv_stride(fast_kernels(b->p))) : nullptr;
     const od_box& x = b->boxes[i];
     return make_stage_args<UT, CT>(b->p, x.nx, x.ny, x.nz, x.lx, x.ly, x.lz, u, tr, fv, nullptr, stage, dt);
 }
@@ -465,7 +465,7 @@ od_status od_batch_create(const od_params* p, const od_box* boxes, int32_t n_box
     const size_t state_bytes = (size_t)5 * 64 * E * b->ubytes;
     bool ok = dmalloc(&b->u[0], state_bytes) && dmalloc(&b->u[1], state_bytes);
     for (int q = 0; q < 3 && ok; ++q) ok = dmalloc(&b->tr[q], (size_t)E * od::kTraceStride * b->cbytes);
-    ok = ok && (!p->viscous || dmalloc(&b->fv, (size_t)E * od::kFvStride * b->cbytes));
+    ok = ok && (!p->viscous || dmalloc(&b->fv, (size_t)E * od::fv_stride(fast_kernels(*p)) * b->cbytes));
     b->table_bytes = (size_t)n_boxes * sizeof(od::BoxDev<double, double>);
     ok = ok && dmalloc(&b->table, b->table_bytes);
     ok = ok && dmalloc((void**)&b->sums_partial, (size_t)5 * max_box * sizeof(double)) &&

@@ -43,6 +43,9 @@ od::Ops<C> cast_ops(const HostOps& h) {
     return o;
 }
 
+// Whether a context's kernels are the fast build's: f32 compute with fast_math.
+inline bool fast_kernels(const od_params& p) { return p.fast_math && p.compute_real == OD_F32; }
+
 inline bool real_ok(int r) { return r == OD_F32 || r == OD_F64; }
 
 template <class Dst, class Src>

@@ -8,12 +8,11 @@
 //            4 zL, 5 zR              sequential from 0
 //            6 xL, 7 xR              sequential from the first product
 //           (face point fp: x j+4k, y i+4k, z i+4j)
-//   fv      [E][640]         CT   per element: [6][16][4] viscous flux
+//   fv      [E][fv_stride]   CT   per element: [6][16][4] viscous flux
 //                                 components 1..4 at the face points of the
-//                                 element's own faces xL,xR,yL,yR,zL,zR, then
-//                                 [64][4] the volume viscous-flux divergence of
-//                                 components 1..4 at the solution points (fast
-//                                 f32 build only); component fastest.  The
+//                                 element's own faces xL,xR,yL,yR,zL,zR
+//                                 (component fastest), then the volume part
+//                                 (kVolFast, kVolStrict below).  The
 //                                 fast f32 kernels on 2x2x2-element blocks
 //                                 store, at each face interior to a block,
 //                                 the half-difference (F_vL - F_vR) / 2 in
@@ -27,7 +26,11 @@ namespace od {
 constexpr int kTraceFaces = 8;
 constexpr int kTraceStride = kTraceFaces * 5 * 16;  // per element
 constexpr int kFvFaces = 6 * 4 * 16;                // face part, per element
-constexpr int kFvStride = kFvFaces + 4 * 64;        // + volume divergence part
+// Volume part of an element's fv block, written by the visc kernel, which holds
+// the corrected gradient, and read by the update kernel, which then needs none:
+constexpr int kVolFast = 4 * 64;    // fast f32 build: [64][4] the divergence of the viscous fluxes
+constexpr int kVolStrict = 5 * 64;  // strict build: [5][64] the whole volume RHS
+constexpr int fv_stride(bool fast) { return kFvFaces + (fast ? kVolFast : kVolStrict); }
 
 template <class C>
 struct Ops {

@@ -537,14 +537,19 @@ __device__ __forceinline__ C trace4_swz(const C* q, int base, int stride, C c0, 
 // sides of a face see the same two traces either way, so the interface
 // flux stays single-valued (conservative).
 constexpr bool kOneX = OD_FAST;
-// Fast f32 build: the visc kernel, which holds the corrected gradient anyway,
-// also forms the divergence of the volume viscous fluxes and stores it after
-// the element's face viscous fluxes (fv + kFvFaces); the update kernel then
-// takes the divergence of the Euler fluxes only and needs no gradient of its
-// own.  The strict build keeps the reference's single divergence of
-// F_e - F_v (rhs.cu:229-266) and its rounding.
+// The visc kernel, which holds the corrected gradient anyway, also forms what
+// the volume RHS needs of it and stores that after the element's face viscous
+// fluxes (fv + kFvFaces), so that the update kernel forms no gradient of its
+// own.  Fast f32 build (kSplitVisc): the divergence of the viscous fluxes; the
+// update kernel takes that of the Euler fluxes.  Strict build: the reference's
+// single divergence of F_e - F_v (rhs.cu:229-266) keeps its rounding only if it
+// is formed in one place, so the visc kernel forms the whole volume RHS.  The
+// second set of jumps and gradients it saves the update kernel was a third of
+// the strict step's instructions, for one value per variable and point written
+// and read: 48^3 f32, 40 steps 76.2 -> 73.1 ms; 24x26x22 f64, 50 steps 29.8 -> 26.3.
 template <class CT>
 constexpr bool kSplitVisc = OD_FAST && std::is_same<CT, float>::value;
+constexpr int kFvStride = fv_stride(OD_FAST);
 // The x line through point (i, j, k) is the four consecutive lanes of the
 // point's quad, so the fast f32 build contracts it from registers with DPP
 // quad broadcasts instead of an LDS round trip: the same products summed in
@@ -1171,6 +1176,64 @@ __device__ __forceinline__ void visc_divergence(const StageArgs<UT, CT>& a, int6
     *dst = FvQuad<CT>{{acc[0], acc[1], acc[2], acc[3]}};
 }
 
+// Volume RHS at the lane's point -> rs (rhs.cu:229-266, 490-510): minus the
+// divergence of F_e (VISC: of F_e - F_v, from the corrected gradient g), x then
+// y then z, plus the body force, with the RHS_REAL round trip (rhs.cu:509,
+// rk.cu:52).  S: this wave's [5][64] LDS staging area.  Strict build, and the
+// fast build's Euler fluxes (vdiv: the divergence of the viscous ones).
+template <bool VISC, class UT, class CT>
+__device__ __forceinline__ void volume_rhs(const StageArgs<UT, CT>& a, const CT (*sUe)[64], const CT* g, CT mu,
+                                           const CT* vdiv, CT (*S)[64], int i, int j, int k, int pt, CT* out) {
+    CT st[5];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) st[v] = sUe[v][pt];
+    CT rs[5] = {(CT)0, (CT)0, (CT)0, (CT)0, (CT)0};
+    ViscPoint<CT> vp;
+    if constexpr (VISC) vp = viscous_point(st, g, mu, 7);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        CT F[5];
+        euler_flux(d, st, F);
+        if constexpr (VISC) {
+            CT fvv[5];
+            viscous_flux_dir(d, vp, fvv);
+#pragma unroll
+            for (int v = 0; v < 5; ++v) F[v] = F[v] - fvv[v];
+        }
+        if constexpr (kDppX<CT>) {
+            if (d == 0) {
+                const CT* Dx = coef_lds<CT>().D[i];
+#pragma unroll
+                for (int v = 0; v < 5; ++v) rs[v] += quad_line(Dx, F[v]) * a.jx;
+                continue;
+            }
+        }
+        if (d > (kDppX<CT> ? 1 : 0)) wave_sync();  // the previous direction's reads are done
+#pragma unroll
+        for (int v = 0; v < 5; ++v) S[v][pt] = F[v];
+        wave_sync();
+        const int idx = d == 0 ? i : (d == 1 ? j : k);
+        const int base = d == 0 ? 4 * j + 16 * k : (d == 1 ? i + 16 * k : i + 4 * j);
+        const int stride = d == 0 ? 1 : (d == 1 ? 4 : 16);
+        const CT jac = d == 0 ? a.jx : (d == 1 ? a.jy : a.jz);
+        const CT* Dd = coef_lds<CT>().D[idx];
+#pragma unroll
+        for (int v = 0; v < 5; ++v) {
+            CT dd = 0;
+#pragma unroll
+            for (int m = 0; m < 4; ++m) dd += Dd[m] * S[v][base + m * stride];
+            rs[v] += dd * jac;
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+        CT val = -rs[v];
+        if (vdiv && v > 0) val += vdiv[v - 1];  // + div F_v from the visc kernel
+        if (v == 1) val += a.bf;
+        out[v] = a.round_rhs ? (CT)(float)val : val;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Kernels.
 // ---------------------------------------------------------------------------
@@ -1180,10 +1243,10 @@ __device__ __forceinline__ void visc_divergence(const StageArgs<UT, CT>& a, int6
 // traces and the BR1 jumps (960 floats each, contiguous): element 0's
 // gradients take the prefetch buffer, element 1's the jumps, written only
 // after both waves have finished reading them (a barrier).  Between the
-// jumps and the gradient tile the fast f32 build stages the volume viscous
-// fluxes of element w in pf[256 w, 256 w + 256) (visc_divergence): the
-// prefetched traces are consumed by then and sG is written only after the
-// next barrier.
+// jumps and the gradient tile the volume fluxes' lines of element w are staged
+// (vol_stage) in its half of the prefetch buffer, whose traces are consumed by
+// then, or without a prefetch in the element's own jumps, which only wave w
+// reads and has read by then.
 template <class CT>
 struct ViscLds {
     static constexpr bool kPF = std::is_same<CT, float>::value;
@@ -1196,29 +1259,28 @@ struct ViscLds {
         if constexpr (kPF) return reinterpret_cast<CT(*)[15][64]>(pf);
         else return sG_own;
     }
+    __device__ CT* vol_stage(int w) {  // 5 * 64 values
+        if constexpr (kPF) return reinterpret_cast<CT*>(pf) + w * 320;
+        else return &sJmp[w][0][0][0];
+    }
 };
 
 // With the prefetch (f32 compute) the face-correction array sJ shares the
 // prefetched neighbour traces (group A has sJ's exact layout and each face
-// point's lane reads its entries there before it writes them), and the
-// volume-flux staging sF of element w shares the BR1 jumps of element w
-// (read only by wave w, before it writes sF).
+// point's lane reads its entries there before it writes them).  sF: staging of
+// the volume fluxes' lines, where this kernel forms them (kVol): the Euler mode
+// and the fast build.
 template <class CT, bool VISC>
 struct UpdateLds {
     static constexpr bool kPF = std::is_same<CT, float>::value;
-    static constexpr bool kJmp = VISC && !kSplitVisc<CT>;  // BR1 jumps formed in this kernel
+    static constexpr bool kVol = !VISC || kSplitVisc<CT>;
     float pf[kPF ? kPfFloatsUpdate : 4];
     CT sU[kEpb][5][64];
-    CT sJmp[kJmp ? kEpb : 0][6][5][16];
     CT sJ_own[kPF ? 0 : kEpb][6][5][16];  // zero-length when aliased
-    CT sF_own[kJmp ? 0 : kEpb][5][64];
+    CT sF[kVol ? kEpb : 0][5][64];
     __device__ CT (*sJ())[6][5][16] {
         if constexpr (kPF) return reinterpret_cast<CT(*)[6][5][16]>(pf + kPfA);
         else return sJ_own;
-    }
-    __device__ CT (*sF(int w))[64] {
-        if constexpr (kJmp) return reinterpret_cast<CT(*)[64]>(&sJmp[w][0][0][0]);
-        else return sF_own[w];
     }
 };
 
@@ -1255,9 +1317,21 @@ __device__ __forceinline__ void visc_body(const StageArgs<UT, CT>& a, const Tile
     __syncthreads();
     CT g[15];
     if (tile_valid(tl, wave)) lane_gradient(a, L.sU[wave], L.sJmp[wave], i, j, k, g);
-    if constexpr (kSplitVisc<CT>) {
-        if (tile_valid(tl, wave))
-            visc_divergence(a, tile_eidx(tl, wave), L.sU[wave], g, L.pf + wave * 256, i, j, k, pt);
+    if (tile_valid(tl, wave)) {
+        const int64_t e = tile_eidx(tl, wave);
+        if constexpr (kSplitVisc<CT>) {
+            visc_divergence(a, e, L.sU[wave], g, L.vol_stage(wave), i, j, k, pt);
+        } else {
+            CT st[5], r[5];
+#pragma unroll
+            for (int v = 0; v < 5; ++v) st[v] = L.sU[wave][v][pt];
+            CT mu = a.sutherland ? sutherland(st, a.mu_ref, a.t_ref, a.s_suth) : a.mu;
+            if (a.mu_t) mu = mu + a.mu_t[e];
+            wave_sync();  // without a prefetch the staging area is the jumps just read
+            volume_rhs<true>(a, L.sU[wave], g, mu, (const CT*)nullptr, (CT(*)[64])L.vol_stage(wave), i, j, k, pt, r);
+#pragma unroll
+            for (int v = 0; v < 5; ++v) a.fv[e * kFvStride + kFvFaces + v * 64 + pt] = r[v];
+        }
     }
     if constexpr (PF) __syncthreads();  // sG overwrites the jumps the other wave may still read
     if (tile_valid(tl, wave)) {
@@ -1307,78 +1381,25 @@ __device__ __forceinline__ void update_body(const StageArgs<UT, CT>& a, const Ti
     if constexpr (PF) __builtin_amdgcn_s_waitcnt(0);  // this wave's LDS copies have landed
     __syncthreads();
 
-    // with kSplitVisc the volume viscous terms come from the visc kernel
-    constexpr bool VOLV = VISC && !kSplitVisc<CT>;
-    CT g[15];
-    if constexpr (VOLV) {
-        run_br1_jumps<PF>(a, L.sU, L.sJmp, tl, pfc, wave, pt);
-        __syncthreads();
-        lane_gradient(a, L.sU[wave], L.sJmp[wave], i, j, k, g);
-    }
-    CT st[5];
+    // Volume RHS: formed here in the Euler mode and the fast build (which adds
+    // the visc kernel's viscous divergence) and kept in LDS during the face
+    // passes; else the visc kernel's, read after them.
+    constexpr bool VOL = UpdateLds<CT, VISC>::kVol;
+    if constexpr (VOL) {
+        CT vdiv[4] = {(CT)0, (CT)0, (CT)0, (CT)0}, r[5];
+        if constexpr (VISC) {
+            if (mine) {
+                const FvQuad<CT> src =
+                    *reinterpret_cast<const FvQuad<CT>*>(a.fv + tile_eidx(tl, wave) * kFvStride + kFvFaces + pt * 4);
 #pragma unroll
-    for (int v = 0; v < 5; ++v) st[v] = L.sU[wave][v][pt];
-    CT mu = (CT)0;
-    if (VOLV) mu = a.sutherland ? sutherland(st, a.mu_ref, a.t_ref, a.s_suth) : a.mu;
-    if (VOLV && a.mu_t) mu = mu + (mine ? a.mu_t[tile_eidx(tl, wave)] : (CT)0);
-    CT vdiv[4] = {(CT)0, (CT)0, (CT)0, (CT)0};
-    if (VISC && !VOLV && mine) {
-        const FvQuad<CT> src =
-            *reinterpret_cast<const FvQuad<CT>*>(a.fv + tile_eidx(tl, wave) * kFvStride + kFvFaces + pt * 4);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) vdiv[q] = src.c[q];
-    }
-
-    // Volume flux divergence, x then y then z (rhs.cu:229-266, 490-510).
-    CT rs[5] = {(CT)0, (CT)0, (CT)0, (CT)0, (CT)0};
-    ViscPoint<CT> vp;
-    if (VOLV) vp = viscous_point(st, g, mu, 7);
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        CT fe[5], F[5];
-        euler_flux(d, st, fe);
-        if (VOLV) {
-            CT fvv[5];
-            viscous_flux_dir(d, vp, fvv);
-#pragma unroll
-            for (int v = 0; v < 5; ++v) F[v] = fe[v] - fvv[v];
-        } else {
-#pragma unroll
-            for (int v = 0; v < 5; ++v) F[v] = fe[v];
-        }
-        if constexpr (kDppX<CT>) {
-            if (d == 0) {
-                const CT* Dx = coef_lds<CT>().D[i];
-#pragma unroll
-                for (int v = 0; v < 5; ++v) rs[v] += quad_line(Dx, F[v]) * a.jx;
-                continue;
+                for (int q = 0; q < 4; ++q) vdiv[q] = src.c[q];
             }
         }
-        if (d > (kDppX<CT> ? 1 : 0)) __syncthreads();
+        volume_rhs<false>(a, L.sU[wave], (const CT*)nullptr, (CT)0, VISC ? vdiv : (const CT*)nullptr, L.sF[wave], i, j,
+                          k, pt, r);
+        wave_sync();
 #pragma unroll
-        for (int v = 0; v < 5; ++v) L.sF(wave)[v][pt] = F[v];
-        __syncthreads();
-        const int idx = d == 0 ? i : (d == 1 ? j : k);
-        const int base = d == 0 ? 4 * j + 16 * k : (d == 1 ? i + 16 * k : i + 4 * j);
-        const int stride = d == 0 ? 1 : (d == 1 ? 4 : 16);
-        const CT jac = d == 0 ? a.jx : (d == 1 ? a.jy : a.jz);
-        const CT* Dd = coef_lds<CT>().D[idx];
-#pragma unroll
-        for (int v = 0; v < 5; ++v) {
-            CT dd = 0;
-#pragma unroll
-            for (int m = 0; m < 4; ++m) dd += Dd[m] * L.sF(wave)[v][base + m * stride];
-            rs[v] += dd * jac;
-        }
-    }
-    // the volume RHS waits in LDS (this wave's sF slot) during the face passes
-    __syncthreads();
-#pragma unroll
-    for (int v = 0; v < 5; ++v) {
-        CT val = -rs[v];
-        if (VISC && !VOLV && v > 0) val += vdiv[v - 1];  // + div F_v from the visc kernel
-        if (v == 1) val += a.bf;
-        L.sF(wave)[v][pt] = a.round_rhs ? (CT)(float)val : val;  // RHS_REAL round trip (rhs.cu:509, rk.cu:52)
+        for (int v = 0; v < 5; ++v) L.sF[wave][v][pt] = r[v];
     }
 
     // Interface fluxes at all own faces, direction by direction.
@@ -1409,7 +1430,10 @@ __device__ __forceinline__ void update_body(const StageArgs<UT, CT>& a, const Ti
 #pragma unroll
     for (int v = 0; v < 5; ++v) {
         ucr[v] = SAME ? (UT)L.sU[wave][v][pt] : ucur[v];
-        r[v] = L.sF(wave)[v][pt];
+        if constexpr (VOL)
+            r[v] = L.sF[wave][v][pt];
+        else
+            r[v] = mine ? stream_load(&a.fv[tile_eidx(tl, wave) * kFvStride + kFvFaces + v * 64 + pt]) : (CT)0;
     }
     if (a.stage1) {  // u^n is the state this stage read (uprev == uin): no second load
 #pragma unroll
