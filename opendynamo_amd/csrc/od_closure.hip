@@ -15,6 +15,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
 #include <random>
 #include <string>
@@ -617,6 +618,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void o
 struct Adam {
     float *p, *m, *v;
     float lr, b1t, b2t;
+    float* sse;  // the batch's sum of squared errors goes here as well
 };
 
 // grad[p] = sum over the partial rows, in row order (deterministic), for the 32
@@ -661,7 +663,10 @@ __global__ __launch_bounds__(256) void od_mlp_reduce_kernel(const float* __restr
     if (threadIdx.x >= C || p > NPARAM) return;
     grad[p] = s;
     if constexpr (STEP) {
-        if (p == NPARAM) return;
+        if (p == NPARAM) {
+            *ad.sse = s;
+            return;
+        }
         const float mm = 0.9f * ad.m[p] + 0.1f * s;
         const float vv = 0.999f * ad.v[p] + 0.001f * s * s;
         ad.m[p] = mm;
@@ -725,7 +730,8 @@ struct od_mlp {
     float* grad = nullptr;    // NPARAM + 1
     unsigned short* wb = nullptr;  // bf16 copies: w1 | w2 | w3 | w2t | w3t | w4
     Scaling sc{};
-    std::vector<float> host_params;
+    float* partial = nullptr;  // partial gradient rows of the largest batch so far (at most 1024)
+    size_t partial_rows = 0;
     uint64_t adam_t = 0;
 };
 
@@ -755,30 +761,69 @@ struct DevBuf {  // scoped device allocation
     }
 };
 
+// One epoch of a training run in flight (od_mlp_train).
+struct EpochSlot {
+    int *idx = nullptr, *host_idx = nullptr;      // sample order: device, pinned host
+    float *sse = nullptr, *host_sse = nullptr;    // per batch
+    hipEvent_t done = nullptr;
+    uint32_t epoch = 0;
+    bool busy = false;
+    EpochSlot() = default;
+    EpochSlot(const EpochSlot&) = delete;
+    EpochSlot& operator=(const EpochSlot&) = delete;
+    ~EpochSlot() {
+        // frees wait for the device, the event's work included
+        if (idx) (void)hipFree(idx);
+        if (sse) (void)hipFree(sse);
+        if (host_idx) (void)hipHostFree(host_idx);
+        if (host_sse) (void)hipHostFree(host_sse);
+        if (done) (void)hipEventDestroy(done);
+    }
+};
+
+// x mod d for d <= n without a 64-bit division: q = the high half of x times
+// floor((2^64 - 1) / d) is floor(x / d) or one less.  An epoch's shuffle takes
+// one modulus per sample, with the same n - 1 divisors every time.
+struct ModTable {
+    uint64_t* inv = nullptr;
+    ModTable() = default;
+    ModTable(const ModTable&) = delete;
+    ModTable& operator=(const ModTable&) = delete;
+    ~ModTable() { std::free(inv); }
+    void fill(size_t n) {
+        inv = (uint64_t*)std::malloc((n + 1) * sizeof(uint64_t));
+        for (size_t d = 1; inv && d <= n; ++d) inv[d] = ~(uint64_t)0 / d;
+    }
+    size_t mod(uint64_t x, size_t d) const {
+        if (!inv) return (size_t)(x % d);
+        const uint64_t r = x - (uint64_t)(((unsigned __int128)x * inv[d]) >> 64) * d;
+        return (size_t)(r >= d ? r - d : r);
+    }
+};
+
 // Gradient of the mean squared error over n gathered samples; grad and the
 // sum of squared errors in m->grad (device).  With `adam` the parameters take
 // their step in the same launch as the sum over the groups.
-od_status run_grad(od_mlp* m, const float* dx, const float* dt, const int* didx, int64_t n, const Adam* adam,
-                   float** partial, size_t* partial_cap) {
+od_status run_grad(od_mlp* m, const float* dx, const float* dt, const int* didx, int64_t n, const Adam* adam) {
     const int64_t tiles = (n + 15) / 16;
     const int tpg = (int)std::max<int64_t>(1, (tiles + 1023) / 1024);
     const int64_t groups = (tiles + tpg - 1) / tpg;
-    const size_t need = (size_t)groups * kPartialRow * sizeof(float);
-    if (need > *partial_cap) {
-        if (*partial) (void)hipFree(*partial);
-        *partial = nullptr;
-        *partial_cap = 0;
-        HIP_TRY(hipMalloc((void**)partial, need));
-        *partial_cap = need;
+    if ((size_t)groups > m->partial_rows) {
+        HIP_TRY(hipStreamSynchronize(m->stream));  // no batch still reads the smaller array
+        if (m->partial) (void)hipFree(m->partial);
+        m->partial = nullptr;
+        m->partial_rows = 0;
+        HIP_TRY(hipMalloc((void**)&m->partial, (size_t)groups * kPartialRow * sizeof(float)));
+        m->partial_rows = (size_t)groups;
     }
     hipLaunchKernelGGL(od_mlp_grad_kernel, dim3((unsigned)groups), dim3(256), 0, m->stream, dev_net(m), m->sc, dx, dt,
-                       didx, n, tpg, *partial);
+                       didx, n, tpg, m->partial);
     if (check()) return fail(OD_ERR_HIP, "od_mlp_grad_kernel launch failed");
     if (adam)
-        hipLaunchKernelGGL(od_mlp_reduce_kernel<true>, dim3(kPartialRow / 32), dim3(256), 0, m->stream, *partial,
+        hipLaunchKernelGGL(od_mlp_reduce_kernel<true>, dim3(kPartialRow / 32), dim3(256), 0, m->stream, m->partial,
                            (int)groups, m->grad, *adam, dev_net(m));
     else
-        hipLaunchKernelGGL(od_mlp_reduce_kernel<false>, dim3(kPartialRow / 32), dim3(256), 0, m->stream, *partial,
+        hipLaunchKernelGGL(od_mlp_reduce_kernel<false>, dim3(kPartialRow / 32), dim3(256), 0, m->stream, m->partial,
                            (int)groups, m->grad, Adam{}, dev_net(m));
     if (check()) return fail(OD_ERR_HIP, "od_mlp_reduce_kernel launch failed");
     return OD_OK;
@@ -978,7 +1023,8 @@ void od_mlp_destroy(od_mlp* m) {
     if (!m) return;
     (void)hipSetDevice(m->device);
     if (m->stream) (void)hipStreamSynchronize(m->stream);
-    for (void* q : {(void*)m->params, (void*)m->adam_m, (void*)m->adam_v, (void*)m->grad, (void*)m->wb})
+    for (void* q : {(void*)m->params, (void*)m->adam_m, (void*)m->adam_v, (void*)m->grad, (void*)m->wb,
+                    (void*)m->partial})
         if (q) (void)hipFree(q);
     if (m->stream) (void)hipStreamDestroy(m->stream);
     delete m;
@@ -1053,15 +1099,12 @@ od_status od_mlp_loss_grad(od_mlp* m, const float* x, const float* t, size_t n, 
     HIP_TRY(hipMalloc(&dt.p, n * sizeof(float)));
     HIP_TRY(hipMemcpyAsync(dx.p, x, n * NF * sizeof(float), hipMemcpyHostToDevice, m->stream));
     HIP_TRY(hipMemcpyAsync(dt.p, t, n * sizeof(float), hipMemcpyHostToDevice, m->stream));
-    float* partial = nullptr;
-    size_t cap = 0;
-    od_status s = run_grad(m, (const float*)dx.p, (const float*)dt.p, nullptr, (int64_t)n, nullptr, &partial, &cap);
+    od_status s = run_grad(m, (const float*)dx.p, (const float*)dt.p, nullptr, (int64_t)n, nullptr);
     std::vector<float> g(NPARAM + 1);
     if (s == OD_OK && hipMemcpyAsync(g.data(), m->grad, (NPARAM + 1) * sizeof(float), hipMemcpyDeviceToHost,
                                      m->stream) != hipSuccess)
         s = fail(OD_ERR_HIP, "od_mlp_loss_grad: copy failed");
     (void)hipStreamSynchronize(m->stream);
-    if (partial) (void)hipFree(partial);
     if (s != OD_OK) return s;
     if (loss) *loss = (double)g[NPARAM] / (double)n;
     if (grad) std::memcpy(grad, g.data(), NPARAM * sizeof(float));
@@ -1074,54 +1117,68 @@ od_status od_mlp_train(od_mlp* m, const float* x, const float* t, size_t n, uint
     if (n == 0 || batch == 0) return fail(OD_ERR_INVALID, "od_mlp_train: empty data or batch");
     if (n > (size_t)0x7fffffff) return fail(OD_ERR_INVALID, "od_mlp_train: too many samples");
     HIP_TRY(hipSetDevice(m->device));
-    DevBuf dx, dt, di;
+    // Two epochs are in flight: while the device works through one, the host
+    // orders the next one's samples.  Each slot has its index array, the sums of
+    // squared errors of its batches and an event at the end of its work.
+    const size_t n_batches = (n + batch - 1) / batch;
+    DevBuf dx, dt;
+    EpochSlot slot[2];
+    ModTable mod;
     HIP_TRY(hipMalloc(&dx.p, n * NF * sizeof(float)));
     HIP_TRY(hipMalloc(&dt.p, n * sizeof(float)));
-    HIP_TRY(hipMalloc(&di.p, n * sizeof(int)));
+    for (EpochSlot& q : slot) {
+        HIP_TRY(hipMalloc((void**)&q.idx, n * sizeof(int)));
+        HIP_TRY(hipMalloc((void**)&q.sse, n_batches * sizeof(float)));
+        HIP_TRY(hipHostMalloc((void**)&q.host_idx, n * sizeof(int), hipHostMallocDefault));
+        HIP_TRY(hipHostMalloc((void**)&q.host_sse, n_batches * sizeof(float), hipHostMallocDefault));
+        HIP_TRY(hipEventCreateWithFlags(&q.done, hipEventDisableTiming));
+    }
     HIP_TRY(hipMemcpyAsync(dx.p, x, n * NF * sizeof(float), hipMemcpyHostToDevice, m->stream));
     HIP_TRY(hipMemcpyAsync(dt.p, t, n * sizeof(float), hipMemcpyHostToDevice, m->stream));
-    std::vector<int> perm(n);
+    if (epochs > 1) mod.fill(n);
     std::mt19937_64 rng(seed);
-    float* partial = nullptr;
-    size_t cap = 0;
-    std::vector<float> g(NPARAM + 1);
-    od_status s = OD_OK;
-    for (uint32_t ep = 0; ep < epochs && s == OD_OK; ++ep) {
-        for (size_t q = 0; q < n; ++q) perm[q] = (int)q;
-        for (size_t q = n - 1; q > 0; --q) {  // Fisher-Yates with the seeded generator
-            const size_t r = (size_t)(rng() % (q + 1));
-            std::swap(perm[q], perm[r]);
-        }
-        HIP_TRY(hipStreamSynchronize(m->stream));  // the previous epoch's gathers are done with the index
-        HIP_TRY(hipMemcpy(di.p, perm.data(), n * sizeof(int), hipMemcpyHostToDevice));
+    // waits for the epoch in slot q and takes its loss
+    auto finish = [&](EpochSlot& q) -> od_status {
+        if (!q.busy) return OD_OK;
+        q.busy = false;
+        HIP_TRY(hipEventSynchronize(q.done));
         double sse = 0.0;
-        for (size_t b0 = 0; b0 < n && s == OD_OK; b0 += batch) {
-            const int64_t nb = (int64_t)std::min<size_t>(batch, n - b0);
-            m->adam_t += 1;
+        for (size_t k = 0; k < n_batches; ++k) sse += q.host_sse[k];
+        if (loss_per_epoch) loss_per_epoch[q.epoch] = (float)(sse / (double)n);
+        return OD_OK;
+    };
+    auto run_epoch = [&](EpochSlot& q, uint32_t ep) -> od_status {
+        od_status s = finish(q);
+        if (s != OD_OK) return s;
+        int* perm = q.host_idx;
+        for (size_t k = 0; k < n; ++k) perm[k] = (int)k;
+        for (size_t k = n - 1; k > 0; --k)  // Fisher-Yates with the seeded generator
+            std::swap(perm[k], perm[mod.mod(rng(), k + 1)]);
+        HIP_TRY(hipMemcpyAsync(q.idx, perm, n * sizeof(int), hipMemcpyHostToDevice, m->stream));
+        for (size_t b0 = 0, k = 0; b0 < n; b0 += batch, ++k) {
+            const uint64_t at = m->adam_t + 1;
             const Adam ad{m->params,
                           m->adam_m,
                           m->adam_v,
                           lr,
-                          (float)std::pow(0.9, (double)m->adam_t),
-                          (float)std::pow(0.999, (double)m->adam_t)};
-            s = run_grad(m, (const float*)dx.p, (const float*)dt.p, (const int*)di.p + b0, nb, &ad, &partial, &cap);
-            if (s != OD_OK) {
-                m->adam_t -= 1;
-                break;
-            }
-            if (loss_per_epoch && s == OD_OK) {
-                float v = 0.0f;
-                if (hipMemcpyAsync(&v, m->grad + NPARAM, sizeof(float), hipMemcpyDeviceToHost, m->stream) !=
-                        hipSuccess ||
-                    hipStreamSynchronize(m->stream) != hipSuccess)
-                    s = fail(OD_ERR_HIP, "od_mlp_train: loss copy failed");
-                sse += v;
-            }
+                          (float)std::pow(0.9, (double)at),
+                          (float)std::pow(0.999, (double)at),
+                          q.sse + k};
+            s = run_grad(m, (const float*)dx.p, (const float*)dt.p, q.idx + b0, (int64_t)std::min<size_t>(batch, n - b0),
+                         &ad);
+            if (s != OD_OK) return s;
+            m->adam_t = at;
         }
-        if (loss_per_epoch) loss_per_epoch[ep] = (float)(sse / (double)n);
-    }
+        HIP_TRY(hipMemcpyAsync(q.host_sse, q.sse, n_batches * sizeof(float), hipMemcpyDeviceToHost, m->stream));
+        HIP_TRY(hipEventRecord(q.done, m->stream));
+        q.epoch = ep;
+        q.busy = true;
+        return OD_OK;
+    };
+    od_status s = OD_OK;
+    for (uint32_t ep = 0; ep < epochs && s == OD_OK; ++ep) s = run_epoch(slot[ep & 1], ep);
+    for (uint32_t k = 0; k < 2 && s == OD_OK; ++k) s = finish(slot[(epochs + k) & 1]);
     (void)hipStreamSynchronize(m->stream);
-    if (partial) (void)hipFree(partial);
     return s;
 }
 

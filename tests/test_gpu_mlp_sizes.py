@@ -53,3 +53,27 @@ def test_forward_at_the_edges_of_the_work_split(n):
         y = m.forward(x)
     want, _ = M.forward(p, x, shift, scale)
     assert np.max(np.abs(y - want)) < 0.02 * np.max(np.abs(want))
+
+
+# one sample, fewer samples than a batch, ragged batches, one batch per sample
+@pytest.mark.parametrize("n,batch", [(1, 64), (40, 64), (1000, 300), (5, 1)])
+def test_epochs_in_flight_keep_their_order_and_losses(n, batch):
+    """Two epochs are in flight at a time: a run of e epochs has the losses of
+    the first e epochs of a longer one, byte for byte, and its first loss is
+    that of the starting weights (one batch: to f32 rounding of the sum)."""
+    p, shift, scale = network(n)
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((n, od.MLP_FEATURES)).astype(np.float32)
+    t = rng.uniform(0.0, 1.0, n).astype(np.float32)
+    runs = {}
+    for epochs in (1, 2, 3, 6):
+        print(f"CASE test=epochs n={n} batch={batch} epochs={epochs}", flush=True)
+        with od.MLP(params=p) as m:
+            m.set_scaling(shift, scale)
+            first, _ = m.loss_grad(x, t)
+            runs[epochs] = m.train(x, t, epochs=epochs, batch=batch, lr=1e-3, seed=4)
+    assert len(np.unique(runs[6])) == 6
+    for epochs in (1, 2, 3):
+        assert runs[epochs].tobytes() == runs[6][:epochs].tobytes()
+    if batch >= n:
+        assert abs(runs[1][0] - first) <= 1e-5 * first
