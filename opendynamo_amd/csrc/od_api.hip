@@ -191,10 +191,11 @@ od_status enqueue_step(od_ctx* c, double dt) {
 // 8-step graph plus n % 8 of the one-step graph (same kernels, same order).
 constexpr uint32_t kStepsPerGraph = 8;
 
-od_status capture_steps(od_ctx* c, uint32_t steps, hipGraphExec_t* out) {
+// refresh: the closure's mu_t refresh before the first step.
+od_status capture_steps(od_ctx* c, bool refresh, uint32_t steps, hipGraphExec_t* out) {
     hipGraph_t g = nullptr;
     HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    od_status s = OD_OK;
+    od_status s = refresh ? od_closure_refresh_internal(c) : OD_OK;
     for (uint32_t q = 0; q < steps && s == OD_OK; ++q) s = enqueue_step(c, kTableDt);
     hipError_t e = hipStreamEndCapture(c->stream, &g);
     if (s != OD_OK) {
@@ -219,7 +220,7 @@ int write_dt(od_ctx* c, double dt) {
         v[s].cc = stage_dt_coef<CT>(s, dt);
         v[s].uc = stage_dt_coef<UT>(s, dt);
     }
-    return od::launch_set_dt<UT, CT>((od::StageDt<UT, CT>*)c->dt_table, v, c->stream);
+    return od::launch_set_dt<UT, CT>((od::StageDt<UT, CT>*)c->dt_table, v, c->dt_value, dt, c->stream);
 }
 
 // The dt of the steps enqueued from here on, written in stream order (steps
@@ -249,7 +250,7 @@ od_status ensure_graph(od_ctx* c, bool multi) {
         c->graph_mu_t = c->mu_t_on;
     }
     hipGraphExec_t* gx = multi ? &c->graph_k : &c->graph;
-    return *gx ? OD_OK : capture_steps(c, multi ? kStepsPerGraph : 1, gx);
+    return *gx ? OD_OK : capture_steps(c, false, multi ? kStepsPerGraph : 1, gx);
 }
 
 // Enqueue n steps of size dt of the captured graphs on the library stream.
@@ -262,6 +263,39 @@ od_status launch_steps(od_ctx* c, double dt, uint32_t n) {
     for (; q + kStepsPerGraph <= n; q += kStepsPerGraph) HIP_TRY(hipGraphLaunch(c->graph_k, c->stream));
     for (; q < n; ++q) HIP_TRY(hipGraphLaunch(c->graph, c->stream));
     return OD_OK;
+}
+
+// n steps of size dt with the closure's refresh of mu_t every update_interval
+// steps, all enqueued without waiting.  Whole intervals of up to kStepsPerGraph
+// steps are one graph, refresh included; it is captured again when what its
+// refresh was captured with (network, scaling, budget) has changed.
+od_status closure_steps(od_ctx* c, double dt, uint32_t n) {
+    const uint32_t interval = (uint32_t)c->closure.update_interval;
+    od_status s = set_dt(c, dt);
+    if (s != OD_OK) return s;
+    if (od_closure_key_changed_internal(c) && c->graph_c) {
+        HIP_TRY(hipGraphExecDestroy(c->graph_c));
+        c->graph_c = nullptr;
+    }
+    bool refreshed = false;
+    for (uint32_t q = 0; q < n && s == OD_OK;) {
+        const uint32_t at = (uint32_t)(c->steps_done % interval);
+        const uint32_t run = std::min(n - q, interval - at);
+        if (at == 0) refreshed = true;
+        if (at == 0 && run == interval && interval <= kStepsPerGraph) {
+            if (!c->graph_c) s = capture_steps(c, true, interval, &c->graph_c);
+            if (s == OD_OK && hipGraphLaunch(c->graph_c, c->stream) != hipSuccess)
+                s = fail(OD_ERR_HIP, "closure step graph launch failed");
+        } else {
+            if (at == 0) s = od_closure_refresh_internal(c);
+            if (s == OD_OK) s = launch_steps(c, dt, run);
+        }
+        if (s != OD_OK) break;
+        q += run;
+        c->steps_done += run;
+    }
+    const od_status u = refreshed ? od_closure_used_internal(c) : OD_OK;
+    return s != OD_OK ? s : u;
 }
 
 }  // namespace
@@ -344,10 +378,16 @@ od_status od_create(const od_params* p, int device, od_ctx** out) {
     bool ok = dmalloc(&c->u[0], state_bytes) && dmalloc(&c->u[1], state_bytes);
     for (int q = 0; q < 3 && ok; ++q) ok = dmalloc(&c->tr[q], tr_bytes);
     ok = ok && (!p->viscous || dmalloc(&c->fv, fv_bytes));
-    ok = ok && dmalloc((void**)&c->sums_partial, (size_t)5 * E * sizeof(double)) &&
-         dmalloc((void**)&c->sums_out, 8 * sizeof(double)) &&
-         dmalloc((void**)&c->cfl_partial, od::kCflGroups * sizeof(double)) &&
-         dmalloc(&c->dt_table, 3 * sizeof(od::StageDt<double, double>));
+    // the small arrays share the partial sums' allocation
+    static_assert(sizeof(od::StageDt<double, double>) % sizeof(double) == 0, "table of doubles");
+    const size_t dt_doubles = 3 * sizeof(od::StageDt<double, double>) / sizeof(double) + 1;
+    ok = ok && dmalloc((void**)&c->sums_partial, ((size_t)5 * E + 8 + od::kCflGroups + dt_doubles) * sizeof(double));
+    if (ok) {
+        c->sums_out = c->sums_partial + (size_t)5 * E;
+        c->cfl_partial = c->sums_out + 8;
+        c->dt_value = c->cfl_partial + od::kCflGroups;
+        c->dt_table = c->dt_value + 1;
+    }
     if (!ok) return cleanup(fail(OD_ERR_NOMEM, "device allocation failed"));
     for (int q = 0; q < 3; ++q)
         if (hipHostMalloc(&c->pinned[q], state_bytes, hipHostMallocDefault) != hipSuccess ||
@@ -364,6 +404,7 @@ void od_destroy(od_ctx* c) {
     if (c->io_stream) (void)hipStreamSynchronize(c->io_stream);
     if (c->graph) (void)hipGraphExecDestroy(c->graph);
     if (c->graph_k) (void)hipGraphExecDestroy(c->graph_k);
+    if (c->graph_c) (void)hipGraphExecDestroy(c->graph_c);
     for (void* q : c->u)
         if (q) (void)hipFree(q);
     for (void* q : c->tr)
@@ -371,9 +412,6 @@ void od_destroy(od_ctx* c) {
     if (c->fv) (void)hipFree(c->fv);
     if (c->dbg) (void)hipFree(c->dbg);
     if (c->sums_partial) (void)hipFree(c->sums_partial);
-    if (c->sums_out) (void)hipFree(c->sums_out);
-    if (c->cfl_partial) (void)hipFree(c->cfl_partial);
-    if (c->dt_table) (void)hipFree(c->dt_table);
     od_closure_release_internal(c);
     for (int q = 0; q < 3; ++q) {
         if (c->pinned[q]) (void)hipHostFree(c->pinned[q]);
@@ -491,22 +529,10 @@ od_status od_step(od_ctx* c, double dt, uint32_t n_steps) {
     if (!c->state_set) return fail(OD_ERR_STATE, "od_step: state not set");
     if (!(dt > 0.0) || !std::isfinite(dt)) return fail(OD_ERR_INVALID, "od_step: dt must be positive and finite");
     HIP_TRY(hipSetDevice(c->device));
-    od_status s = OD_OK;
-    if (!c->mlp) {
-        s = launch_steps(c, dt, n_steps);
-        if (s == OD_OK) c->steps_done += n_steps;
-        return s;
-    }
-    if ((s = set_dt(c, dt)) != OD_OK || (s = ensure_graph(c, false)) != OD_OK) return s;
-    for (uint32_t q = 0; q < n_steps; ++q) {  // the closure refreshes mu_t between steps
-        if (c->steps_done % (uint64_t)c->closure.update_interval == 0) {
-            s = od_closure_update_internal(c, dt * c->closure.update_interval);
-            if (s != OD_OK) return s;
-        }
-        HIP_TRY(hipGraphLaunch(c->graph, c->stream));
-        c->steps_done += 1;
-    }
-    return OD_OK;
+    if (c->mlp) return closure_steps(c, dt, n_steps);
+    od_status s = launch_steps(c, dt, n_steps);
+    if (s == OD_OK) c->steps_done += n_steps;
+    return s;
 }
 
 od_status od_synchronize(od_ctx* c) {

@@ -34,9 +34,9 @@ struct od_batch {
     void* fv = nullptr;
     void* table = nullptr;
     size_t table_bytes = 0;
-    double* sums_partial = nullptr;
-    double* sums_out = nullptr;
-    double* cfl_partial = nullptr;  // od::kCflGroups doubles
+    double* sums_partial = nullptr;  // [5][largest box], then (one allocation):
+    double* sums_out = nullptr;      // 8 doubles
+    double* cfl_partial = nullptr;   // od::kCflGroups doubles
     HostOps ops;
     std::vector<char> state_set;
     od_schedule sched{0, 1, 0, 0};
@@ -468,9 +468,11 @@ od_status od_batch_create(const od_params* p, const od_box* boxes, int32_t n_box
     ok = ok && (!p->viscous || dmalloc(&b->fv, (size_t)E * od::fv_stride(fast_kernels(*p)) * b->cbytes));
     b->table_bytes = (size_t)n_boxes * sizeof(od::BoxDev<double, double>);
     ok = ok && dmalloc(&b->table, b->table_bytes);
-    ok = ok && dmalloc((void**)&b->sums_partial, (size_t)5 * max_box * sizeof(double)) &&
-         dmalloc((void**)&b->sums_out, 8 * sizeof(double)) &&
-         dmalloc((void**)&b->cfl_partial, od::kCflGroups * sizeof(double));
+    ok = ok && dmalloc((void**)&b->sums_partial, ((size_t)5 * max_box + 8 + od::kCflGroups) * sizeof(double));
+    if (ok) {
+        b->sums_out = b->sums_partial + (size_t)5 * max_box;
+        b->cfl_partial = b->sums_out + 8;
+    }
     if (!ok) return cleanup(fail(OD_ERR_NOMEM, "device allocation failed"));
     *out = b;
     return OD_OK;
@@ -488,8 +490,6 @@ void od_batch_destroy(od_batch* b) {
     if (b->fv) (void)hipFree(b->fv);
     if (b->table) (void)hipFree(b->table);
     if (b->sums_partial) (void)hipFree(b->sums_partial);
-    if (b->sums_out) (void)hipFree(b->sums_out);
-    if (b->cfl_partial) (void)hipFree(b->cfl_partial);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
 }

@@ -15,8 +15,11 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstddef>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
+#include <mutex>
 #include <random>
 #include <string>
 #include <vector>
@@ -678,16 +681,31 @@ __global__ __launch_bounds__(256) void od_mlp_reduce_kernel(const float* __restr
     }
 }
 
-// Deterministic sums of three float arrays of length n (one block of 256,
-// fixed order): out[0..2].
-__global__ __launch_bounds__(256) void od_sum3_kernel(const float* __restrict__ a, int as, const float* __restrict__ b,
-                                                      const float* __restrict__ c, int64_t n, double* __restrict__ out) {
+// The kinetic-energy budget of a closure interval, on the device: its state is
+// kept there so that a step with a network never waits for the device.
+enum { kKePrev, kEpsPrev, kActive, kStats, kBudget = kStats + 6 };
+
+// Sums (one block of 256, fixed order) of the elements' kinetic energy, model
+// dissipation and out-of-range flags, then the check of the interval that just
+// ended; when it fails, mu_t is zero for the next one.  dt: the step size;
+// interval = update_interval.
+// The model over-dissipates when, over an interval in which the kinetic energy
+// decayed, the energy it removed exceeds kappa times the whole observed decay.
+// An interval in which the energy grew is not held against the model (it only
+// removes energy).
+template <class CT>
+__global__ __launch_bounds__(256) void od_budget_kernel(const float* __restrict__ feat, const float* __restrict__ eps,
+                                                        const float* __restrict__ oor, int64_t n,
+                                                        const double* __restrict__ dt, double interval, double kappa,
+                                                        double* __restrict__ st, CT* __restrict__ mu_t) {
     __shared__ double ra[256], rb[256], rc[256];
+    __shared__ int off;
     double sa = 0.0, sb = 0.0, sc = 0.0;
+#pragma unroll 4
     for (int64_t q = threadIdx.x; q < n; q += 256) {
-        sa += (double)a[q * as];
-        sb += (double)b[q];
-        sc += (double)c[q];
+        sa += (double)feat[q * FS + 14];
+        sb += (double)eps[q];
+        sc += (double)oor[q];
     }
     ra[threadIdx.x] = sa;
     rb[threadIdx.x] = sb;
@@ -702,10 +720,27 @@ __global__ __launch_bounds__(256) void od_sum3_kernel(const float* __restrict__ 
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        out[0] = ra[0];
-        out[1] = rb[0];
-        out[2] = rc[0];
+        const double ke = ra[0], eps_now = rb[0];
+        bool active = true;
+        if (kappa > 0.0 && st[kKePrev] >= 0.0 && st[kActive] != 0.0) {
+            const double dke = st[kKePrev] - ke;                    // observed decay
+            const double work = st[kEpsPrev] * (*dt * interval);    // energy the model removed
+            if (dke > 0.0 && work > kappa * dke) active = false;
+        }
+        off = !active;
+        st[kKePrev] = ke;
+        st[kEpsPrev] = active ? eps_now : 0.0;
+        st[kActive] = active ? 1.0 : 0.0;
+        st[kStats + 0] += 1.0;
+        if (!active) st[kStats + 1] += 1.0;
+        st[kStats + 2] += rc[0];
+        st[kStats + 3] = ke;
+        st[kStats + 4] = eps_now;
+        st[kStats + 5] = active ? 1.0 : 0.0;
     }
+    __syncthreads();
+    if (off)
+        for (int64_t q = threadIdx.x; q < n; q += 256) mu_t[q] = (CT)0;
 }
 
 template <class CT>
@@ -730,6 +765,8 @@ struct od_mlp {
     float* grad = nullptr;    // NPARAM + 1
     unsigned short* wb = nullptr;  // bf16 copies: w1 | w2 | w3 | w2t | w3t | w4
     Scaling sc{};
+    std::mutex uses_mu;
+    std::vector<std::shared_ptr<od::UseEvent>> uses;  // of the solvers the network was attached to
     float* partial = nullptr;  // partial gradient rows of the largest batch so far (at most 1024)
     size_t partial_rows = 0;
     uint64_t adam_t = 0;
@@ -866,9 +903,10 @@ od_status ensure_closure_buffers(od_ctx* c) {
             return fail(OD_ERR_NOMEM, "closure buffers: allocation failed");
         c->device_bytes += (size_t)c->E * (FS + 2) * sizeof(float);
     }
-    if (!c->red) {
-        HIP_TRY(hipMalloc((void**)&c->red, 4 * sizeof(double)));
-        HIP_TRY(hipHostMalloc((void**)&c->red_host, 4 * sizeof(double), hipHostMallocDefault));
+    if (!c->budget) {
+        const double zero[kBudget] = {};
+        HIP_TRY(hipMalloc((void**)&c->budget, sizeof(zero)));
+        HIP_TRY(hipMemcpy(c->budget, zero, sizeof(zero), hipMemcpyHostToDevice));
     }
     return OD_OK;
 }
@@ -900,73 +938,84 @@ int launch_features(od_ctx* c) {
 
 }  // namespace
 
-// Refresh mu_t from the current state (called by od_step every
-// update_interval steps while a network is attached).  Defined here, used by
-// od_api.hip.
-od_status od_closure_update_internal(od_ctx* c, double dt_interval) {
-    od_status st = ensure_closure_buffers(c);
-    if (st == OD_OK) st = ensure_mu_t(c);
-    if (st != OD_OK) return st;
+namespace {
+
+// Everything a refresh is launched with that can change between two refreshes
+// of one attachment, as bytes.
+struct RefreshKey {
+    DevNet net;
+    Scaling sc;
+    int32_t interval;
+    double kappa;
+};
+static_assert(sizeof(RefreshKey) <= sizeof(od_ctx::closure_key), "room for the key");
+void refresh_key(const od_ctx* c, unsigned char* bytes) {
+    const DevNet net = dev_net(c->mlp);
+    std::memset(bytes, 0, sizeof(RefreshKey));  // padding too
+    std::memcpy(bytes + offsetof(RefreshKey, net), &net, sizeof(net));
+    std::memcpy(bytes + offsetof(RefreshKey, sc), &c->mlp->sc, sizeof(Scaling));
+    std::memcpy(bytes + offsetof(RefreshKey, interval), &c->closure.update_interval, sizeof(int32_t));
+    std::memcpy(bytes + offsetof(RefreshKey, kappa), &c->closure.budget_kappa, sizeof(double));
+}
+
+template <class CT>
+od_status enqueue_refresh(od_ctx* c) {
     if (launch_features(c)) return fail(OD_ERR_HIP, "od_features_kernel launch failed");
+    const float* feat = (const float*)c->feat;
     float* eps = (float*)c->feat + (size_t)c->E * FS;
     float* oor = eps + c->E;
     const unsigned blocks = (unsigned)std::min<int64_t>(2048, (c->E + 15) / 16);  // up to 8 groups a CU
-    const DevNet net = dev_net(c->mlp);
-    if (c->cbytes == 4)
-        hipLaunchKernelGGL(od_mlp_infer_kernel<float>, dim3(blocks), dim3(256), 0, c->stream, net, c->mlp->sc,
-                           (const float*)c->feat, c->E, (float*)c->mu_t, eps, oor);
-    else
-        hipLaunchKernelGGL(od_mlp_infer_kernel<double>, dim3(blocks), dim3(256), 0, c->stream, net, c->mlp->sc,
-                           (const float*)c->feat, c->E, (double*)c->mu_t, eps, oor);
+    hipLaunchKernelGGL(od_mlp_infer_kernel<CT>, dim3(blocks), dim3(256), 0, c->stream, dev_net(c->mlp), c->mlp->sc, feat,
+                       c->E, (CT*)c->mu_t, eps, oor);
     if (check()) return fail(OD_ERR_HIP, "od_mlp_infer_kernel launch failed");
-    // kinetic energy, model dissipation rate and out-of-range count (exact in f64)
-    hipLaunchKernelGGL(od_sum3_kernel, dim3(1), dim3(256), 0, c->stream, (const float*)c->feat + 14, FS,
-                       (const float*)eps, (const float*)oor, c->E, c->red);
-    if (check()) return fail(OD_ERR_HIP, "od_sum3_kernel launch failed");
-    HIP_TRY(hipMemcpyAsync(c->red_host, c->red, 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    const double ke = c->red_host[0], eps_now = c->red_host[1];
-    const int64_t n_oor = (int64_t)c->red_host[2];
-    // budget check over the interval that just ended
-    bool active = true;
-    if (c->closure.budget_kappa > 0.0 && c->ke_prev >= 0.0 && c->closure_active) {
-        // The model over-dissipates when, over an interval in which the kinetic
-        // energy decayed, the energy it removed exceeds kappa times the whole
-        // observed decay.  An interval in which the energy grew is not held
-        // against the model (it only removes energy).
-        const double dke = c->ke_prev - ke;               // observed decay
-        const double work = c->eps_prev * dt_interval;    // energy the model removed
-        if (dke > 0.0 && work > c->closure.budget_kappa * dke) active = false;
-    }
-    if (!active) {
-        const unsigned fb = (unsigned)((c->E + 255) / 256);
-        if (c->cbytes == 4)
-            hipLaunchKernelGGL(od_fill_kernel<float>, dim3(fb), dim3(256), 0, c->stream, (float*)c->mu_t, c->E);
-        else
-            hipLaunchKernelGGL(od_fill_kernel<double>, dim3(fb), dim3(256), 0, c->stream, (double*)c->mu_t, c->E);
-        if (check()) return fail(OD_ERR_HIP, "fill kernel launch failed");
-        c->closure_stats[1] += 1.0;
-    }
-    c->closure_active = active;
-    c->ke_prev = ke;
-    c->eps_prev = active ? eps_now : 0.0;
-    c->closure_stats[0] += 1.0;
-    c->closure_stats[2] += (double)n_oor;
-    c->closure_stats[3] = ke;
-    c->closure_stats[4] = eps_now;
-    c->closure_stats[5] = active ? 1.0 : 0.0;
+    hipLaunchKernelGGL(od_budget_kernel<CT>, dim3(1), dim3(256), 0, c->stream, feat, eps, oor, c->E, c->dt_value,
+                       (double)c->closure.update_interval, c->closure.budget_kappa, c->budget, (CT*)c->mu_t);
+    return check() ? fail(OD_ERR_HIP, "od_budget_kernel launch failed") : OD_OK;
+}
+
+// Drops the uses of solvers that are gone or attached anew (both wait for
+// their streams).
+void prune_uses(od_mlp* m) {
+    m->uses.erase(std::remove_if(m->uses.begin(), m->uses.end(), [](const auto& u) { return u.use_count() == 1; }),
+                  m->uses.end());
+}
+
+// Waits for the refreshes that still read the network's weights.
+void wait_for_uses(od_mlp* m) {
+    std::lock_guard<std::mutex> lk(m->uses_mu);
+    for (const auto& u : m->uses) (void)hipEventSynchronize(u->ev);
+    prune_uses(m);
+}
+
+}  // namespace
+
+// Enqueues a refresh of mu_t from the current state (od_step, every
+// update_interval steps while a network is attached).
+od_status od_closure_refresh_internal(od_ctx* c) {
+    return c->cbytes == 4 ? enqueue_refresh<float>(c) : enqueue_refresh<double>(c);
+}
+
+bool od_closure_key_changed_internal(od_ctx* c) {
+    unsigned char key[sizeof(RefreshKey)];
+    refresh_key(c, key);
+    if (std::memcmp(key, c->closure_key, sizeof(key)) == 0) return false;
+    std::memcpy(c->closure_key, key, sizeof(key));
+    return true;
+}
+
+od_status od_closure_used_internal(od_ctx* c) {
+    HIP_TRY(hipEventRecord(c->mlp_use->ev, c->stream));
     return OD_OK;
 }
 
 void od_closure_release_internal(od_ctx* c) {
     if (c->feat) (void)hipFree(c->feat);
-    if (c->red) (void)hipFree(c->red);
-    if (c->red_host) (void)hipHostFree(c->red_host);
+    if (c->budget) (void)hipFree(c->budget);
     if (c->mu_t) (void)hipFree(c->mu_t);
     c->feat = nullptr;
-    c->red = nullptr;
-    c->red_host = nullptr;
+    c->budget = nullptr;
     c->mu_t = nullptr;
+    c->mlp_use.reset();
 }
 
 extern "C" {
@@ -1022,6 +1071,7 @@ od_status od_mlp_create(int device, od_mlp** out) {
 void od_mlp_destroy(od_mlp* m) {
     if (!m) return;
     (void)hipSetDevice(m->device);
+    wait_for_uses(m);
     if (m->stream) (void)hipStreamSynchronize(m->stream);
     for (void* q : {(void*)m->params, (void*)m->adam_m, (void*)m->adam_v, (void*)m->grad, (void*)m->wb,
                     (void*)m->partial})
@@ -1034,6 +1084,7 @@ od_status od_mlp_set_params(od_mlp* m, const float* params, size_t n) {
     if (!m || !params) return fail(OD_ERR_INVALID, "od_mlp_set_params: null argument");
     if (n != (size_t)NPARAM) return fail(OD_ERR_INVALID, "od_mlp_set_params: expected OD_MLP_PARAMS values");
     HIP_TRY(hipSetDevice(m->device));
+    wait_for_uses(m);
     HIP_TRY(hipStreamSynchronize(m->stream));
     HIP_TRY(hipMemcpy(m->params, params, NPARAM * sizeof(float), hipMemcpyHostToDevice));
     HIP_TRY(hipMemsetAsync(m->adam_m, 0, NPARAM * sizeof(float), m->stream));
@@ -1117,6 +1168,7 @@ od_status od_mlp_train(od_mlp* m, const float* x, const float* t, size_t n, uint
     if (n == 0 || batch == 0) return fail(OD_ERR_INVALID, "od_mlp_train: empty data or batch");
     if (n > (size_t)0x7fffffff) return fail(OD_ERR_INVALID, "od_mlp_train: too many samples");
     HIP_TRY(hipSetDevice(m->device));
+    wait_for_uses(m);
     // Two epochs are in flight: while the device works through one, the host
     // orders the next one's samples.  Each slot has its index array, the sums of
     // squared errors of its batches and an event at the end of its work.
@@ -1261,20 +1313,33 @@ od_status od_closure_attach(od_ctx* c, od_mlp* m, const od_closure_opts* opts) {
     od_status s = ensure_closure_buffers(c);
     if (s == OD_OK) s = ensure_mu_t(c);
     if (s != OD_OK) return s;
+    // a fresh budget: no previous energy, nothing removed, active
+    double st[kBudget] = {};
+    st[kKePrev] = -1.0;
+    st[kActive] = 1.0;
+    HIP_TRY(hipMemcpy(c->budget, st, sizeof(st), hipMemcpyHostToDevice));
+    auto use = std::make_shared<od::UseEvent>();
+    HIP_TRY(hipEventCreateWithFlags(&use->ev, hipEventDisableTiming));
+    {
+        std::lock_guard<std::mutex> lk(m->uses_mu);
+        prune_uses(m);
+        m->uses.push_back(use);
+    }
+    c->mlp_use = use;
     c->mlp = m;
     c->closure = *opts;
     c->steps_done = 0;
-    c->ke_prev = -1.0;
-    c->eps_prev = 0.0;
-    c->closure_active = true;
-    for (double& v : c->closure_stats) v = 0.0;
     c->mu_t_on = true;
     return OD_OK;
 }
 
 od_status od_closure_stats(od_ctx* c, double out[6]) {
     if (!c || !out) return fail(OD_ERR_INVALID, "od_closure_stats: null argument");
-    for (int q = 0; q < 6; ++q) out[q] = c->closure_stats[q];
+    for (int q = 0; q < 6; ++q) out[q] = 0.0;
+    if (!c->budget) return OD_OK;
+    HIP_TRY(hipSetDevice(c->device));
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    HIP_TRY(hipMemcpy(out, c->budget + kStats, 6 * sizeof(double), hipMemcpyDeviceToHost));
     return OD_OK;
 }
 

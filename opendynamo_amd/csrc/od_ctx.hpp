@@ -3,9 +3,21 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <memory>
 
 #include "od_host.hpp"
 #include "od_slots.hpp"
+
+namespace od {
+// The last use of a network by a solver's stream, shared by both so that
+// either may go first: the network waits for it before its weights change.
+struct UseEvent {
+    hipEvent_t ev = nullptr;
+    ~UseEvent() {
+        if (ev) (void)hipEventDestroy(ev);
+    }
+};
+}  // namespace od
 
 struct od_ctx {
     od_params p;
@@ -17,15 +29,17 @@ struct od_ctx {
     void* tr[3] = {nullptr, nullptr, nullptr};
     void* fv = nullptr;
     void* dbg = nullptr;
-    double* sums_partial = nullptr;
-    double* sums_out = nullptr;
-    double* cfl_partial = nullptr;  // od::kCflGroups doubles
+    double* sums_partial = nullptr;  // [5][E], then (one allocation):
+    double* sums_out = nullptr;      // 8 doubles
+    double* cfl_partial = nullptr;   // od::kCflGroups doubles
     od::host::HostOps ops;
     bool state_set = false;
     bool blocks = false;               // step kernels on 2x2x2-element blocks (fast f32, even dims),
                                        // which store the traces of the blocks' external faces only
     hipGraphExec_t graph = nullptr;    // one RK3 step
     hipGraphExec_t graph_k = nullptr;  // kStepsPerGraph RK3 steps
+    hipGraphExec_t graph_c = nullptr;  // closure: a refresh of mu_t and one interval's steps
+    double* dt_value = nullptr;        // dt on the device, and behind it
     void* dt_table = nullptr;          // StageDt[3] that the graphs' kernels read
     double table_dt = 0.0;             // the dt it holds (in stream order), 0: none yet
     void* pinned[3] = {nullptr, nullptr, nullptr};
@@ -47,15 +61,14 @@ struct od_ctx {
     od_mlp* mlp = nullptr;        // attached network (not owned)
     od_closure_opts closure{};    // attach options
     uint64_t steps_done = 0;      // steps since attach (update cadence)
-    double ke_prev = -1.0;        // kinetic energy at the previous update
-    double eps_prev = 0.0;        // model dissipation rate applied since then
-    bool closure_active = false;  // false: budget fallback, plain FR until the next update
-    double closure_stats[6] = {0, 0, 0, 0, 0, 0};
     void* feat = nullptr;         // [E][16] features, then eps [E] and out-of-range flags [E] (f32)
-    double* red = nullptr;        // budget-check reductions (device)
-    double* red_host = nullptr;   // pinned copy
+    double* budget = nullptr;     // budget check's state on the device (od_closure.hip)
+    unsigned char closure_key[512] = {};      // what graph_c's refresh was captured with
+    std::shared_ptr<od::UseEvent> mlp_use;   // recorded after the last refresh enqueued
 };
 
-// Closure refresh and release (od_closure.hip), used by od_step / od_destroy.
-od_status od_closure_update_internal(od_ctx* c, double dt_interval);
+// The closure's part of od_step / od_destroy (od_closure.hip).
+od_status od_closure_refresh_internal(od_ctx* c);     // enqueues a refresh of mu_t
+bool od_closure_key_changed_internal(od_ctx* c);      // since the last call
+od_status od_closure_used_internal(od_ctx* c);        // marks the network as read up to here
 void od_closure_release_internal(od_ctx* c);

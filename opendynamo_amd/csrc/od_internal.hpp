@@ -126,9 +126,9 @@ int launch_batch_update(const StageArgs<UT, CT>& a, const BatchArgs<UT, CT>& b, 
 // Resident work-groups per CU of a batch kernel (kind 0 visc, 1 update).
 template <class UT, class CT>
 int batch_occupancy(int kind, int pairs, bool visc, int* groups_per_cu);
-// The three stages' c * dt -> table, in stream order.
+// The three stages' c * dt -> table, and dt itself, in stream order.
 template <class UT, class CT>
-int launch_set_dt(StageDt<UT, CT>* table, const StageDt<UT, CT> v[3], void* stream);
+int launch_set_dt(StageDt<UT, CT>* table, const StageDt<UT, CT> v[3], double* dt_value, double dt, void* stream);
 // Largest sum over d of (|u_d| + c) / dx_d of the points of each work-group, in
 // f64, -> partial[groups] (host: their maximum); groups = cfl_groups(n_elem).
 constexpr int kCflGroups = 1024;

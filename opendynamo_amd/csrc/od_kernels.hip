@@ -2349,9 +2349,11 @@ struct DtTable {
     StageDt<UT, CT> s[3];
 };
 template <class UT, class CT>
-__global__ void od_set_dt_kernel(StageDt<UT, CT>* table, DtTable<UT, CT> v) {
-    if (threadIdx.x == 0 && blockIdx.x == 0)
+__global__ void od_set_dt_kernel(StageDt<UT, CT>* table, DtTable<UT, CT> v, double* dt_value, double dt) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) {
         for (int s = 0; s < 3; ++s) table[s] = v.s[s];
+        *dt_value = dt;
+    }
 }
 
 // The largest signal speed of the CFL condition, in f64 from the state's values
@@ -2515,10 +2517,10 @@ int launch_sums(const UT* u, double* partial, double* out, int64_t n_elem, const
 
 #if !OD_FAST
 template <class UT, class CT>
-int launch_set_dt(StageDt<UT, CT>* table, const StageDt<UT, CT> v[3], void* stream) {
+int launch_set_dt(StageDt<UT, CT>* table, const StageDt<UT, CT> v[3], double* dt_value, double dt, void* stream) {
     DtTable<UT, CT> t;
     for (int s = 0; s < 3; ++s) t.s[s] = v[s];
-    hipLaunchKernelGGL((od_set_dt_kernel<UT, CT>), dim3(1), dim3(64), 0, (hipStream_t)stream, table, t);
+    hipLaunchKernelGGL((od_set_dt_kernel<UT, CT>), dim3(1), dim3(64), 0, (hipStream_t)stream, table, t, dt_value, dt);
     return check_launch();
 }
 template <class UT>
@@ -2557,10 +2559,10 @@ OD_INST(float, double)
 #endif
 #undef OD_INST
 #if !OD_FAST
-template int launch_set_dt<float, float>(StageDt<float, float>*, const StageDt<float, float>*, void*);
-template int launch_set_dt<double, float>(StageDt<double, float>*, const StageDt<double, float>*, void*);
-template int launch_set_dt<double, double>(StageDt<double, double>*, const StageDt<double, double>*, void*);
-template int launch_set_dt<float, double>(StageDt<float, double>*, const StageDt<float, double>*, void*);
+template int launch_set_dt<float, float>(StageDt<float, float>*, const StageDt<float, float>*, double*, double, void*);
+template int launch_set_dt<double, float>(StageDt<double, float>*, const StageDt<double, float>*, double*, double, void*);
+template int launch_set_dt<double, double>(StageDt<double, double>*, const StageDt<double, double>*, double*, double, void*);
+template int launch_set_dt<float, double>(StageDt<float, double>*, const StageDt<float, double>*, double*, double, void*);
 template int launch_cfl<float>(const float*, double*, int64_t, double, double, double, void*);
 template int launch_cfl<double>(const double*, double*, int64_t, double, double, double, void*);
 template int launch_sums<float>(const float*, double*, double*, int64_t, const double*, double, void*);
