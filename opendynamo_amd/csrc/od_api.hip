@@ -105,6 +105,17 @@ HostOps fr_operators() {
     return o;
 }
 
+int launch_block_form(const od::StageArgs<float, float>& a, bool viscous, int kind, hipStream_t stream) {
+    if (a.nx % 2 == 0 && a.ny % 2 == 0 && a.nz % 2 == 0) {
+        if (kind == 0) return od::fastmath::launch_visc_block(a, stream);
+        return viscous ? od::fastmath::launch_update_block<true>(a, stream)
+                       : od::fastmath::launch_update_block<false>(a, stream);
+    }
+    if (kind == 0) return od::fastmath::launch_visc_core_shell(a, stream);
+    return viscous ? od::fastmath::launch_update_core_shell<true>(a, stream)
+                   : od::fastmath::launch_update_core_shell<false>(a, stream);
+}
+
 od_status cfl_dt_of_state(const void* u, int u_real, int64_t E, double dx, double dy, double dz, double cfl,
                           double* partial, hipStream_t stream, double* dt_out) {
     const int rc = u_real == OD_F32 ? od::launch_cfl<float>((const float*)u, partial, E, dx, dy, dz, stream)
@@ -154,10 +165,8 @@ int launch_kind(od_ctx* c, int kind, int stage, double dt, int mode) {
     if constexpr (sizeof(CT) == 4) {
         if (c->p.fast_math) {
             if constexpr (sizeof(UT) == 4) {
-                if (kind == 0 && c->blocks) return od::fastmath::launch_visc_block(a, c->stream);
-                if (kind == 1 && c->blocks)
-                    return c->p.viscous ? od::fastmath::launch_update_block<true>(a, true, c->stream)
-                                        : od::fastmath::launch_update_block<false>(a, true, c->stream);
+                if (box_form(c->p, c->p.nx, c->p.ny, c->p.nz) != BoxForm::tiles)
+                    return launch_block_form(a, c->p.viscous != 0, kind, c->stream);
             }
             if (kind == 0) return od::fastmath::launch_visc<UT, CT>(a, c->E, c->stream);
             if (c->p.viscous) return od::fastmath::launch_update<UT, CT, true>(a, c->E, c->stream);
@@ -348,9 +357,6 @@ od_status od_create(const od_params* p, int device, od_ctx** out) {
     c->NP = E * 64;
     c->ubytes = (size_t)p->u_real;
     c->cbytes = (size_t)p->compute_real;
-    // fast f32 with even dimensions: the step kernels on 2x2x2-element blocks
-    c->blocks = p->fast_math && p->u_real == OD_F32 && p->compute_real == OD_F32 && p->nx % 2 == 0 &&
-                p->ny % 2 == 0 && p->nz % 2 == 0;
     c->ops = fr_operators();
     {
         const od::Ops<float> of = cast_ops<float>(c->ops);
@@ -653,8 +659,10 @@ od_status od_time_kernels(od_ctx* c, double dt, uint32_t n_steps, double out_ms[
     for (int k = 0; k < 4; ++k) {
         out_ms[k] = (k < kinds && cnt[k]) ? sum[k] / cnt[k] : 0.0;
         const char* nm = k < kinds ? od::kernel_name(k) : "";
-        if (k == 0 && c->blocks) nm = "od_visc_block_kernel";
-        if (k == 1 && c->blocks) nm = "od_update_block_kernel";
+        const BoxForm form = box_form(c->p, c->p.nx, c->p.ny, c->p.nz);
+        if (form == BoxForm::blocks) nm = k == 0 ? "od_visc_block_kernel" : k == 1 ? "od_update_block_kernel" : nm;
+        if (form == BoxForm::core_shell)
+            nm = k == 0 ? "od_visc_core_shell_kernel" : k == 1 ? "od_update_core_shell_kernel" : nm;
         if (names) names[k] = nm;
     }
     if (n_kinds) *n_kinds = kinds;

@@ -34,8 +34,6 @@ struct od_ctx {
     double* cfl_partial = nullptr;   // od::kCflGroups doubles
     od::host::HostOps ops;
     bool state_set = false;
-    bool blocks = false;               // step kernels on 2x2x2-element blocks (fast f32, even dims),
-                                       // which store the traces of the blocks' external faces only
     hipGraphExec_t graph = nullptr;    // one RK3 step
     hipGraphExec_t graph_k = nullptr;  // kStepsPerGraph RK3 steps
     hipGraphExec_t graph_c = nullptr;  // closure: a refresh of mu_t and one interval's steps

@@ -46,6 +46,19 @@ od::Ops<C> cast_ops(const HostOps& h) {
 // Whether a context's kernels are the fast build's: f32 compute with fast_math.
 inline bool fast_kernels(const od_params& p) { return p.fast_math && p.compute_real == OD_F32; }
 
+// The kernels a box runs on when it is stepped by itself: fast f32 boxes at
+// least 2 elements wide in each direction on 2x2x2-element blocks, with the
+// last layer along each odd dimension on two-element tiles in the same launch;
+// all others on tiles.
+enum class BoxForm { tiles, blocks, core_shell };
+inline BoxForm box_form(const od_params& p, int nx, int ny, int nz) {
+    if (!p.fast_math || p.u_real != OD_F32 || p.compute_real != OD_F32 || nx < 2 || ny < 2 || nz < 2)
+        return BoxForm::tiles;
+    return nx % 2 || ny % 2 || nz % 2 ? BoxForm::core_shell : BoxForm::blocks;
+}
+// Launch of kind 0 visc, 1 update of a box whose form is not tiles.
+int launch_block_form(const od::StageArgs<float, float>& a, bool viscous, int kind, hipStream_t stream);
+
 inline bool real_ok(int r) { return r == OD_F32 || r == OD_F64; }
 
 template <class Dst, class Src>

@@ -101,6 +101,14 @@ struct BatchArgs {
     int32_t tile_off[kInlineBoxes];  // first tile of each box (n_boxes <= kInlineBoxes)
 };
 
+// Two-element tiles of the shell of a box (its last layer along each odd
+// dimension): the x slab paired along y, the rest of the y and z slabs paired
+// along x.
+inline int64_t shell_tiles(int64_t nx, int64_t ny, int64_t nz) {
+    const int64_t hx = nx / 2, hy = (ny + 1) / 2, cy = ny & ~(int64_t)1;
+    return (nx % 2 ? hy * nz : 0) + (ny % 2 ? hx * nz : 0) + (nz % 2 ? hx * cy : 0);
+}
+
 // The boxes of a batch whose core runs on 2x2x2-element blocks (fast f32
 // build; the core is the box less the last layer along each odd dimension):
 // blk_off[i] = the first block of box i in the batch block numbering (a box
@@ -159,11 +167,16 @@ int batch_occupancy(int kind, int pairs, bool visc, int* groups_per_cu);
 int upload_ops(const Ops<float>& f32, const Ops<double>& f64);
 // Kernels on blocks of 2x2x2 elements (f32 state and compute, nx, ny, nz
 // even): the same results as launch_update / launch_visc, bit for bit.
-// ext_traces: the update kernel writes the traces of the blocks' external
-// faces only, which is all the block visc kernel reads.
+// The update kernel writes the traces of the blocks' external faces only, which
+// is all the block visc kernel reads.
 template <bool VISC>
-int launch_update_block(const StageArgs<float, float>& a, bool ext_traces, void* stream);
+int launch_update_block(const StageArgs<float, float>& a, void* stream);
 int launch_visc_block(const StageArgs<float, float>& a, void* stream);
+// A box with an odd dimension, none below 2: its core on blocks and the rest on
+// tiles, in one launch.
+template <bool VISC>
+int launch_update_core_shell(const StageArgs<float, float>& a, void* stream);
+int launch_visc_core_shell(const StageArgs<float, float>& a, void* stream);
 // The same kernels over every block box of a batch, one launch each.
 template <bool VISC>
 int launch_batch_update_block(const StageArgs<float, float>& a, const BlockBatch& bb, void* stream);

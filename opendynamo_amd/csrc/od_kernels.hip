@@ -1538,15 +1538,14 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(kMinWavesUp
 
 #if OD_FAST
 // ---------------------------------------------------------------------------
-// Fast f32 build, one box with even nx, ny, nz: the update kernel on blocks
-// of 2x2x2 elements (512 threads; wave w owns local element w = lx + 2 ly +
+// Fast f32 build: the update kernel on blocks of 2x2x2 elements (512 threads; wave w owns local element w = lx + 2 ly +
 // 4 lz in the point-wise phases).  Three of an element's six faces face
 // another element of the block.  Their neighbour traces come from the
 // block's LDS state tiles instead of HBM, and the interface flux of such an
 // internal face is evaluated once for both of its elements.  Every value is
 // formed from the same operands in the same order as in update_body, so each
-// element gets the same bits as in the two-element-tile kernels (which the
-// ensemble kernels and meshes with an odd dimension use).
+// element gets the same bits as in the two-element-tile kernels (which take the
+// last layers of boxes with an odd dimension, and boxes 1 element wide).
 // ---------------------------------------------------------------------------
 constexpr int kBlk = 8;
 
@@ -1736,11 +1735,11 @@ __device__ __forceinline__ void blk_int_pass(const StageArgs<float, float>& a, c
     }
 }
 
-// EXT: write the new state's traces of the external faces only (the block
-// visc kernel forms the internal ones from its LDS state tiles).
-template <bool VISC, bool EXT>
-__device__ __forceinline__ void update_block_body(const StageArgs<float, float>& a, const Block& b) {
-    __shared__ BlockUpdateLds L;
+// The new state's traces are written on the external faces only (the block visc
+// kernel forms the internal ones from its LDS state tiles).
+template <bool VISC>
+__device__ __forceinline__ void update_block_body(const StageArgs<float, float>& a, const Block& b,
+                                                  BlockUpdateLds& L) {
     const int wave = wave_index(), pt = threadIdx.x & 63;
     const int i = pt & 3, j = (pt >> 2) & 3, k = pt >> 4;
     const int64_t NP = (int64_t)a.nx * a.ny * a.nz * 64;
@@ -1885,11 +1884,7 @@ __device__ __forceinline__ void update_block_body(const StageArgs<float, float>&
 #pragma unroll
     for (int v = 0; v < 5; ++v) L.sU[wave][v][pt] = unew[v];
     wave_sync();
-    if constexpr (EXT) {
-        blk_write_ext_traces(L.sU[wave], a.tr_out + e * kTraceStride, wave, pt);
-    } else {
-        write_traces_own<float, true>(L.sU[wave], a.tr_out + e * kTraceStride, pt, VISC);
-    }
+    blk_write_ext_traces(L.sU[wave], a.tr_out + e * kTraceStride, wave, pt);
 }
 
 // ---------------------------------------------------------------------------
@@ -1983,8 +1978,7 @@ __device__ __forceinline__ void blk_fv_pass(const StageArgs<float, float>& a, co
     }
 }
 
-__device__ __forceinline__ void visc_block_body(const StageArgs<float, float>& a, const Block& b) {
-    __shared__ BlockViscLds L;
+__device__ __forceinline__ void visc_block_body(const StageArgs<float, float>& a, const Block& b, BlockViscLds& L) {
     const int wave = wave_index(), pt = threadIdx.x & 63;
     const int i = pt & 3, j = (pt >> 2) & 3, k = pt >> 4;
     const int64_t NP = (int64_t)a.nx * a.ny * a.nz * 64;
@@ -2036,13 +2030,15 @@ __device__ __forceinline__ void visc_block_body(const StageArgs<float, float>& a
 
 // One box: the update kernel walks the blocks backwards, the visc kernel
 // forwards (make_block).
-template <bool VISC, bool EXT>
+template <bool VISC>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8))) void od_update_block_kernel(
     StageArgs<float, float> a) {
-    update_block_body<VISC, EXT>(a, make_block<true>(a));
+    __shared__ BlockUpdateLds L;
+    update_block_body<VISC>(a, make_block<true>(a), L);
 }
 __global__ __launch_bounds__(512) void od_visc_block_kernel(StageArgs<float, float> a) {
-    visc_block_body(a, make_block<false>(a));
+    __shared__ BlockViscLds L;
+    visc_block_body(a, make_block<false>(a), L);
 }
 #endif
 
@@ -2175,6 +2171,16 @@ __device__ __forceinline__ void batch_tile(const StageArgs<UT, CT>& a, const Bat
 }
 
 #if OD_FAST
+// Block lb of a box's core, x fastest.
+__device__ __forceinline__ Block core_block(const StageArgs<float, float>& a, int lb) {
+    Block b;
+    const int gx = a.nx >> 1, gy = a.ny >> 1;
+    b.ex0 = 2 * (lb % gx);
+    b.ey0 = 2 * ((lb / gx) % gy);
+    b.ez0 = 2 * (lb / (gx * gy));
+    b.e0 = b.ex0 + a.nx * (b.ey0 + a.ny * b.ez0);
+    return b;
+}
 // Ensembles on 2x2x2-element blocks: the core of every box (the box less the
 // last layer along each odd dimension; the whole box when all are even) runs
 // the block kernels, one launch per phase for all boxes, and the shell the
@@ -2212,12 +2218,7 @@ __device__ __forceinline__ void batch_block(const StageArgs<float, float>& a, co
         off = uni(bb.boxes[lo].blk_off);
     }
     batch_box_args(a, bb.boxes[lo], bb.stage, ab);
-    const int lb = t - off;
-    const int gx = ab.nx >> 1, gy = ab.ny >> 1;
-    b.ex0 = 2 * (lb % gx);
-    b.ey0 = 2 * ((lb / gx) % gy);
-    b.ez0 = 2 * (lb / (gx * gy));
-    b.e0 = b.ex0 + ab.nx * (b.ey0 + ab.ny * b.ez0);
+    b = core_block(ab, t - off);
 }
 
 template <bool VISC>
@@ -2226,14 +2227,65 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8))) void o
     StageArgs<float, float> ab;
     Block b;
     batch_block<true>(a, bb, ab, b);
-    update_block_body<VISC, true>(ab, b);
+    __shared__ BlockUpdateLds L;
+    update_block_body<VISC>(ab, b, L);
 }
 
 __global__ __launch_bounds__(512) void od_batch_visc_block_kernel(StageArgs<float, float> a, BlockBatch bb) {
     StageArgs<float, float> ab;
     Block b;
     batch_block<false>(a, bb, ab, b);
-    visc_block_body(ab, b);
+    __shared__ BlockViscLds L;
+    visc_block_body(ab, b, L);
+}
+
+// One box with an odd dimension: its core on blocks and its shell on tiles in
+// one launch.  A 512-thread work-group takes a block of the core, or four tiles
+// of the shell (which need as much LDS: 10.4 KB each in the visc kernel, 9.1 KB
+// in the update kernel).  The blocks come first (the update kernel's backwards,
+// as in the even boxes) and the shell, a small part of the box, fills up the
+// last work-groups' wave; a launch of its own would cost its latency twice a
+// stage.  33x25x37 (AUSM+, 100 steps): 37.4 ms with every element on tiles,
+// 33.6 here.
+struct CoreShell {
+    int32_t n_blocks, n_tiles;  // blocks of the core, tiles of the shell
+};
+// Tile of this 128-thread part of shell work-group `group`; past the shell's
+// end an empty one.
+__device__ __forceinline__ Tile core_shell_tile(const StageArgs<float, float>& a, const CoreShell& cs, int group) {
+    const int lt = uni(4 * group + (int)(threadIdx.x >> 7));
+    const bool ok = lt < cs.n_tiles;
+    Tile tl = shell_tile(a, ok ? lt : 0);
+    tl.v0 = ok;
+    tl.v1 = ok && tl.v1;
+    return tl;
+}
+
+template <bool VISC>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8))) void od_update_core_shell_kernel(
+    StageArgs<float, float> a, CoreShell cs) {
+    __shared__ union {
+        BlockUpdateLds block;
+        UpdateLds<float, VISC> tile[4];
+    } L;
+    const int w = (int)blockIdx.x;
+    if (w < cs.n_blocks)
+        update_block_body<VISC>(a, core_block(a, cs.n_blocks - 1 - w), L.block);
+    else
+        update_body<float, float, VISC>(a, core_shell_tile(a, cs, w - cs.n_blocks), L.tile[threadIdx.x >> 7],
+                                        wave_index() & 1, threadIdx.x & 63);
+}
+__global__ __launch_bounds__(512) void od_visc_core_shell_kernel(StageArgs<float, float> a, CoreShell cs) {
+    __shared__ union {
+        BlockViscLds block;
+        ViscLds<float> tile[4];
+    } L;
+    const int w = (int)blockIdx.x;
+    if (w < cs.n_blocks)
+        visc_block_body(a, core_block(a, w), L.block);
+    else
+        visc_body(a, core_shell_tile(a, cs, w - cs.n_blocks), L.tile[threadIdx.x >> 7], wave_index() & 1,
+                  threadIdx.x & 63);
 }
 #endif
 
@@ -2409,22 +2461,45 @@ inline dim3 block_grid(const StageArgs<float, float>& a) {
 }
 
 template <bool VISC>
-int launch_update_block(const StageArgs<float, float>& a, bool ext_traces, void* stream) {
+int launch_update_block(const StageArgs<float, float>& a, void* stream) {
     if (a.nx % 2 || a.ny % 2 || a.nz % 2) return 1;  // blocks of 2x2x2 elements tile the box exactly
-    if (ext_traces)
-        hipLaunchKernelGGL((od_update_block_kernel<VISC, true>), block_grid(a), dim3(64 * kBlk), 0,
-                           (hipStream_t)stream, a);
-    else
-        hipLaunchKernelGGL((od_update_block_kernel<VISC, false>), block_grid(a), dim3(64 * kBlk), 0,
-                           (hipStream_t)stream, a);
+    hipLaunchKernelGGL((od_update_block_kernel<VISC>), block_grid(a), dim3(64 * kBlk), 0, (hipStream_t)stream, a);
     return check_launch();
 }
-template int launch_update_block<true>(const StageArgs<float, float>&, bool, void*);
-template int launch_update_block<false>(const StageArgs<float, float>&, bool, void*);
+template int launch_update_block<true>(const StageArgs<float, float>&, void*);
+template int launch_update_block<false>(const StageArgs<float, float>&, void*);
 
 int launch_visc_block(const StageArgs<float, float>& a, void* stream) {
     if (a.nx % 2 || a.ny % 2 || a.nz % 2) return 1;
     hipLaunchKernelGGL(od_visc_block_kernel, block_grid(a), dim3(64 * kBlk), 0, (hipStream_t)stream, a);
+    return check_launch();
+}
+namespace {
+// Blocks and shell tiles of a box at least 2 elements wide in each direction.
+CoreShell core_shell(const StageArgs<float, float>& a) {
+    CoreShell cs;
+    cs.n_blocks = (a.nx / 2) * (a.ny / 2) * (a.nz / 2);
+    cs.n_tiles = (int32_t)shell_tiles(a.nx, a.ny, a.nz);
+    return cs;
+}
+dim3 core_shell_grid(const CoreShell& cs) { return dim3((unsigned)(cs.n_blocks + (cs.n_tiles + 3) / 4)); }
+}  // namespace
+
+template <bool VISC>
+int launch_update_core_shell(const StageArgs<float, float>& a, void* stream) {
+    if (a.nx < 2 || a.ny < 2 || a.nz < 2) return 1;
+    const CoreShell cs = core_shell(a);
+    hipLaunchKernelGGL((od_update_core_shell_kernel<VISC>), core_shell_grid(cs), dim3(64 * kBlk), 0,
+                       (hipStream_t)stream, a, cs);
+    return check_launch();
+}
+template int launch_update_core_shell<true>(const StageArgs<float, float>&, void*);
+template int launch_update_core_shell<false>(const StageArgs<float, float>&, void*);
+
+int launch_visc_core_shell(const StageArgs<float, float>& a, void* stream) {
+    if (a.nx < 2 || a.ny < 2 || a.nz < 2) return 1;
+    const CoreShell cs = core_shell(a);
+    hipLaunchKernelGGL(od_visc_core_shell_kernel, core_shell_grid(cs), dim3(64 * kBlk), 0, (hipStream_t)stream, a, cs);
     return check_launch();
 }
 template <bool VISC>
