@@ -273,6 +273,65 @@ __device__ __forceinline__ void viscous_flux(int d, const C* s, const C* g, C mu
     viscous_flux_dir(d, viscous_point(s, g, mu, 1 << d), f);
 }
 
+#if OD_FAST
+// The fast build's viscous fluxes, every fusion written out, so that the tile
+// and the block kernels form the same bits.  The heat flux takes the gradient
+// of the internal energy e = E / rho - |u|^2 / 2 (its p / rho is (gamma - 1) e):
+//   grad e = (grad E - (E / rho) grad rho) / rho - sum_a u_a grad u_a,
+// from the velocity gradients that the stresses need anyway, where the
+// reference's form (heat_flux above, the strict build's) goes through the
+// gradients of the kinetic energy and the pressure: 10 instructions fewer a
+// face point and 27 a solution point.
+struct FastVisc {
+    float r, u[3], er;  // 1 / rho, velocity, E / rho
+    float G[3][3];      // du_a / dx_b
+    float h[3];         // grad e
+    float mu;
+};
+// s: state, g: its gradient [var][3].  e: the element, for its eddy viscosity.
+template <class Args>
+__device__ __forceinline__ FastVisc fast_visc(const Args& a, const float* s, const float* g, int64_t e) {
+#pragma clang fp contract(off)
+    FastVisc f;
+    f.r = __builtin_amdgcn_rcpf(s[0]);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) f.u[c] = s[1 + c] * f.r;
+    f.er = s[4] * f.r;
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int b = 0; b < 3; ++b) f.G[c][b] = __builtin_fmaf(-f.u[c], g[b], g[3 * (c + 1) + b]) * f.r;
+#pragma unroll
+    for (int b = 0; b < 3; ++b) {
+        const float x = __builtin_fmaf(-f.er, g[b], g[12 + b]) * f.r;
+        f.h[b] = __builtin_fmaf(-f.u[2], f.G[2][b], __builtin_fmaf(-f.u[1], f.G[1][b], __builtin_fmaf(-f.u[0], f.G[0][b], x)));
+    }
+    f.mu = a.mu;
+    if (a.sutherland) {  // theta = gamma p / rho, p as in pressure()
+        const float k = __builtin_fmaf(f.u[2], f.u[2], __builtin_fmaf(f.u[1], f.u[1], f.u[0] * f.u[0]));
+        const float th = fmaxf((1.4f * gamma_m1<float>()) * __builtin_fmaf(-0.5f, k, f.er), 1.4e-7f * f.r);
+        f.mu = (a.mu_ref * (a.t_ref + a.s_suth)) * (th * __builtin_amdgcn_sqrtf(th)) *
+               __builtin_amdgcn_rcpf(__builtin_fmaf(a.t_ref, th, a.s_suth));
+    }
+    if (a.mu_t) f.mu = f.mu + a.mu_t[e];
+    return f;
+}
+// Components 1..4 of the viscous flux along d.
+__device__ __forceinline__ void fast_visc_flux(int d, const FastVisc& f, float* out) {
+#pragma clang fp contract(off)
+    const float div = (f.G[0][0] + f.G[1][1]) + f.G[2][2];
+    float t[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+        t[c] = f.mu * (c == d ? __builtin_fmaf(-2.0f / 3.0f, div, 2.0f * f.G[c][c]) : f.G[c][d] + f.G[d][c]);
+    out[0] = t[0];
+    out[1] = t[1];
+    out[2] = t[2];
+    const float q = (f.mu * (1.4f / 0.72f)) * sel3(f.h[0], f.h[1], f.h[2], d);
+    out[3] = __builtin_fmaf(f.u[0], t[0], __builtin_fmaf(f.u[1], t[1], __builtin_fmaf(f.u[2], t[2], q)));
+}
+#endif
+
 template <class C>
 __device__ __forceinline__ C sound_speed(C p, Recip<C> ir) {
     OD_CONTRACT_IN_EXPRESSIONS
@@ -583,9 +642,9 @@ __device__ __forceinline__ constexpr int br1_order(int d) { return (d == 2 && !k
 // 663-674, 716-727): x sequential from the first product, y pairwise, z from 0.
 __device__ __forceinline__ constexpr int face_order(int d) { return kOneX ? 0 : (d == 0 ? 2 : (d == 1 ? 0 : 1)); }
 // Order of the state and gradient traces the viscous face fluxes take: the
-// reference's face order; the fast build, whose viscous traces are formed and
-// used inside one kernel, takes the fused sequential form (one instruction
-// fewer per trace than the pairwise one).
+// reference's face order; the fast build takes the state traces of BR1 and, for
+// the gradient's, which are formed and used inside one kernel, the fused
+// sequential form (one instruction fewer per trace than the pairwise one).
 __device__ __forceinline__ constexpr int fv_order(int d) { return kOneX ? 1 : face_order(d); }
 // Faces of the trace layout the build writes, and the direction and order of face f.
 constexpr int kOwnFaces = kOneX ? 6 : 8;
@@ -851,9 +910,9 @@ __device__ __forceinline__ void lane_gradient_faces(const StageArgs<UT, CT>& a, 
         for (int m = 0; m < 4; ++m) deta += Dj[m] * sU[v][yb + 4 * m];
 #if OD_FAST
         // one Jacobian factor per direction
-        CT gx = (dxi + J0[v * 16 + fpx] * gLi + J1[v * 16 + fpx] * gRi) * a.jx;
-        CT gy = (deta + J2[v * 16 + fpy] * gLj + J3[v * 16 + fpy] * gRj) * a.jy;
-        CT gz = (dz + J4[v * 16 + fpz] * gLk + J5[v * 16 + fpz] * gRk) * a.jz;
+        CT gx = fma_t(J1[v * 16 + fpx], gRi, fma_t(J0[v * 16 + fpx], gLi, dxi)) * a.jx;
+        CT gy = fma_t(J3[v * 16 + fpy], gRj, fma_t(J2[v * 16 + fpy], gLj, deta)) * a.jy;
+        CT gz = fma_t(J5[v * 16 + fpz], gRk, fma_t(J4[v * 16 + fpz], gLk, dz)) * a.jz;
 #else
         CT gx = dxi * a.jx, gy = deta * a.jy, gz = dz * a.jz;
         gx += J0[v * 16 + fpx] * gLi * a.jx;
@@ -919,12 +978,17 @@ __device__ __forceinline__ FvQuad<CT> fv_value(const StageArgs<UT, CT>& a, const
     const Coef4<CT> c = side_coef<CT>(side);
     CT st[5], gt[15], fvv[5];
 #pragma unroll
-    for (int v = 0; v < 5; ++v) st[v] = trace4(sUe[v], base, stride, c.c0, c.c1, c.c2, c.c3, fv_order(D));
+    for (int v = 0; v < 5; ++v)
+        st[v] = trace4(sUe[v], base, stride, c.c0, c.c1, c.c2, c.c3, kOneX ? br1_order(D) : fv_order(D));
 #pragma unroll
     for (int q = 0; q < 15; ++q) gt[q] = trace4_swz(sGe[q], base, stride, c.c0, c.c1, c.c2, c.c3, fv_order(D));
+#if OD_FAST
+    fast_visc_flux(D, fast_visc(a, st, gt, e), fvv + 1);
+#else
     CT mu = a.sutherland ? sutherland(st, a.mu_ref, a.t_ref, a.s_suth) : a.mu;
     if (a.mu_t) mu = mu + a.mu_t[e];
     viscous_flux(D, st, gt, mu, fvv);
+#endif
     return FvQuad<CT>{{fvv[1], fvv[2], fvv[3], fvv[4]}};
 }
 
@@ -1128,53 +1192,48 @@ __device__ __forceinline__ void load_state_tile(const UT* u, int64_t NP, int64_t
     }
 }
 
+#if OD_FAST
 // Divergence of the volume viscous fluxes at the lane's point (the F_v half
-// of accumulate_volume_rhs_shfl / _z, rhs.cu:229-266) from the corrected
-// gradient g, x then y then z, components 1..4 (F_v of the mass equation is
-// zero) -> the element's fv block after its face part.  S: this wave's
-// 256-float LDS staging area.  Used by the fast f32 build (kSplitVisc).
-template <class UT, class CT>
-__device__ __forceinline__ void visc_divergence(const StageArgs<UT, CT>& a, int64_t e, const CT (*sUe)[64],
-                                                const CT* g, CT* S, int i, int j, int k, int pt) {
-    CT st[5];
-#pragma unroll
-    for (int v = 0; v < 5; ++v) st[v] = sUe[v][pt];
-    CT mu = a.sutherland ? sutherland(st, a.mu_ref, a.t_ref, a.s_suth) : a.mu;
-    if (a.mu_t) mu = mu + a.mu_t[e];
-    const ViscPoint<CT> vp = viscous_point(st, g, mu, 7);
-    CT acc[4] = {(CT)0, (CT)0, (CT)0, (CT)0};
+// of accumulate_volume_rhs_shfl / _z, rhs.cu:229-266) from its state st and
+// corrected gradient g, x then y then z, components 1..4 (F_v of the mass
+// equation is zero) -> the element's fv block after its face part.  S: this
+// wave's 256-float LDS staging area.
+template <class UT>
+__device__ __forceinline__ void visc_divergence(const StageArgs<UT, float>& a, int64_t e, const float* st,
+                                                const float* g, float* S, int i, int j, int k, int pt) {
+    const FastVisc f = fast_visc(a, st, g, e);
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-        CT fvv[5];
-        viscous_flux_dir(d, vp, fvv);
-        if constexpr (kDppX<CT>) {
-            if (d == 0) {
-                const CT* Dx = coef_lds<CT>().D[i];
+        float fvv[4];
+        fast_visc_flux(d, f, fvv);
+        if (d == 0) {
+            const float* Dx = coef_lds<float>().D[i];
 #pragma unroll
-                for (int q = 0; q < 4; ++q) acc[q] += quad_line(Dx, fvv[1 + q]) * a.jx;
-                continue;
-            }
+            for (int q = 0; q < 4; ++q) acc[q] += quad_line(Dx, fvv[q]) * a.jx;
+            continue;
         }
-        if (d > (kDppX<CT> ? 1 : 0)) wave_sync();  // the previous direction's reads are done
+        if (d > 1) wave_sync();  // the previous direction's reads are done
 #pragma unroll
-        for (int q = 0; q < 4; ++q) S[q * 64 + pt] = fvv[1 + q];
+        for (int q = 0; q < 4; ++q) S[q * 64 + pt] = fvv[q];
         wave_sync();
-        const int idx = d == 0 ? i : (d == 1 ? j : k);
-        const int base = d == 0 ? 4 * j + 16 * k : (d == 1 ? i + 16 * k : i + 4 * j);
-        const int stride = d == 0 ? 1 : (d == 1 ? 4 : 16);
-        const CT jac = d == 0 ? a.jx : (d == 1 ? a.jy : a.jz);
-        const CT* Dd = coef_lds<CT>().D[idx];
+        const int idx = d == 1 ? j : k;
+        const int base = d == 1 ? i + 16 * k : i + 4 * j;
+        const int stride = d == 1 ? 4 : 16;
+        const float jac = d == 1 ? a.jy : a.jz;
+        const float* Dd = coef_lds<float>().D[idx];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            CT dd = 0;
+            float dd = 0;
 #pragma unroll
             for (int m = 0; m < 4; ++m) dd += Dd[m] * S[q * 64 + base + m * stride];
             acc[q] += dd * jac;
         }
     }
-    FvQuad<CT>* dst = reinterpret_cast<FvQuad<CT>*>(a.fv + e * kFvStride + kFvFaces + pt * 4);
-    *dst = FvQuad<CT>{{acc[0], acc[1], acc[2], acc[3]}};
+    FvQuad<float>* dst = reinterpret_cast<FvQuad<float>*>(a.fv + e * kFvStride + kFvFaces + pt * 4);
+    *dst = FvQuad<float>{{acc[0], acc[1], acc[2], acc[3]}};
 }
+#endif
 
 // Volume RHS at the lane's point -> rs (rhs.cu:229-266, 490-510): minus the
 // divergence of F_e (VISC: of F_e - F_v, from the corrected gradient g), x then
@@ -1319,19 +1378,20 @@ __device__ __forceinline__ void visc_body(const StageArgs<UT, CT>& a, const Tile
     if (tile_valid(tl, wave)) lane_gradient(a, L.sU[wave], L.sJmp[wave], i, j, k, g);
     if (tile_valid(tl, wave)) {
         const int64_t e = tile_eidx(tl, wave);
-        if constexpr (kSplitVisc<CT>) {
-            visc_divergence(a, e, L.sU[wave], g, L.vol_stage(wave), i, j, k, pt);
-        } else {
-            CT st[5], r[5];
+        CT st[5];
 #pragma unroll
-            for (int v = 0; v < 5; ++v) st[v] = L.sU[wave][v][pt];
-            CT mu = a.sutherland ? sutherland(st, a.mu_ref, a.t_ref, a.s_suth) : a.mu;
-            if (a.mu_t) mu = mu + a.mu_t[e];
-            wave_sync();  // without a prefetch the staging area is the jumps just read
-            volume_rhs<true>(a, L.sU[wave], g, mu, (const CT*)nullptr, (CT(*)[64])L.vol_stage(wave), i, j, k, pt, r);
+        for (int v = 0; v < 5; ++v) st[v] = L.sU[wave][v][pt];
+        wave_sync();  // without a prefetch the staging area is the jumps just read
+#if OD_FAST
+        visc_divergence(a, e, st, g, L.vol_stage(wave), i, j, k, pt);
+#else
+        CT r[5];
+        CT mu = a.sutherland ? sutherland(st, a.mu_ref, a.t_ref, a.s_suth) : a.mu;
+        if (a.mu_t) mu = mu + a.mu_t[e];
+        volume_rhs<true>(a, L.sU[wave], g, mu, (const CT*)nullptr, (CT(*)[64])L.vol_stage(wave), i, j, k, pt, r);
 #pragma unroll
-            for (int v = 0; v < 5; ++v) a.fv[e * kFvStride + kFvFaces + v * 64 + pt] = r[v];
-        }
+        for (int v = 0; v < 5; ++v) a.fv[e * kFvStride + kFvFaces + v * 64 + pt] = r[v];
+#endif
     }
     if constexpr (PF) __syncthreads();  // sG overwrites the jumps the other wave may still read
     if (tile_valid(tl, wave)) {
@@ -1888,145 +1948,220 @@ __device__ __forceinline__ void update_block_body(const StageArgs<float, float>&
 }
 
 // ---------------------------------------------------------------------------
-// The visc kernel on the same 2x2x2 blocks: the BR1 jumps of the internal
-// faces come from the block's LDS state tiles (one task per internal face
-// point forms both sides' jumps), those of the external faces from the
-// prefetched neighbour traces; gradient, volume viscous divergence and the
-// face viscous fluxes are visc_body's, element by element.  LDS: the jumps
-// [le][ext d0..d2, int d0..d2][5][16] (the external part first holds the
-// prefetched traces) share one buffer with the gradient tile [le][15][64]
-// (written after a barrier), and the state tiles.
+// The visc kernel on the same 2x2x2 blocks, by lines.  A lane of a line wave
+// owns one line of four points along direction D of one element (8 elements x
+// 16 lines x 3 directions = 6 full waves; lane = [pair of elements][line][side]
+// with side = the element's coordinate along D): it reads the line's states
+// once, forms both end traces, both BR1 jumps and the corrected derivative at
+// its four points, and later, from the gradients of the line, the viscous
+// fluxes at both ends.  The neighbour across the block's internal face is the
+// neighbouring lane (DPP); the external trace comes straight from memory.  The
+// operators are wave-uniform here (scalar registers).  Point-wise work (volume
+// fluxes and their divergence) stays a wave per element.
+//
+// The point-wise form of all this (a lane per solution point for the gradient,
+// a lane per face point for jumps and fluxes) read each state 12 times and each
+// gradient 6 to 8 times from LDS and formed the state's face traces twice: its
+// VALU instructions (753 per element's wave) took 78 % of the kernel's time and
+// its LDS reads about as much, at 6 waves to a SIMD.  By lines it is 8 waves
+// (63 VGPRs, 31 KB per work-group) and at 48^3 132 us a launch instead of 195
+// (0.51 GB moved, 82 us at the update kernel's 6.2 TB/s).
+// Every value is the same expression as in visc_body.
+//
+// LDS: one area per element, first its state [5][64], then, once every line has
+// been read, its gradient [15][64], both in swz64 order, under which the 16
+// lines of an element fall in distinct banks; areas lie 4 floats further apart
+// than their size, so that the partner along x, y, z is 4, 8, 16 banks away,
+// the bit that swz64 keeps fixed over a face of that direction.
 // ---------------------------------------------------------------------------
+constexpr int kAreaStride = 15 * 64 + 4;
 struct BlockViscLds {
-    alignas(16) float buf[kBlk * 15 * 64];
-    BlockTiles sU;
-    // 480 jumps per element, 496 apart (the tiles' bank offset again)
-    __device__ float* jumps(int le) { return buf + le * 496; }
-    __device__ float (*sG())[15][64] { return reinterpret_cast<float(*)[15][64]>(buf); }
+    alignas(16) float area[kBlk * kAreaStride];
+    __device__ float* of(int le) { return area + le * kAreaStride; }
 };
 
-// BR1 jump at the external face of direction D of elements 4h .. 4h+3 (as br1_jumps).
+// swz64 position of the line point m of direction D relative (XOR) to m = 0.
 template <int D>
-__device__ __forceinline__ void blk_br1_ext(const StageArgs<float, float>& a, const Block& b, BlockViscLds& L, int h,
-                                            int lane) {
-    const int le = 4 * h + (lane >> 4), fp = lane & 15;
-    const int side = blk_bit(le, D);
+__device__ constexpr int line_xor(int m) {
+    const int lo = m & 1, hi = m >> 1;
+    return D == 0 ? ((lo ? 1 | 2 | 32 : 0) | hi << 2) : (D == 1 ? (lo | hi << 3) : (hi << 1 | lo << 4));
+}
+// The value of the lane's partner, lane ^ 1.
+__device__ __forceinline__ float lane_partner(float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xF, 0xF, false));  // quad_perm [1,0,3,2]
+}
+// End trace sum_m q[m] l_m(+-1) in the BR1 order (the right end's coefficients
+// are the left one's backwards).
+__device__ __forceinline__ float line_trace(const float* q, const float* c) {
+    return __builtin_fmaf(q[1], c[1], q[0] * c[0]) + __builtin_fmaf(q[3], c[3], q[2] * c[2]);
+}
+
+// One line wave's state through the kernel's phases.
+struct LineWave {
+    int le, side, fp;       // element, its coordinate along D, face point of the line
+    float u[5][4];          // the line's states
+    float tl[5], tr[5];     // their traces at the left and right end
+    float ext[5];           // the neighbour's trace across the external face
+    int pos[4];             // positions of the four points in the element's area
+};
+
+template <int D>
+__device__ __forceinline__ void line_begin(const StageArgs<float, float>& a, const Block& b, int half, int lane,
+                                           LineWave& w) {
+    w.side = lane & 1;
+    w.fp = (lane >> 1) & 15;
+    const int p = 2 * half + (lane >> 5);  // pair of elements along D
+    w.le = (D == 0 ? 2 * p : (D == 1 ? ((p & 1) | ((p >> 1) << 2)) : p)) + (w.side << D);
+    const int nb = blk_ext_nb(a, b, w.le, D);
+    const int src = nb >= 0 ? nb : blk_elem(a, b, w.le);  // at a slip wall its own, unused
+    const float* t = a.tr_in + (int64_t)src * kTraceStride + (2 * D + 1 - w.side) * 80 + w.fp;
+#pragma unroll
+    for (int v = 0; v < 5; ++v) w.ext[v] = t[v * 16];
     int base, stride;
-    face_line(D, fp, base, stride);
-    const Coef4<float> c = side_coef<float>(side);
-    const bool wall = D == 1 && blk_ext_nb(a, b, le, D) < 0;
-    float* J = L.jumps(le) + D * 80;
+    face_line(D, w.fp, base, stride);
+    const int s0 = swz64(base);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) w.pos[m] = w.le * kAreaStride + (s0 ^ line_xor<D>(m));
+}
+
+// Jumps and corrected derivative along D (br1_jumps, lane_gradient_faces) ->
+// the gradient's rows 3 v + D.
+template <int D>
+__device__ __forceinline__ void line_gradient(const StageArgs<float, float>& a, const Block& b, BlockViscLds& L,
+                                              LineWave& w) {
+    const Ops<float>& o = dev_ops<float>();
+    const bool wall = D == 1 && blk_ext_nb(a, b, w.le, D) < 0;
+    const float jac = D == 0 ? a.jx : (D == 1 ? a.jy : a.jz);
 #pragma unroll
     for (int v = 0; v < 5; ++v) {
-        float own = trace4(L.sU[le][v], base, stride, c.c0, c.c1, c.c2, c.c3, br1_order(D));
-        const float sign = (v > 0 && v < 4) ? -1.0f : 1.0f;
-        const float far = J[v * 16 + fp];
-        float nbv = !wall ? far : own * sign;
-        J[v * 16 + fp] = 0.5f * (nbv + own) - own;
+        const float* u = w.u[v];
+        const float tl = line_trace(u, o.eL), tr = line_trace(u, o.eR);
+        const float in = lane_partner(w.side ? tl : tr);
+        const float own = w.side ? tr : tl;
+        const float ext = wall ? ((v > 0 && v < 4) ? -own : own) : w.ext[v];
+        const float nl = w.side ? in : ext, nr = w.side ? ext : in;
+        const float jl = __builtin_fmaf(0.5f, nl + tl, -tl), jr = __builtin_fmaf(0.5f, nr + tr, -tr);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float d = 0.f;
+#pragma unroll
+            for (int m = 0; m < 4; ++m) d = __builtin_fmaf(o.D[4 * i + m], u[m], d);
+            L.area[w.pos[i] + (3 * v + D) * 64] =
+                __builtin_fmaf(jr, o.gR[i], __builtin_fmaf(jl, o.gL[i], d)) * jac;
+        }
+        w.tl[v] = tl;
+        w.tr[v] = tr;
+        asm volatile("" : "+v"(w.tl[v]), "+v"(w.tr[v])::"memory");  // variable by variable (see lane_gradient_faces)
     }
 }
 
-// BR1 jumps of both sides of the internal faces of direction D (pairs as in
-// blk_int_pass); each side's jump as br1_jumps forms it with the other
-// side's trace as the neighbour value.
+// Viscous fluxes at both ends of the line (fv_value).  The external end's goes
+// to the element's slot of that face; of the pair's internal face the left
+// element stores the half-difference (F_vL - F_vR) / 2, all the update kernel
+// reads there.
 template <int D>
-__device__ __forceinline__ void blk_br1_int(BlockViscLds& L, int lane) {
-    const int p = lane >> 4, fp = lane & 15;
-    const int lL = D == 0 ? 2 * p : (D == 1 ? ((p & 1) | ((p >> 1) << 2)) : p);
-    const int lR = lL + (1 << D);
-    int base, stride;
-    face_line(D, fp, base, stride);
-    const Coef4<float> cr = side_coef<float>(true), cl = side_coef<float>(false);
-    float* JL = L.jumps(lL) + (3 + D) * 80;
-    float* JR = L.jumps(lR) + (3 + D) * 80;
+__device__ __forceinline__ void line_flux(const StageArgs<float, float>& a, const Block& b, const BlockViscLds& L,
+                                          const LineWave& w) {
+    const Ops<float>& o = dev_ops<float>();
+    float gl[15], gr[15];
 #pragma unroll
-    for (int v = 0; v < 5; ++v) {
-        const float tl = trace4(L.sU[lL][v], base, stride, cr.c0, cr.c1, cr.c2, cr.c3, br1_order(D));
-        const float tr = trace4(L.sU[lR][v], base, stride, cl.c0, cl.c1, cl.c2, cl.c3, br1_order(D));
-        JL[v * 16 + fp] = 0.5f * (tr + tl) - tl;
-        JR[v * 16 + fp] = 0.5f * (tl + tr) - tr;
+    for (int q = 0; q < 15; ++q) {
+        // what the flux along D reads: the density's gradient, the momenta's
+        // along D, across D of momentum D and on the diagonal, the energy's along D
+        const int v = q / 3, c = q % 3;
+        const bool used = v == 0 || c == D || (v < 4 && (v - 1 == D || v - 1 == c));
+        if (!used) {
+            gl[q] = gr[q] = 0.f;
+            continue;
+        }
+        float x[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) x[m] = L.area[w.pos[m] + q * 64];
+        gl[q] = __builtin_fmaf(x[3], o.eL[3], __builtin_fmaf(x[2], o.eL[2], __builtin_fmaf(x[1], o.eL[1], x[0] * o.eL[0])));
+        gr[q] = __builtin_fmaf(x[3], o.eR[3], __builtin_fmaf(x[2], o.eR[2], __builtin_fmaf(x[1], o.eR[1], x[0] * o.eR[0])));
+        asm volatile("" : "+v"(gl[q]), "+v"(gr[q])::"memory");
     }
+    const int64_t e = blk_elem(a, b, w.le);
+    float fl[4], fr[4];
+    fast_visc_flux(D, fast_visc(a, w.tl, gl, e), fl);
+    asm volatile("" : "+v"(fl[0]), "+v"(fl[1]), "+v"(fl[2]), "+v"(fl[3])::"memory");  // one end, then the other
+    fast_visc_flux(D, fast_visc(a, w.tr, gr, e), fr);
+    FvQuad<float> ext, h;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        ext.c[c] = w.side ? fr[c] : fl[c];
+        const float other = lane_partner(w.side ? fl[c] : fr[c]);
+        h.c[c] = 0.5f * (fr[c] - other);  // left element
+    }
+    FvQuad<float>* dst = reinterpret_cast<FvQuad<float>*>(a.fv + e * kFvStride + 2 * D * 64 + w.fp * 4);
+    dst[w.side ? 16 : 0] = ext;
+    if (!w.side) dst[16] = h;
 }
 
-// Viscous normal fluxes at the faces of direction D of the q-th element pair
-// along D (left lL, right lL + 2^D): lane = (element of the pair, side,
-// face point).  External faces store their flux as the tile kernels do; at
-// the pair's interior face the left element's lane (16..31) takes the right
-// element's flux from lane + 16 (32..47) and stores the half-difference
-// (F_vL - F_vR) / 2 in the left element's slot, which is all the update
-// kernel reads there.
-template <int D>
-__device__ __forceinline__ void blk_fv_pass(const StageArgs<float, float>& a, const Block& b, BlockViscLds& L, int q,
-                                            int pt) {
-    const int lL = D == 0 ? 2 * q : (D == 1 ? ((q & 1) | ((q >> 1) << 2)) : q);
-    const int second = pt >> 5, side = (pt >> 4) & 1, fp = pt & 15;
-    const int le = second ? lL + (1 << D) : lL;
-    const int64_t e = blk_elem(a, b, le);
-    const FvQuad<float> f = fv_value<D>(a, L.sU[le], L.sG()[le], e, side, fp);
-    FvQuad<float> g;
-    const int from = (pt ^ 48) << 2;  // lane 16 + fp <-> 32 + fp (byte address of the source lane)
-#pragma unroll
-    for (int c = 0; c < 4; ++c) g.c[c] = __int_as_float(__builtin_amdgcn_ds_bpermute(from, __float_as_int(f.c[c])));
-    FvQuad<float>* dst = reinterpret_cast<FvQuad<float>*>(a.fv + e * kFvStride + (2 * D + side) * 64 + fp * 4);
-    if (second == side) {
-        *dst = f;  // external face
-    } else if (!second) {
-        FvQuad<float> h;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) h.c[c] = 0.5f * (f.c[c] - g.c[c]);
-        *dst = h;
-    }
-}
-
-__device__ __forceinline__ void visc_block_body(const StageArgs<float, float>& a, const Block& b, BlockViscLds& L) {
+// role: 0..5 the line waves (direction role % 3, half of the pairs role / 3),
+// 6 and 7 none.
+__device__ __forceinline__ void visc_block_body(const StageArgs<float, float>& a, const Block& b, BlockViscLds& L,
+                                                int role) {
     const int wave = wave_index(), pt = threadIdx.x & 63;
     const int i = pt & 3, j = (pt >> 2) & 3, k = pt >> 4;
     const int64_t NP = (int64_t)a.nx * a.ny * a.nz * 64;
     const int64_t e = blk_elem(a, b, wave);
+    const int half = role / 3, D = role < 6 ? role - 3 * half : 3;
     const float cf = coef_load<float>((int)threadIdx.x);
-    if (pt < 60) {  // the element's three external neighbour traces: 60 16-byte LDS-DMA chunks
-        const float* src = blk_ext_trace_src(a, b, wave, pt);
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                         (__attribute__((address_space(3))) void*)L.jumps(wave), 16, 0, 0);
-    }
-    load_state_tile(a.uin, NP, e, L.sU[wave], pt);
-    coef_store<float>((int)threadIdx.x, cf);
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    switch (wave) {
-        case 0: blk_br1_ext<0>(a, b, L, 0, pt); blk_br1_int<2>(L, pt); break;
-        case 1: blk_br1_ext<0>(a, b, L, 1, pt); break;
-        case 2: blk_br1_ext<1>(a, b, L, 0, pt); break;
-        case 3: blk_br1_ext<1>(a, b, L, 1, pt); break;
-        case 4: blk_br1_ext<2>(a, b, L, 0, pt); break;
-        case 5: blk_br1_ext<2>(a, b, L, 1, pt); break;
-        case 6: blk_br1_int<0>(L, pt); break;
-        default: blk_br1_int<1>(L, pt); break;
-    }
-    __syncthreads();
-    // the wave's element: face f = 2d + s has its jumps in the external slot
-    // d when s is the element's coordinate bit d, else in the internal slot
-    const float* Jw = L.jumps(wave);
-    const int lx = wave & 1, ly = (wave >> 1) & 1, lz = wave >> 2;
-    float g[15];
-    lane_gradient_faces(a, L.sU[wave], Jw + (lx == 0 ? 0 : 240), Jw + (lx == 1 ? 0 : 240), Jw + (ly == 0 ? 80 : 320),
-                        Jw + (ly == 1 ? 80 : 320), Jw + (lz == 0 ? 160 : 400), Jw + (lz == 1 ? 160 : 400), i, j, k, g);
-    // staging of the volume viscous-flux lines in the element's own jumps,
-    // which only this wave has read
-    visc_divergence(a, e, L.sU[wave], g, L.jumps(wave), i, j, k, pt);
-    __syncthreads();  // the gradient tile overwrites jumps other waves may still read
+    float s0[5];
 #pragma unroll
-    for (int q = 0; q < 15; ++q) L.sG()[wave][q][swz64(pt)] = g[q];
-    __syncthreads();
-    // face viscous fluxes: pass (D, q) = the q-th pair of elements along D,
-    // both faces of direction D (waves 0..3: x then z, waves 4..7: y)
-    if (wave < 4) {
-        blk_fv_pass<0>(a, b, L, wave, pt);
-        blk_fv_pass<2>(a, b, L, wave, pt);
-    } else {
-        blk_fv_pass<1>(a, b, L, wave - 4, pt);
+    for (int v = 0; v < 5; ++v) s0[v] = a.uin[v * NP + e * 64 + pt];
+    LineWave w;
+    if (D == 0)
+        line_begin<0>(a, b, half, pt, w);
+    else if (D == 1)
+        line_begin<1>(a, b, half, pt, w);
+    else if (D == 2)
+        line_begin<2>(a, b, half, pt, w);
+    {
+        float* A = L.of(wave) + swz64(pt);
+#pragma unroll
+        for (int v = 0; v < 5; ++v) A[v * 64] = s0[v];
     }
+    coef_store<float>((int)threadIdx.x, cf);
+    __syncthreads();
+    if (D < 3) {
+#pragma unroll
+        for (int v = 0; v < 5; ++v)
+#pragma unroll
+            for (int m = 0; m < 4; ++m) w.u[v][m] = L.area[w.pos[m] + v * 64];
+    }
+    __syncthreads();  // the gradients overwrite the states
+    if (D == 0)
+        line_gradient<0>(a, b, L, w);
+    else if (D == 1)
+        line_gradient<1>(a, b, L, w);
+    else if (D == 2)
+        line_gradient<2>(a, b, L, w);
+    __syncthreads();
+    if (D == 0)
+        line_flux<0>(a, b, L, w);
+    else if (D == 1)
+        line_flux<1>(a, b, L, w);
+    else if (D == 2)
+        line_flux<2>(a, b, L, w);
+    float g[15];
+    {
+        const float* A = L.of(wave) + swz64(pt);
+#pragma unroll
+        for (int q = 0; q < 15; ++q) g[q] = A[q * 64];
+    }
+    float st[5];  // the point's state again (from L2), not held through the line phases
+#pragma unroll
+    for (int v = 0; v < 5; ++v) st[v] = a.uin[v * NP + e * 64 + pt];
+    __syncthreads();  // the volume fluxes' lines are staged over the gradients
+    visc_divergence(a, e, st, g, L.of(wave), i, j, k, pt);
 }
+
+// The line waves are waves 0..5 or 2..7 of a work-group in turn, so that the
+// SIMDs of a CU get equally many of them.  Work-groups go round the XCDs, so
+// it is every eighth that turns.
+__device__ __forceinline__ int line_role(int group) { return (wave_index() + ((group >> 3) & 1) * 6) & 7; }
 
 // One box: the update kernel walks the blocks backwards, the visc kernel
 // forwards (make_block).
@@ -2036,9 +2171,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8))) void o
     __shared__ BlockUpdateLds L;
     update_block_body<VISC>(a, make_block<true>(a), L);
 }
-__global__ __launch_bounds__(512) void od_visc_block_kernel(StageArgs<float, float> a) {
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8))) void od_visc_block_kernel(StageArgs<float, float> a) {
     __shared__ BlockViscLds L;
-    visc_block_body(a, make_block<false>(a), L);
+    const int group = (int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
+    visc_block_body(a, make_block<false>(a), L, line_role(group));
 }
 #endif
 
@@ -2231,30 +2367,33 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8))) void o
     update_block_body<VISC>(ab, b, L);
 }
 
-__global__ __launch_bounds__(512) void od_batch_visc_block_kernel(StageArgs<float, float> a, BlockBatch bb) {
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8))) void od_batch_visc_block_kernel(StageArgs<float, float> a, BlockBatch bb) {
     StageArgs<float, float> ab;
     Block b;
     batch_block<false>(a, bb, ab, b);
     __shared__ BlockViscLds L;
-    visc_block_body(ab, b, L);
+    visc_block_body(ab, b, L, line_role((int)blockIdx.x));
 }
 
 // One box with an odd dimension: its core on blocks and its shell on tiles in
-// one launch.  A 512-thread work-group takes a block of the core, or four tiles
-// of the shell (which need as much LDS: 10.4 KB each in the visc kernel, 9.1 KB
-// in the update kernel).  The blocks come first (the update kernel's backwards,
+// one launch.  A 512-thread work-group takes a block of the core, or as many
+// tiles of the shell as fit its threads and a block's LDS: three in the visc
+// kernel (10.3 KB each), four in the update kernel (9.1 KB).  The blocks come first (the update kernel's backwards,
 // as in the even boxes) and the shell, a small part of the box, fills up the
 // last work-groups' wave; a launch of its own would cost its latency twice a
 // stage.  33x25x37 (AUSM+, 100 steps): 37.4 ms with every element on tiles,
-// 33.6 here.
+// 33.6 so (30.0 with the visc kernel's blocks by lines).
 struct CoreShell {
     int32_t n_blocks, n_tiles;  // blocks of the core, tiles of the shell
 };
-// Tile of this 128-thread part of shell work-group `group`; past the shell's
-// end an empty one.
+constexpr int kShellTiles[2] = {3, 4};  // tiles of a shell work-group: visc, update kernel
+// Tile of this 128-thread part of shell work-group `group`; none left for it:
+// an empty one, which touches no LDS of its own.
+template <int TILES>
 __device__ __forceinline__ Tile core_shell_tile(const StageArgs<float, float>& a, const CoreShell& cs, int group) {
-    const int lt = uni(4 * group + (int)(threadIdx.x >> 7));
-    const bool ok = lt < cs.n_tiles;
+    const int part = uni((int)(threadIdx.x >> 7));
+    const int lt = TILES * group + part;
+    const bool ok = part < TILES && lt < cs.n_tiles;
     Tile tl = shell_tile(a, ok ? lt : 0);
     tl.v0 = ok;
     tl.v1 = ok && tl.v1;
@@ -2266,26 +2405,27 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8))) void o
     StageArgs<float, float> a, CoreShell cs) {
     __shared__ union {
         BlockUpdateLds block;
-        UpdateLds<float, VISC> tile[4];
+        UpdateLds<float, VISC> tile[kShellTiles[1]];
     } L;
     const int w = (int)blockIdx.x;
     if (w < cs.n_blocks)
         update_block_body<VISC>(a, core_block(a, cs.n_blocks - 1 - w), L.block);
     else
-        update_body<float, float, VISC>(a, core_shell_tile(a, cs, w - cs.n_blocks), L.tile[threadIdx.x >> 7],
+        update_body<float, float, VISC>(a, core_shell_tile<kShellTiles[1]>(a, cs, w - cs.n_blocks),
+                                        L.tile[threadIdx.x >> 7],
                                         wave_index() & 1, threadIdx.x & 63);
 }
-__global__ __launch_bounds__(512) void od_visc_core_shell_kernel(StageArgs<float, float> a, CoreShell cs) {
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8))) void od_visc_core_shell_kernel(StageArgs<float, float> a, CoreShell cs) {
     __shared__ union {
         BlockViscLds block;
-        ViscLds<float> tile[4];
+        ViscLds<float> tile[kShellTiles[0]];
     } L;
     const int w = (int)blockIdx.x;
     if (w < cs.n_blocks)
-        visc_block_body(a, core_block(a, w), L.block);
+        visc_block_body(a, core_block(a, w), L.block, line_role(w));
     else
-        visc_body(a, core_shell_tile(a, cs, w - cs.n_blocks), L.tile[threadIdx.x >> 7], wave_index() & 1,
-                  threadIdx.x & 63);
+        visc_body(a, core_shell_tile<kShellTiles[0]>(a, cs, w - cs.n_blocks),
+                  L.tile[min((int)(threadIdx.x >> 7), kShellTiles[0] - 1)], wave_index() & 1, threadIdx.x & 63);
 }
 #endif
 
@@ -2482,14 +2622,16 @@ CoreShell core_shell(const StageArgs<float, float>& a) {
     cs.n_tiles = (int32_t)shell_tiles(a.nx, a.ny, a.nz);
     return cs;
 }
-dim3 core_shell_grid(const CoreShell& cs) { return dim3((unsigned)(cs.n_blocks + (cs.n_tiles + 3) / 4)); }
+dim3 core_shell_grid(const CoreShell& cs, int kind) {
+    return dim3((unsigned)(cs.n_blocks + (cs.n_tiles + kShellTiles[kind] - 1) / kShellTiles[kind]));
+}
 }  // namespace
 
 template <bool VISC>
 int launch_update_core_shell(const StageArgs<float, float>& a, void* stream) {
     if (a.nx < 2 || a.ny < 2 || a.nz < 2) return 1;
     const CoreShell cs = core_shell(a);
-    hipLaunchKernelGGL((od_update_core_shell_kernel<VISC>), core_shell_grid(cs), dim3(64 * kBlk), 0,
+    hipLaunchKernelGGL((od_update_core_shell_kernel<VISC>), core_shell_grid(cs, 1), dim3(64 * kBlk), 0,
                        (hipStream_t)stream, a, cs);
     return check_launch();
 }
@@ -2499,7 +2641,7 @@ template int launch_update_core_shell<false>(const StageArgs<float, float>&, voi
 int launch_visc_core_shell(const StageArgs<float, float>& a, void* stream) {
     if (a.nx < 2 || a.ny < 2 || a.nz < 2) return 1;
     const CoreShell cs = core_shell(a);
-    hipLaunchKernelGGL(od_visc_core_shell_kernel, core_shell_grid(cs), dim3(64 * kBlk), 0, (hipStream_t)stream, a, cs);
+    hipLaunchKernelGGL(od_visc_core_shell_kernel, core_shell_grid(cs, 0), dim3(64 * kBlk), 0, (hipStream_t)stream, a, cs);
     return check_launch();
 }
 template <bool VISC>
