@@ -1235,17 +1235,14 @@ __device__ __forceinline__ void visc_divergence(const StageArgs<UT, float>& a, i
 }
 #endif
 
-// Volume RHS at the lane's point -> rs (rhs.cu:229-266, 490-510): minus the
+// Volume RHS at the lane's point, state st (rhs.cu:229-266, 490-510): minus the
 // divergence of F_e (VISC: of F_e - F_v, from the corrected gradient g), x then
 // y then z, plus the body force, with the RHS_REAL round trip (rhs.cu:509,
 // rk.cu:52).  S: this wave's [5][64] LDS staging area.  Strict build, and the
 // fast build's Euler fluxes (vdiv: the divergence of the viscous ones).
 template <bool VISC, class UT, class CT>
-__device__ __forceinline__ void volume_rhs(const StageArgs<UT, CT>& a, const CT (*sUe)[64], const CT* g, CT mu,
+__device__ __forceinline__ void volume_rhs(const StageArgs<UT, CT>& a, const CT* st, const CT* g, CT mu,
                                            const CT* vdiv, CT (*S)[64], int i, int j, int k, int pt, CT* out) {
-    CT st[5];
-#pragma unroll
-    for (int v = 0; v < 5; ++v) st[v] = sUe[v][pt];
     CT rs[5] = {(CT)0, (CT)0, (CT)0, (CT)0, (CT)0};
     ViscPoint<CT> vp;
     if constexpr (VISC) vp = viscous_point(st, g, mu, 7);
@@ -1388,7 +1385,7 @@ __device__ __forceinline__ void visc_body(const StageArgs<UT, CT>& a, const Tile
         CT r[5];
         CT mu = a.sutherland ? sutherland(st, a.mu_ref, a.t_ref, a.s_suth) : a.mu;
         if (a.mu_t) mu = mu + a.mu_t[e];
-        volume_rhs<true>(a, L.sU[wave], g, mu, (const CT*)nullptr, (CT(*)[64])L.vol_stage(wave), i, j, k, pt, r);
+        volume_rhs<true>(a, st, g, mu, (const CT*)nullptr, (CT(*)[64])L.vol_stage(wave), i, j, k, pt, r);
 #pragma unroll
         for (int v = 0; v < 5; ++v) a.fv[e * kFvStride + kFvFaces + v * 64 + pt] = r[v];
 #endif
@@ -1455,8 +1452,11 @@ __device__ __forceinline__ void update_body(const StageArgs<UT, CT>& a, const Ti
                 for (int q = 0; q < 4; ++q) vdiv[q] = src.c[q];
             }
         }
-        volume_rhs<false>(a, L.sU[wave], (const CT*)nullptr, (CT)0, VISC ? vdiv : (const CT*)nullptr, L.sF[wave], i, j,
-                          k, pt, r);
+        CT st[5];
+#pragma unroll
+        for (int v = 0; v < 5; ++v) st[v] = L.sU[wave][v][pt];
+        volume_rhs<false>(a, st, (const CT*)nullptr, (CT)0, VISC ? vdiv : (const CT*)nullptr, L.sF[wave], i, j, k, pt,
+                          r);
         wave_sync();
 #pragma unroll
         for (int v = 0; v < 5; ++v) L.sF[wave][v][pt] = r[v];
@@ -1571,11 +1571,13 @@ __global__ __launch_bounds__(128) void od_trace_kernel(StageArgs<UT, CT> a) {
     trace_body(a, make_tile(a), sU, wave_index(), threadIdx.x & 63);
 }
 
+#if OD_FAST
 template <class UT, class CT>
 __global__ __launch_bounds__(128) void od_visc_kernel(StageArgs<UT, CT> a) {
     __shared__ ViscLds<CT> L;
     visc_body(a, make_tile(a), L, wave_index(), threadIdx.x & 63);
 }
+#endif
 
 // Occupancy target of the update kernels.  The strict f32 build needs ~78
 // VGPRs (6 waves per SIMD).  The fast all-f32 single-box kernel and the batch
@@ -1595,6 +1597,231 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(kMinWavesUp
     __shared__ UpdateLds<CT, VISC> L;
     update_body<UT, CT, VISC>(a, make_tile_reversed(a), L, wave_index(), threadIdx.x & 63);
 }
+
+// LDS area of one element in the kernels that work by lines: [5][64] or
+// [15][64] in swz64 order; areas lie 4 values further apart than their size.
+constexpr int kAreaStride = 15 * 64 + 4;
+// swz64 position of the line point m of direction D relative (XOR) to m = 0.
+template <int D>
+__device__ constexpr int line_xor(int m) {
+    const int lo = m & 1, hi = m >> 1;
+    return D == 0 ? ((lo ? 1 | 2 | 32 : 0) | hi << 2) : (D == 1 ? (lo | hi << 3) : (hi << 1 | lo << 4));
+}
+
+#if !OD_FAST
+// ---------------------------------------------------------------------------
+// Strict build, one box: the visc kernel by lines.  A 256-thread work-group has
+// four consecutive elements; in the line phases wave d < 3 takes direction d,
+// lane = (element, line of four points), and forms from one read of the line's
+// states both end traces, both BR1 jumps and the corrected derivative at its
+// four points, then from one read of the line's gradients the viscous fluxes at
+// both ends.  The neighbours' traces come straight from memory, the operators
+// are wave-uniform.  The volume RHS is point-wise, a wave per element.  Every
+// value is the expression of visc_body, in the reference's order.
+// Bounds: instruction issue.  Against the point-wise form (visc_body, which the
+// batches' tiles use), whose lanes read each state 12 and each gradient 6 to 8
+// times from LDS: 24x26x22 f64 102 -> 61 us, 48^3 f32 279 -> 231 us, 24x20x28
+// f64 state with f32 fluxes 40 -> 33 us a launch.
+// LDS: one area per element, the states, then the gradients over them.
+// ---------------------------------------------------------------------------
+constexpr int kQuad = 4;
+
+template <class CT>
+struct StrictLine {
+    int le, fp;
+    CT u[5][4];
+    CT tl[5], tr[5];  // end traces in the order of the viscous fluxes
+    CT nl[5], nr[5];  // the neighbours' facing traces
+    bool wl, wr;      // slip walls
+    int pos[4];
+};
+
+// Element e0's coordinates and the neighbours across both faces of direction D
+// of the lane's element e0 + le (those past the mesh's last one repeat it).
+template <int D, class UT, class CT>
+__device__ __forceinline__ void strict_line_begin(const StageArgs<UT, CT>& a, int e0, int E, int lane,
+                                                  StrictLine<CT>& w) {
+    w.le = lane >> 4;
+    w.fp = lane & 15;
+    int ez = e0 / (a.nx * a.ny), ey = (e0 - ez * a.nx * a.ny) / a.nx, ex = e0 - a.nx * (ey + a.ny * ez);
+    int l[kQuad], r[kQuad];
+#pragma unroll
+    for (int q = 0; q < kQuad; ++q) {
+        const Elem n = make_elem(ex, ey, ez, a.nx, a.ny, a.nz, a.wall);
+        l[q] = D == 0 ? n.xl : (D == 1 ? n.yl : n.zl);
+        r[q] = D == 0 ? n.xr : (D == 1 ? n.yr : n.zr);
+        if (e0 + q + 1 < E) {
+            ++ex;
+            if (ex == a.nx) {
+                ex = 0;
+                ++ey;
+                if (ey == a.ny) {
+                    ey = 0;
+                    ++ez;
+                }
+            }
+        }
+    }
+    const bool b0 = w.le & 1, b1 = w.le & 2;
+    const int nl = b1 ? (b0 ? l[3] : l[2]) : (b0 ? l[1] : l[0]);
+    const int nr = b1 ? (b0 ? r[3] : r[2]) : (b0 ? r[1] : r[0]);
+    w.wl = D == 1 && nl < 0;
+    w.wr = D == 1 && nr < 0;
+    const CT* tl = a.tr_in + (int64_t)(w.wl ? 0 : nl) * kTraceStride + (2 * D + 1) * 80 + w.fp;
+    const CT* tr = a.tr_in + (int64_t)(w.wr ? 0 : nr) * kTraceStride + (2 * D) * 80 + w.fp;
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+        w.nl[v] = tl[v * 16];
+        w.nr[v] = tr[v * 16];
+    }
+    int base, stride;
+    face_line(D, w.fp, base, stride);
+    const int s0 = swz64(base);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) w.pos[m] = w.le * kAreaStride + (s0 ^ line_xor<D>(m));
+}
+
+// Jumps (br1_jumps) and corrected derivative along D (lane_gradient_faces) ->
+// the gradient's rows 3 v + D.
+template <int D, class UT, class CT>
+__device__ __forceinline__ void strict_line_gradient(const StageArgs<UT, CT>& a, CT* area, StrictLine<CT>& w) {
+    const Ops<CT>& o = dev_ops<CT>();
+    const CT jac = D == 0 ? a.jx : (D == 1 ? a.jy : a.jz);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+        const CT* u = w.u[v];
+        const CT tl = trace4(u, 0, 1, o.eL[0], o.eL[1], o.eL[2], o.eL[3], br1_order(D));
+        const CT tr = trace4(u, 0, 1, o.eR[0], o.eR[1], o.eR[2], o.eR[3], br1_order(D));
+        const CT sign = (v > 0 && v < 4) ? ((CT)-1.0) : ((CT)1.0);
+        const CT nl = w.wl ? tl * sign : w.nl[v], nr = w.wr ? tr * sign : w.nr[v];
+        const CT jl = ((CT)0.5) * (nl + tl) - tl, jr = ((CT)0.5) * (nr + tr) - tr;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            CT d = 0;
+#pragma unroll
+            for (int m = 0; m < 4; ++m) d += o.D[4 * i + m] * u[m];
+            CT g = d * jac;
+            g += jl * o.gL[i] * jac;
+            g += jr * o.gR[i] * jac;
+            if (a.round_q) g = (CT)(float)g;  // Q_REAL round trip (rhs.cu:457-461)
+            area[w.pos[i] + (3 * v + D) * 64] = g;
+        }
+        w.tl[v] = D == 0 ? trace4(u, 0, 1, o.eL[0], o.eL[1], o.eL[2], o.eL[3], fv_order(D)) : tl;
+        w.tr[v] = D == 0 ? trace4(u, 0, 1, o.eR[0], o.eR[1], o.eR[2], o.eR[3], fv_order(D)) : tr;
+        asm volatile("" : "+v"(w.tl[v]), "+v"(w.tr[v])::"memory");  // variable by variable (see lane_gradient_faces)
+    }
+}
+
+// Viscous flux at one end of the line (fv_value) from its state trace and
+// gradient trace -> the element's slot of face 2 D + side.
+template <int D, class UT, class CT>
+__device__ __forceinline__ void strict_end_flux(const StageArgs<UT, CT>& a, int64_t e, bool valid, const CT* st,
+                                                const CT* gt, int side, int fp) {
+    CT f[5];
+    CT mu = a.sutherland ? sutherland(st, a.mu_ref, a.t_ref, a.s_suth) : a.mu;
+    if (a.mu_t) mu = mu + a.mu_t[e];
+    viscous_flux(D, st, gt, mu, f);
+    if (valid)
+        *reinterpret_cast<FvQuad<CT>*>(a.fv + e * kFvStride + (2 * D + side) * 64 + fp * 4) =
+            FvQuad<CT>{{f[1], f[2], f[3], f[4]}};
+}
+template <int D, class UT, class CT>
+__device__ __forceinline__ void strict_line_flux(const StageArgs<UT, CT>& a, const CT* area, int e0, int E,
+                                                 const StrictLine<CT>& w) {
+    const Ops<CT>& o = dev_ops<CT>();
+    CT gl[15], gr[15];
+#pragma unroll
+    for (int q = 0; q < 15; ++q) {
+        // what the flux along D reads: the density's gradient, the momenta's
+        // along D, across D of momentum D and on the diagonal, the energy's along D
+        const int v = q / 3, c = q % 3;
+        const bool used = v == 0 || c == D || (v < 4 && (v - 1 == D || v - 1 == c));
+        if (!used) {
+            gl[q] = gr[q] = (CT)0;
+            continue;
+        }
+        CT x[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) x[m] = area[w.pos[m] + q * 64];
+        gl[q] = trace4(x, 0, 1, o.eL[0], o.eL[1], o.eL[2], o.eL[3], fv_order(D));
+        gr[q] = trace4(x, 0, 1, o.eR[0], o.eR[1], o.eR[2], o.eR[3], fv_order(D));
+        asm volatile("" : "+v"(gl[q]), "+v"(gr[q])::"memory");
+    }
+    const bool valid = e0 + w.le < E;
+    const int64_t e = valid ? e0 + w.le : E - 1;
+    strict_end_flux<D>(a, e, valid, w.tl, gl, 0, w.fp);
+    asm volatile("" ::: "memory");  // one end, then the other
+    strict_end_flux<D>(a, e, valid, w.tr, gr, 1, w.fp);
+}
+
+template <class UT, class CT>
+__global__ __launch_bounds__(64 * kQuad) void od_visc_line_kernel(StageArgs<UT, CT> a) {
+    __shared__ CT area[kQuad * kAreaStride];
+    const int wave = wave_index(), pt = threadIdx.x & 63;
+    const int i = pt & 3, j = (pt >> 2) & 3, k = pt >> 4;
+    const int E = a.nx * a.ny * a.nz, e0 = kQuad * (int)blockIdx.x;
+    const int64_t NP = (int64_t)E * 64;
+    const bool valid = e0 + wave < E;
+    const int64_t e = valid ? e0 + wave : E - 1;
+    // wave -> direction (3: none), turning from work-group to work-group of an
+    // XCD so that the SIMDs get equally many line waves
+    const int D = (wave + ((int)blockIdx.x >> 3)) & 3;
+    const CT cf = coef_load<CT>((int)threadIdx.x);
+    UT s0[5];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) s0[v] = a.uin[v * NP + e * 64 + pt];
+    StrictLine<CT> w;
+    if (D == 0)
+        strict_line_begin<0>(a, e0, E, pt, w);
+    else if (D == 1)
+        strict_line_begin<1>(a, e0, E, pt, w);
+    else if (D == 2)
+        strict_line_begin<2>(a, e0, E, pt, w);
+    {
+        CT* A = area + wave * kAreaStride + swz64(pt);
+#pragma unroll
+        for (int v = 0; v < 5; ++v) A[v * 64] = (CT)s0[v];
+    }
+    coef_store<CT>((int)threadIdx.x, cf);
+    __syncthreads();
+    if (D < 3) {
+#pragma unroll
+        for (int v = 0; v < 5; ++v)
+#pragma unroll
+            for (int m = 0; m < 4; ++m) w.u[v][m] = area[w.pos[m] + v * 64];
+    }
+    __syncthreads();  // the gradients overwrite the states
+    if (D == 0)
+        strict_line_gradient<0>(a, area, w);
+    else if (D == 1)
+        strict_line_gradient<1>(a, area, w);
+    else if (D == 2)
+        strict_line_gradient<2>(a, area, w);
+    __syncthreads();
+    if (D == 0)
+        strict_line_flux<0>(a, area, e0, E, w);
+    else if (D == 1)
+        strict_line_flux<1>(a, area, e0, E, w);
+    else if (D == 2)
+        strict_line_flux<2>(a, area, e0, E, w);
+    CT g[15], st[5], r[5];
+    {
+        const CT* A = area + wave * kAreaStride + swz64(pt);
+#pragma unroll
+        for (int q = 0; q < 15; ++q) g[q] = A[q * 64];
+    }
+#pragma unroll
+    for (int v = 0; v < 5; ++v) st[v] = (CT)a.uin[v * NP + e * 64 + pt];  // again (from L2), not held all along
+    __syncthreads();  // the volume fluxes' lines are staged over the gradients
+    CT mu = a.sutherland ? sutherland(st, a.mu_ref, a.t_ref, a.s_suth) : a.mu;
+    if (a.mu_t) mu = mu + a.mu_t[e];
+    volume_rhs<true>(a, st, g, mu, (const CT*)nullptr, (CT(*)[64])(area + wave * kAreaStride), i, j, k, pt, r);
+    if (valid) {
+#pragma unroll
+        for (int v = 0; v < 5; ++v) a.fv[e * kFvStride + kFvFaces + v * 64 + pt] = r[v];
+    }
+}
+#endif
 
 #if OD_FAST
 // ---------------------------------------------------------------------------
@@ -1974,18 +2201,11 @@ __device__ __forceinline__ void update_block_body(const StageArgs<float, float>&
 // than their size, so that the partner along x, y, z is 4, 8, 16 banks away,
 // the bit that swz64 keeps fixed over a face of that direction.
 // ---------------------------------------------------------------------------
-constexpr int kAreaStride = 15 * 64 + 4;
 struct BlockViscLds {
     alignas(16) float area[kBlk * kAreaStride];
     __device__ float* of(int le) { return area + le * kAreaStride; }
 };
 
-// swz64 position of the line point m of direction D relative (XOR) to m = 0.
-template <int D>
-__device__ constexpr int line_xor(int m) {
-    const int lo = m & 1, hi = m >> 1;
-    return D == 0 ? ((lo ? 1 | 2 | 32 : 0) | hi << 2) : (D == 1 ? (lo | hi << 3) : (hi << 1 | lo << 4));
-}
 // The value of the lane's partner, lane ^ 1.
 __device__ __forceinline__ float lane_partner(float x) {
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xF, 0xF, false));  // quad_perm [1,0,3,2]
@@ -2585,7 +2805,12 @@ int launch_trace(const StageArgs<UT, CT>& a, int64_t n_elem, void* stream) {
 
 template <class UT, class CT>
 int launch_visc(const StageArgs<UT, CT>& a, int64_t n_elem, void* stream) {
+#if OD_FAST
     hipLaunchKernelGGL((od_visc_kernel<UT, CT>), grid_of(a), dim3(64 * kEpb), 0, (hipStream_t)stream, a);
+#else
+    hipLaunchKernelGGL((od_visc_line_kernel<UT, CT>), dim3((unsigned)((n_elem + kQuad - 1) / kQuad)),
+                       dim3(64 * kQuad), 0, (hipStream_t)stream, a);
+#endif
     return check_launch();
 }
 
