@@ -801,53 +801,43 @@ __device__ __forceinline__ int64_t tile_nb_rt(const Tile& t, int le, int f) {
 // Neighbour-trace prefetch (f32 compute).  At kernel start each work-group
 // copies the neighbour traces it will read straight from global memory into
 // LDS with gfx950's global_load_lds_dwordx4 (no registers, one exposed
-// latency), as 16-byte chunks:
-//   A [0, 240)    neighbour facing traces, BR1 order, faces 0..5: 2 x 6 x 80
-//   B [240, 320)  neighbour facing x traces, sequential order:   2 x 2 x 80
-//                 (strict build only; the fast build has one x trace)
+// latency), as 240 16-byte chunks: the facing traces of faces 0..5 of both
+// elements, [2][6][5][16] -- in the BR1 order for the visc kernel, in that of
+// the Riemann inputs for the update kernel (RIEMANN; in the strict build the x
+// faces' other trace).
 // The face viscous fluxes fv are read from global memory in the face pass
 // instead: staging them too (another 1536 floats) limited the update kernel
 // to 4.5 waves per SIMD by LDS; without them it runs 6 (a step measured
 // ~6 % faster in both builds).
-// The float offsets of the two groups in the buffer:
-constexpr int kPfA = 0, kPfB = 960;
-constexpr int kPfChunksVisc = 240;                            // visc kernel: A
-constexpr int kPfChunksUpdate = kOneX ? 240 : 320;            // update kernel: A (+ B)
-constexpr int kPfFloatsUpdate = 4 * kPfChunksUpdate;
+constexpr int kPfChunks = 240;
+constexpr int kPfFloats = 4 * kPfChunks;
 
 // Source of chunk `id`; false for chunks of a missing second element (odd
 // nx), which are not copied.
-template <class UT, class CT>
+template <bool RIEMANN, class UT, class CT>
 __device__ __forceinline__ bool prefetch_chunk(const StageArgs<UT, CT>& a, const Tile& tl, int id, const CT*& src) {
-    if (id < 240) {  // A
-        const int le = id / 120, f = (id % 120) / 20, c = id % 20;
-        if (!tile_valid(tl, le)) return false;
-        const int64_t own = tile_eidx(tl, le), nb = tile_nb_rt(tl, le, f);
-        src = a.tr_in + (nb >= 0 ? nb : own) * kTraceStride + (f ^ 1) * 80 + c * 4;
-    } else {  // B
-        if (kOneX) return false;  // the x Riemann inputs are group A's
-        const int r = id - 240, le = r / 40, f = (r % 40) / 20, c = r % 20;
-        if (!tile_valid(tl, le)) return false;
-        const int64_t nb = tile_nb_rt(tl, le, f);  // x is periodic: always a neighbour
-        src = a.tr_in + nb * kTraceStride + (f == 0 ? 7 : 6) * 80 + c * 4;
-    }
+    const int le = id / 120, f = (id % 120) / 20, c = id % 20;
+    if (!tile_valid(tl, le)) return false;
+    const int64_t own = tile_eidx(tl, le), nb = tile_nb_rt(tl, le, f);
+    const int slot = (RIEMANN && !kOneX && f < 2) ? 7 - f : f ^ 1;
+    src = a.tr_in + (nb >= 0 ? nb : own) * kTraceStride + slot * 80 + c * 4;
     return true;
 }
 
-// Issue the first n_chunks chunks; waves split the 64-chunk instructions.
+// Issue the chunks; waves split the 64-chunk instructions.
 // The caller waits (s_waitcnt 0, then a barrier for the other wave's copies)
 // before reading the buffer.
-template <class UT, class CT>
-__device__ __forceinline__ void prefetch_issue(const StageArgs<UT, CT>& a, const Tile& tl, float* pf, int n_chunks,
-                                               int wave, int lane) {
-    const int n_inst = (n_chunks + 63) / 64;
+template <bool RIEMANN, class UT, class CT>
+__device__ __forceinline__ void prefetch_issue(const StageArgs<UT, CT>& a, const Tile& tl, float* pf, int wave,
+                                               int lane) {
+    constexpr int n_inst = (kPfChunks + 63) / 64;
     wave = __builtin_amdgcn_readfirstlane(wave);  // wave-uniform: a scalar loop
     const int first = wave == 0 ? 0 : (n_inst + 1) / 2;
     const int last = wave == 0 ? (n_inst + 1) / 2 : n_inst;
     for (int q = first; q < last; ++q) {
         const int id = q * 64 + lane;
         const CT* src = nullptr;
-        if (id < n_chunks && prefetch_chunk(a, tl, id, src)) {
+        if (id < kPfChunks && prefetch_chunk<RIEMANN>(a, tl, id, src)) {
             __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
                                              (__attribute__((address_space(3))) void*)(pf + q * 256), 16, 0, 0);
         }
@@ -875,7 +865,7 @@ __device__ __forceinline__ void br1_jumps(const StageArgs<UT, CT>& a, const CT (
         const CT sign = (v > 0 && v < 4) ? ((CT)-1.0) : ((CT)1.0);
         CT far;
         if constexpr (PF)
-            far = pf[kPfA + (t.le * 6 + t.f) * 80 + v * 16 + t.fp];
+            far = pf[(t.le * 6 + t.f) * 80 + v * 16 + t.fp];
         else
             far = !wall ? a.tr_in[nb * kTraceStride + (t.f ^ 1) * 80 + v * 16 + t.fp] : (CT)0;
         CT nbv = !wall ? far : own * sign;
@@ -1076,8 +1066,7 @@ __device__ __forceinline__ void flux_pass(const StageArgs<UT, CT>& a, const CT (
     for (int v = 0; v < 5; ++v) {
         CT far;
         if constexpr (PF)
-            far = (D == 0 && !kOneX) ? pf[kPfB + (t.le * 2 + t.side) * 80 + v * 16 + t.fp]
-                         : pf[kPfA + (t.le * 6 + t.f) * 80 + v * 16 + t.fp];
+            far = pf[(t.le * 6 + t.f) * 80 + v * 16 + t.fp];
         else
             far = wall ? own[v] : a.tr_in[nb * kTraceStride + rf * 80 + v * 16 + t.fp];
         oth[v] = wall ? own[v] : far;
@@ -1306,12 +1295,12 @@ __device__ __forceinline__ void volume_rhs(const StageArgs<UT, CT>& a, const CT*
 template <class CT>
 struct ViscLds {
     static constexpr bool kPF = std::is_same<CT, float>::value;
-    float pf[kPF ? kPfB : 4];
+    float pf[kPF ? kPfFloats : 4];
     CT sJmp[kEpb][6][5][16];
     CT sU[kEpb][5][64];
     CT sG_own[kPF ? 0 : kEpb][15][64];  // zero-length when aliased
     __device__ CT (*sG())[15][64] {
-        static_assert(!kPF || (kPfB == 15 * 64 && sizeof(sJmp) == kPfB * sizeof(float)), "sG aliasing layout");
+        static_assert(!kPF || (kPfFloats == 15 * 64 && sizeof(sJmp) == kPfFloats * sizeof(float)), "sG aliasing layout");
         if constexpr (kPF) return reinterpret_cast<CT(*)[15][64]>(pf);
         else return sG_own;
     }
@@ -1322,7 +1311,7 @@ struct ViscLds {
 };
 
 // With the prefetch (f32 compute) the face-correction array sJ shares the
-// prefetched neighbour traces (group A has sJ's exact layout and each face
+// prefetched neighbour traces (they have sJ's exact layout and each face
 // point's lane reads its entries there before it writes them).  sF: staging of
 // the volume fluxes' lines, where this kernel forms them (kVol): the Euler mode
 // and the fast build.
@@ -1330,12 +1319,12 @@ template <class CT, bool VISC>
 struct UpdateLds {
     static constexpr bool kPF = std::is_same<CT, float>::value;
     static constexpr bool kVol = !VISC || kSplitVisc<CT>;
-    float pf[kPF ? kPfFloatsUpdate : 4];
+    float pf[kPF ? kPfFloats : 4];
     CT sU[kEpb][5][64];
     CT sJ_own[kPF ? 0 : kEpb][6][5][16];  // zero-length when aliased
     CT sF[kVol ? kEpb : 0][5][64];
     __device__ CT (*sJ())[6][5][16] {
-        if constexpr (kPF) return reinterpret_cast<CT(*)[6][5][16]>(pf + kPfA);
+        if constexpr (kPF) return reinterpret_cast<CT(*)[6][5][16]>(pf);
         else return sJ_own;
     }
 };
@@ -1364,7 +1353,7 @@ __device__ __forceinline__ void visc_body(const StageArgs<UT, CT>& a, const Tile
     const int i = pt & 3, j = (pt >> 2) & 3, k = pt >> 4;
     const int64_t NP = (int64_t)a.nx * a.ny * a.nz * 64;
     const CT cf = coef_load<CT>((int)threadIdx.x);
-    if constexpr (PF) prefetch_issue(a, tl, L.pf, kPfChunksVisc, wave, pt);
+    if constexpr (PF) prefetch_issue<false>(a, tl, L.pf, wave, pt);
     if (tile_valid(tl, wave)) load_state_tile(a.uin, NP, tile_eidx(tl, wave), L.sU[wave], pt);
     coef_store<CT>((int)threadIdx.x, cf);
     if constexpr (PF) __builtin_amdgcn_s_waitcnt(0);  // this wave's LDS copies have landed
@@ -1416,11 +1405,10 @@ __device__ __forceinline__ void update_body(const StageArgs<UT, CT>& a, const Ti
     const int64_t NP = (int64_t)a.nx * a.ny * a.nz * 64;
     const int64_t gbase = tile_eidx(tl, wave) * 64 + pt;
     const CT cf = coef_load<CT>((int)threadIdx.x);
-    if constexpr (PF) prefetch_issue(a, tl, L.pf, kPfChunksUpdate, wave, pt);
+    if constexpr (PF) prefetch_issue<true>(a, tl, L.pf, wave, pt);
 
     constexpr bool SAME = std::is_same<UT, CT>::value;  // sU holds the state exactly
-    UT ucur[5];
-    if constexpr (SAME && PF) {  // f32 state and compute: LDS-DMA, read back from sU below
+    if constexpr (SAME && PF) {  // f32 state and compute: LDS-DMA
         if (mine) {
             load_state_tile(a.uin, NP, tile_eidx(tl, wave), L.sU[wave], pt);
         } else {
@@ -1429,10 +1417,7 @@ __device__ __forceinline__ void update_body(const StageArgs<UT, CT>& a, const Ti
         }
     } else {
 #pragma unroll
-        for (int v = 0; v < 5; ++v) {
-            ucur[v] = mine ? a.uin[v * NP + gbase] : (UT)1;
-            L.sU[wave][v][pt] = (CT)ucur[v];
-        }
+        for (int v = 0; v < 5; ++v) L.sU[wave][v][pt] = (CT)(mine ? a.uin[v * NP + gbase] : (UT)1);
     }
     coef_store<CT>((int)threadIdx.x, cf);
     if constexpr (PF) __builtin_amdgcn_s_waitcnt(0);  // this wave's LDS copies have landed
@@ -1489,7 +1474,12 @@ __device__ __forceinline__ void update_body(const StageArgs<UT, CT>& a, const Ti
     CT r[5];
 #pragma unroll
     for (int v = 0; v < 5; ++v) {
-        ucr[v] = SAME ? (UT)L.sU[wave][v][pt] : ucur[v];
+        // the state in its own type: from LDS, or again from L2 (held in f64
+        // from the start it cost the f32 fluxes a wave per SIMD)
+        if constexpr (SAME)
+            ucr[v] = (UT)L.sU[wave][v][pt];
+        else
+            ucr[v] = mine ? a.uin[v * NP + gbase] : (UT)1;
         if constexpr (VOL)
             r[v] = L.sF[wave][v][pt];
         else
@@ -1579,13 +1569,12 @@ __global__ __launch_bounds__(128) void od_visc_kernel(StageArgs<UT, CT> a) {
 }
 #endif
 
-// Occupancy target of the update kernels.  The strict f32 build needs ~78
-// VGPRs (6 waves per SIMD).  The fast all-f32 single-box kernel and the batch
-// kernel's single-unit form, which need no gradient there (kSplitVisc), are
-// held to 64 (8 waves; they need 61 with no spills; their LDS, 9.1 KB per
-// work-group, allows 8).  The strict build, f64 states and the persistent batch kernel
-// keep their natural allocation (the 4-wave cap does not bind); f64 compute
-// needs ~145 VGPRs.
+// Occupancy target of the update kernels.  The fast all-f32 single-box kernel
+// and the batch kernel's single-unit form are held to 64 VGPRs (8 waves per
+// SIMD; they need 61 with no spills; their LDS, 9.1 KB per work-group, allows
+// 8).  The strict build (70 VGPRs, 7 waves), f64 states and the persistent batch
+// kernel keep their natural allocation (the 4-wave cap does not bind); f64
+// compute needs 120 VGPRs (4 waves).
 template <class CT>
 constexpr int kMinWaves = sizeof(CT) == 4 ? 4 : 1;
 template <class UT, class CT>
