@@ -141,7 +141,7 @@ od_status od_time_steps(od_ctx* ctx, double dt, uint32_t n_steps, double* ms_tot
 
 /* Time every kernel launch of n_steps steps individually (events around each
  * launch, no graph).  out_ms[q] = mean duration of kernel kind q; names[q]
- * its name.  Kinds: 0 = od_visc_kernel, 1 = od_update_kernel. */
+ * its name.  Kinds: 0 = the viscous kernel, 1 = the update kernel. */
 od_status od_time_kernels(od_ctx* ctx, double dt, uint32_t n_steps, double out_ms[4],
                           const char* names[4], int* n_kinds);
 

@@ -173,9 +173,22 @@ int launch_kind(od_ctx* c, int kind, int stage, double dt, int mode) {
             return od::fastmath::launch_update<UT, CT, false>(a, c->E, c->stream);
         }
     }
+    if (strict_blocks(c->p)) return od::launch_strict_block<UT, CT>(a, kind, c->stream);
     if (kind == 0) return od::launch_visc<UT, CT>(a, c->E, c->stream);
     if (c->p.viscous) return od::launch_update<UT, CT, true>(a, c->E, c->stream);
     return od::launch_update<UT, CT, false>(a, c->E, c->stream);
+}
+
+// The kernel that launch_kind launches as kind 0 or 1.
+const char* kernel_name(const od_params& p, int kind) {
+    switch (box_form(p, p.nx, p.ny, p.nz)) {
+        case BoxForm::blocks: return kind ? "od_update_block_kernel" : "od_visc_block_kernel";
+        case BoxForm::core_shell: return kind ? "od_update_core_shell_kernel" : "od_visc_core_shell_kernel";
+        case BoxForm::tiles: break;
+    }
+    if (strict_blocks(p)) return kind ? "od_update_face_block_kernel" : "od_visc_lines_block_kernel";
+    if (kind) return "od_update_kernel";
+    return fast_kernels(p) ? "od_visc_kernel" : "od_visc_line_kernel";
 }
 
 int launch(od_ctx* c, int kind, int stage, double dt, int mode = 0) {
@@ -658,12 +671,7 @@ od_status od_time_kernels(od_ctx* c, double dt, uint32_t n_steps, double out_ms[
     for (hipEvent_t e : ev) (void)hipEventDestroy(e);
     for (int k = 0; k < 4; ++k) {
         out_ms[k] = (k < kinds && cnt[k]) ? sum[k] / cnt[k] : 0.0;
-        const char* nm = k < kinds ? od::kernel_name(k) : "";
-        const BoxForm form = box_form(c->p, c->p.nx, c->p.ny, c->p.nz);
-        if (form == BoxForm::blocks) nm = k == 0 ? "od_visc_block_kernel" : k == 1 ? "od_update_block_kernel" : nm;
-        if (form == BoxForm::core_shell)
-            nm = k == 0 ? "od_visc_core_shell_kernel" : k == 1 ? "od_update_core_shell_kernel" : nm;
-        if (names) names[k] = nm;
+        if (names) names[k] = k < kinds ? kernel_name(c->p, k) : "";
     }
     if (n_kinds) *n_kinds = kinds;
     return OD_OK;

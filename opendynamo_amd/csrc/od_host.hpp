@@ -56,6 +56,18 @@ inline BoxForm box_form(const od_params& p, int nx, int ny, int nz) {
         return BoxForm::tiles;
     return nx % 2 || ny % 2 || nz % 2 ? BoxForm::core_shell : BoxForm::blocks;
 }
+// Whether a strict viscous box runs on 2x2x2-element blocks when it is a context
+// of its own (a batch's boxes all run on tiles): even dimensions, and two and a
+// half blocks for each of the 256 CUs.  Below that the smaller work-groups of
+// the other kernels fill the chip better and finish sooner: us a step, blocks
+// against them, f32 / f64 / f64 state with f32 fluxes: 8^3 44 40 / 59 50 / 47 43,
+// 12^3 54 51 / 73 74 / 56 56, 16^3 71 71 / 102 107 / 80 78, 20^3 107 117 /
+// 178 196 / 124 139.
+constexpr int64_t kStrictBlocks = 640;
+inline bool strict_blocks(const od_params& p) {
+    return !fast_kernels(p) && p.viscous && p.nx % 2 == 0 && p.ny % 2 == 0 && p.nz % 2 == 0 &&
+           (int64_t)p.nx * p.ny * p.nz >= 8 * kStrictBlocks;
+}
 // Launch of kind 0 visc, 1 update of a box whose form is not tiles.
 int launch_block_form(const od::StageArgs<float, float>& a, bool viscous, int kind, hipStream_t stream);
 

@@ -127,6 +127,12 @@ template <class UT, class CT>
 int launch_visc(const StageArgs<UT, CT>& a, int64_t n_elem, void* stream);
 template <class UT, class CT, bool VISC>
 int launch_update(const StageArgs<UT, CT>& a, int64_t n_elem, void* stream);
+// Strict build, viscous, nx, ny, nz even: the same results as launch_visc (kind
+// 0) and launch_update (1), bit for bit, on blocks of 2x2x2 elements.  The update
+// kernel writes the traces of the blocks' external faces only, which is all this
+// visc kernel reads.
+template <class UT, class CT>
+int launch_strict_block(const StageArgs<UT, CT>& a, int kind, void* stream);
 template <class UT, class CT>
 int launch_batch_visc(const StageArgs<UT, CT>& a, const BatchArgs<UT, CT>& b, int pairs, int groups, void* stream);
 template <class UT, class CT, bool VISC>
@@ -146,8 +152,6 @@ int launch_cfl(const UT* u, double* partial, int64_t n_elem, double dx, double d
 template <class UT>
 int launch_sums(const UT* u, double* partial, double* out, int64_t n_elem, const double w3[64],
                 double jac, void* stream);
-
-const char* kernel_name(int kind);
 
 // The same kernels built with fast math (f32 compute only): reciprocal
 // multiplies, hardware square root, contraction (od_kernels_fast.hip).

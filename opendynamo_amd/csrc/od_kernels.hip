@@ -1393,6 +1393,41 @@ __device__ __forceinline__ void visc_body(const StageArgs<UT, CT>& a, const Tile
     }
 }
 
+// Stage update of a point: u^n, the stage's state and its RHS -> the new state
+// (rk.cu:12-25, 63-82).
+template <class UT, class CT>
+__device__ __forceinline__ void rk_stage(const StageArgs<UT, CT>& a, const StageDt<UT, CT>& cdt, const UT* uprv,
+                                         const UT* ucr, const CT* rts, UT* unew) {
+    if constexpr (std::is_same<UT, CT>::value) {
+        // one type: the compute-type and the state-type blends differ only
+        // in their coefficients, chosen once; uniform branch on the stage
+        const CT kA = a.accum_state ? a.ua : a.ca;
+        const CT kB = a.accum_state ? a.ub : a.cb;
+        const CT kC = a.accum_state ? cdt.uc : cdt.cc;
+        if (a.stage1) {
+#pragma unroll
+            for (int v = 0; v < 5; ++v) unew[v] = rk_blend1(kA, kC, uprv[v], rts[v]);
+        } else {
+#pragma unroll
+            for (int v = 0; v < 5; ++v) unew[v] = rk_blend(kA, kB, kC, uprv[v], ucr[v], rts[v]);
+        }
+    } else {
+#pragma unroll
+        for (int v = 0; v < 5; ++v) {
+            const CT rt = rts[v];
+            if (!a.accum_state) {
+                CT up = (CT)uprv[v], uc = (CT)ucr[v];
+                CT val = a.stage1 ? (a.ca * up + cdt.cc * rt) : (a.ca * up + a.cb * uc + cdt.cc * rt);
+                unew[v] = (UT)val;
+            } else {
+                UT rr = (UT)rt;
+                unew[v] =
+                    a.stage1 ? (UT)(a.ua * uprv[v] + cdt.uc * rr) : (UT)(a.ua * uprv[v] + a.ub * ucr[v] + cdt.uc * rr);
+            }
+        }
+    }
+}
+
 // Full stage for the tile: volume RHS, interface fluxes, FR correction, RK
 // blend, and the face traces of the new state.
 template <class UT, class CT, bool VISC>
@@ -1514,34 +1549,7 @@ __device__ __forceinline__ void update_body(const StageArgs<UT, CT>& a, const Ti
         return;
     }
     UT unew[5];
-    if constexpr (std::is_same<UT, CT>::value) {
-        // one type: the compute-type and the state-type blends differ only
-        // in their coefficients, chosen once; uniform branch on the stage
-        const CT kA = a.accum_state ? a.ua : a.ca;
-        const CT kB = a.accum_state ? a.ub : a.cb;
-        const CT kC = a.accum_state ? cdt.uc : cdt.cc;
-        if (a.stage1) {
-#pragma unroll
-            for (int v = 0; v < 5; ++v) unew[v] = rk_blend1(kA, kC, uprv[v], rts[v]);
-        } else {
-#pragma unroll
-            for (int v = 0; v < 5; ++v) unew[v] = rk_blend(kA, kB, kC, uprv[v], ucr[v], rts[v]);
-        }
-    } else {
-#pragma unroll
-        for (int v = 0; v < 5; ++v) {
-            const CT rt = rts[v];
-            if (!a.accum_state) {
-                CT up = (CT)uprv[v], uc = (CT)ucr[v];
-                CT val = a.stage1 ? (a.ca * up + cdt.cc * rt) : (a.ca * up + a.cb * uc + cdt.cc * rt);
-                unew[v] = (UT)val;
-            } else {
-                UT rr = (UT)rt;
-                unew[v] =
-                    a.stage1 ? (UT)(a.ua * uprv[v] + cdt.uc * rr) : (UT)(a.ua * uprv[v] + a.ub * ucr[v] + cdt.uc * rr);
-            }
-        }
-    }
+    rk_stage(a, cdt, uprv, ucr, rts, unew);
 #pragma unroll
     for (int v = 0; v < 5; ++v)
         if (mine) stream_store(unew[v], &a.uout[v * NP + gbase]);
@@ -1597,232 +1605,7 @@ __device__ constexpr int line_xor(int m) {
     return D == 0 ? ((lo ? 1 | 2 | 32 : 0) | hi << 2) : (D == 1 ? (lo | hi << 3) : (hi << 1 | lo << 4));
 }
 
-#if !OD_FAST
-// ---------------------------------------------------------------------------
-// Strict build, one box: the visc kernel by lines.  A 256-thread work-group has
-// four consecutive elements; in the line phases wave d < 3 takes direction d,
-// lane = (element, line of four points), and forms from one read of the line's
-// states both end traces, both BR1 jumps and the corrected derivative at its
-// four points, then from one read of the line's gradients the viscous fluxes at
-// both ends.  The neighbours' traces come straight from memory, the operators
-// are wave-uniform.  The volume RHS is point-wise, a wave per element.  Every
-// value is the expression of visc_body, in the reference's order.
-// Bounds: instruction issue.  Against the point-wise form (visc_body, which the
-// batches' tiles use), whose lanes read each state 12 and each gradient 6 to 8
-// times from LDS: 24x26x22 f64 102 -> 61 us, 48^3 f32 279 -> 231 us, 24x20x28
-// f64 state with f32 fluxes 40 -> 33 us a launch.
-// LDS: one area per element, the states, then the gradients over them.
-// ---------------------------------------------------------------------------
-constexpr int kQuad = 4;
-
-template <class CT>
-struct StrictLine {
-    int le, fp;
-    CT u[5][4];
-    CT tl[5], tr[5];  // end traces in the order of the viscous fluxes
-    CT nl[5], nr[5];  // the neighbours' facing traces
-    bool wl, wr;      // slip walls
-    int pos[4];
-};
-
-// Element e0's coordinates and the neighbours across both faces of direction D
-// of the lane's element e0 + le (those past the mesh's last one repeat it).
-template <int D, class UT, class CT>
-__device__ __forceinline__ void strict_line_begin(const StageArgs<UT, CT>& a, int e0, int E, int lane,
-                                                  StrictLine<CT>& w) {
-    w.le = lane >> 4;
-    w.fp = lane & 15;
-    int ez = e0 / (a.nx * a.ny), ey = (e0 - ez * a.nx * a.ny) / a.nx, ex = e0 - a.nx * (ey + a.ny * ez);
-    int l[kQuad], r[kQuad];
-#pragma unroll
-    for (int q = 0; q < kQuad; ++q) {
-        const Elem n = make_elem(ex, ey, ez, a.nx, a.ny, a.nz, a.wall);
-        l[q] = D == 0 ? n.xl : (D == 1 ? n.yl : n.zl);
-        r[q] = D == 0 ? n.xr : (D == 1 ? n.yr : n.zr);
-        if (e0 + q + 1 < E) {
-            ++ex;
-            if (ex == a.nx) {
-                ex = 0;
-                ++ey;
-                if (ey == a.ny) {
-                    ey = 0;
-                    ++ez;
-                }
-            }
-        }
-    }
-    const bool b0 = w.le & 1, b1 = w.le & 2;
-    const int nl = b1 ? (b0 ? l[3] : l[2]) : (b0 ? l[1] : l[0]);
-    const int nr = b1 ? (b0 ? r[3] : r[2]) : (b0 ? r[1] : r[0]);
-    w.wl = D == 1 && nl < 0;
-    w.wr = D == 1 && nr < 0;
-    const CT* tl = a.tr_in + (int64_t)(w.wl ? 0 : nl) * kTraceStride + (2 * D + 1) * 80 + w.fp;
-    const CT* tr = a.tr_in + (int64_t)(w.wr ? 0 : nr) * kTraceStride + (2 * D) * 80 + w.fp;
-#pragma unroll
-    for (int v = 0; v < 5; ++v) {
-        w.nl[v] = tl[v * 16];
-        w.nr[v] = tr[v * 16];
-    }
-    int base, stride;
-    face_line(D, w.fp, base, stride);
-    const int s0 = swz64(base);
-#pragma unroll
-    for (int m = 0; m < 4; ++m) w.pos[m] = w.le * kAreaStride + (s0 ^ line_xor<D>(m));
-}
-
-// Jumps (br1_jumps) and corrected derivative along D (lane_gradient_faces) ->
-// the gradient's rows 3 v + D.
-template <int D, class UT, class CT>
-__device__ __forceinline__ void strict_line_gradient(const StageArgs<UT, CT>& a, CT* area, StrictLine<CT>& w) {
-    const Ops<CT>& o = dev_ops<CT>();
-    const CT jac = D == 0 ? a.jx : (D == 1 ? a.jy : a.jz);
-#pragma unroll
-    for (int v = 0; v < 5; ++v) {
-        const CT* u = w.u[v];
-        const CT tl = trace4(u, 0, 1, o.eL[0], o.eL[1], o.eL[2], o.eL[3], br1_order(D));
-        const CT tr = trace4(u, 0, 1, o.eR[0], o.eR[1], o.eR[2], o.eR[3], br1_order(D));
-        const CT sign = (v > 0 && v < 4) ? ((CT)-1.0) : ((CT)1.0);
-        const CT nl = w.wl ? tl * sign : w.nl[v], nr = w.wr ? tr * sign : w.nr[v];
-        const CT jl = ((CT)0.5) * (nl + tl) - tl, jr = ((CT)0.5) * (nr + tr) - tr;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            CT d = 0;
-#pragma unroll
-            for (int m = 0; m < 4; ++m) d += o.D[4 * i + m] * u[m];
-            CT g = d * jac;
-            g += jl * o.gL[i] * jac;
-            g += jr * o.gR[i] * jac;
-            if (a.round_q) g = (CT)(float)g;  // Q_REAL round trip (rhs.cu:457-461)
-            area[w.pos[i] + (3 * v + D) * 64] = g;
-        }
-        w.tl[v] = D == 0 ? trace4(u, 0, 1, o.eL[0], o.eL[1], o.eL[2], o.eL[3], fv_order(D)) : tl;
-        w.tr[v] = D == 0 ? trace4(u, 0, 1, o.eR[0], o.eR[1], o.eR[2], o.eR[3], fv_order(D)) : tr;
-        asm volatile("" : "+v"(w.tl[v]), "+v"(w.tr[v])::"memory");  // variable by variable (see lane_gradient_faces)
-    }
-}
-
-// Viscous flux at one end of the line (fv_value) from its state trace and
-// gradient trace -> the element's slot of face 2 D + side.
-template <int D, class UT, class CT>
-__device__ __forceinline__ void strict_end_flux(const StageArgs<UT, CT>& a, int64_t e, bool valid, const CT* st,
-                                                const CT* gt, int side, int fp) {
-    CT f[5];
-    CT mu = a.sutherland ? sutherland(st, a.mu_ref, a.t_ref, a.s_suth) : a.mu;
-    if (a.mu_t) mu = mu + a.mu_t[e];
-    viscous_flux(D, st, gt, mu, f);
-    if (valid)
-        *reinterpret_cast<FvQuad<CT>*>(a.fv + e * kFvStride + (2 * D + side) * 64 + fp * 4) =
-            FvQuad<CT>{{f[1], f[2], f[3], f[4]}};
-}
-template <int D, class UT, class CT>
-__device__ __forceinline__ void strict_line_flux(const StageArgs<UT, CT>& a, const CT* area, int e0, int E,
-                                                 const StrictLine<CT>& w) {
-    const Ops<CT>& o = dev_ops<CT>();
-    CT gl[15], gr[15];
-#pragma unroll
-    for (int q = 0; q < 15; ++q) {
-        // what the flux along D reads: the density's gradient, the momenta's
-        // along D, across D of momentum D and on the diagonal, the energy's along D
-        const int v = q / 3, c = q % 3;
-        const bool used = v == 0 || c == D || (v < 4 && (v - 1 == D || v - 1 == c));
-        if (!used) {
-            gl[q] = gr[q] = (CT)0;
-            continue;
-        }
-        CT x[4];
-#pragma unroll
-        for (int m = 0; m < 4; ++m) x[m] = area[w.pos[m] + q * 64];
-        gl[q] = trace4(x, 0, 1, o.eL[0], o.eL[1], o.eL[2], o.eL[3], fv_order(D));
-        gr[q] = trace4(x, 0, 1, o.eR[0], o.eR[1], o.eR[2], o.eR[3], fv_order(D));
-        asm volatile("" : "+v"(gl[q]), "+v"(gr[q])::"memory");
-    }
-    const bool valid = e0 + w.le < E;
-    const int64_t e = valid ? e0 + w.le : E - 1;
-    strict_end_flux<D>(a, e, valid, w.tl, gl, 0, w.fp);
-    asm volatile("" ::: "memory");  // one end, then the other
-    strict_end_flux<D>(a, e, valid, w.tr, gr, 1, w.fp);
-}
-
-template <class UT, class CT>
-__global__ __launch_bounds__(64 * kQuad) void od_visc_line_kernel(StageArgs<UT, CT> a) {
-    __shared__ CT area[kQuad * kAreaStride];
-    const int wave = wave_index(), pt = threadIdx.x & 63;
-    const int i = pt & 3, j = (pt >> 2) & 3, k = pt >> 4;
-    const int E = a.nx * a.ny * a.nz, e0 = kQuad * (int)blockIdx.x;
-    const int64_t NP = (int64_t)E * 64;
-    const bool valid = e0 + wave < E;
-    const int64_t e = valid ? e0 + wave : E - 1;
-    // wave -> direction (3: none), turning from work-group to work-group of an
-    // XCD so that the SIMDs get equally many line waves
-    const int D = (wave + ((int)blockIdx.x >> 3)) & 3;
-    const CT cf = coef_load<CT>((int)threadIdx.x);
-    UT s0[5];
-#pragma unroll
-    for (int v = 0; v < 5; ++v) s0[v] = a.uin[v * NP + e * 64 + pt];
-    StrictLine<CT> w;
-    if (D == 0)
-        strict_line_begin<0>(a, e0, E, pt, w);
-    else if (D == 1)
-        strict_line_begin<1>(a, e0, E, pt, w);
-    else if (D == 2)
-        strict_line_begin<2>(a, e0, E, pt, w);
-    {
-        CT* A = area + wave * kAreaStride + swz64(pt);
-#pragma unroll
-        for (int v = 0; v < 5; ++v) A[v * 64] = (CT)s0[v];
-    }
-    coef_store<CT>((int)threadIdx.x, cf);
-    __syncthreads();
-    if (D < 3) {
-#pragma unroll
-        for (int v = 0; v < 5; ++v)
-#pragma unroll
-            for (int m = 0; m < 4; ++m) w.u[v][m] = area[w.pos[m] + v * 64];
-    }
-    __syncthreads();  // the gradients overwrite the states
-    if (D == 0)
-        strict_line_gradient<0>(a, area, w);
-    else if (D == 1)
-        strict_line_gradient<1>(a, area, w);
-    else if (D == 2)
-        strict_line_gradient<2>(a, area, w);
-    __syncthreads();
-    if (D == 0)
-        strict_line_flux<0>(a, area, e0, E, w);
-    else if (D == 1)
-        strict_line_flux<1>(a, area, e0, E, w);
-    else if (D == 2)
-        strict_line_flux<2>(a, area, e0, E, w);
-    CT g[15], st[5], r[5];
-    {
-        const CT* A = area + wave * kAreaStride + swz64(pt);
-#pragma unroll
-        for (int q = 0; q < 15; ++q) g[q] = A[q * 64];
-    }
-#pragma unroll
-    for (int v = 0; v < 5; ++v) st[v] = (CT)a.uin[v * NP + e * 64 + pt];  // again (from L2), not held all along
-    __syncthreads();  // the volume fluxes' lines are staged over the gradients
-    CT mu = a.sutherland ? sutherland(st, a.mu_ref, a.t_ref, a.s_suth) : a.mu;
-    if (a.mu_t) mu = mu + a.mu_t[e];
-    volume_rhs<true>(a, st, g, mu, (const CT*)nullptr, (CT(*)[64])(area + wave * kAreaStride), i, j, k, pt, r);
-    if (valid) {
-#pragma unroll
-        for (int v = 0; v < 5; ++v) a.fv[e * kFvStride + kFvFaces + v * 64 + pt] = r[v];
-    }
-}
-#endif
-
-#if OD_FAST
-// ---------------------------------------------------------------------------
-// Fast f32 build: the update kernel on blocks of 2x2x2 elements (512 threads; wave w owns local element w = lx + 2 ly +
-// 4 lz in the point-wise phases).  Three of an element's six faces face
-// another element of the block.  Their neighbour traces come from the
-// block's LDS state tiles instead of HBM, and the interface flux of such an
-// internal face is evaluated once for both of its elements.  Every value is
-// formed from the same operands in the same order as in update_body, so each
-// element gets the same bits as in the two-element-tile kernels (which take the
-// last layers of boxes with an odd dimension, and boxes 1 element wide).
-// ---------------------------------------------------------------------------
+// Blocks of 2x2x2 elements: local element lx + 2 ly + 4 lz.
 constexpr int kBlk = 8;
 
 struct Block {
@@ -1875,6 +1658,571 @@ __device__ __forceinline__ int blk_ext_nb(const StageArgs<UT, CT>& a, const Bloc
     return (s ? wall_r : wall_l) ? -1 : e + (s ? off_r : off_l);
 }
 
+// Left element of pair p (0..3) along direction D of a block; the right one is
+// 2^D further.
+template <int D>
+__device__ __forceinline__ int blk_pair(int p) {
+    return D == 0 ? 2 * p : (D == 1 ? ((p & 1) | ((p >> 1) << 2)) : p);
+}
+
+// The line waves are waves 0..5 or 2..7 of a work-group in turn, so that the
+// SIMDs of a CU get equally many of them.  Work-groups go round the XCDs, so
+// it is every eighth that turns.
+__device__ __forceinline__ int line_role(int group) { return (wave_index() + ((group >> 3) & 1) * 6) & 7; }
+
+// The value of the lane's partner, lane ^ 1.
+__device__ __forceinline__ float lane_partner(float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xF, 0xF, false));  // quad_perm [1,0,3,2]
+}
+__device__ __forceinline__ double lane_partner(double x) {
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(x), 0xB1, 0xF, 0xF, false),
+                            __builtin_amdgcn_mov_dpp(__double2loint(x), 0xB1, 0xF, 0xF, false));
+}
+
+#if !OD_FAST
+// ---------------------------------------------------------------------------
+// Strict build, one box: the visc kernel by lines.  A 256-thread work-group has
+// four consecutive elements; in the line phases wave d < 3 takes direction d,
+// lane = (element, line of four points), and forms from one read of the line's
+// states both end traces, both BR1 jumps and the corrected derivative at its
+// four points, then from one read of the line's gradients the viscous fluxes at
+// both ends.  The neighbours' traces come straight from memory, the operators
+// are wave-uniform.  The volume RHS is point-wise, a wave per element.  Every
+// value is the expression of visc_body, in the reference's order.
+// Bounds: instruction issue.  Against the point-wise form (visc_body, which the
+// batches' tiles use), whose lanes read each state 12 and each gradient 6 to 8
+// times from LDS: 24x26x22 f64 102 -> 61 us, 48^3 f32 279 -> 231 us, 24x20x28
+// f64 state with f32 fluxes 40 -> 33 us a launch.
+// LDS: one area per element, the states, then the gradients over them.
+// ---------------------------------------------------------------------------
+constexpr int kQuad = 4;
+
+template <class CT>
+struct StrictLine {
+    int e;            // element, -1: none
+    int fp, side;     // face point; blocks: the element's coordinate along D
+    CT u[5][4];
+    CT tl[5], tr[5];  // end traces in the order of the viscous fluxes
+    CT nl[5], nr[5];  // the neighbours' facing traces (blocks: nl, across the external face)
+    bool wl, wr;      // slip walls (blocks: wl, at the external face)
+    int pos[4];
+};
+
+// A block's line wave: half of the pairs of elements along D, lane = (pair,
+// line, side).  The neighbour across the internal face is the next lane.
+template <int D, class UT, class CT>
+__device__ __forceinline__ void strict_block_begin(const StageArgs<UT, CT>& a, const Block& b, int half, int lane,
+                                                   StrictLine<CT>& w) {
+    w.side = lane & 1;
+    w.fp = (lane >> 1) & 15;
+    const int le = blk_pair<D>(2 * half + (lane >> 5)) + (w.side << D);
+    w.e = blk_elem(a, b, le);
+    const int nb = blk_ext_nb(a, b, le, D);
+    w.wl = D == 1 && nb < 0;
+    const CT* t = a.tr_in + (int64_t)(w.wl ? w.e : nb) * kTraceStride + (2 * D + 1 - w.side) * 80 + w.fp;
+#pragma unroll
+    for (int v = 0; v < 5; ++v) w.nl[v] = t[v * 16];
+    int base, stride;
+    face_line(D, w.fp, base, stride);
+    const int s0 = swz64(base);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) w.pos[m] = le * kAreaStride + (s0 ^ line_xor<D>(m));
+}
+
+// Element e0's coordinates and the neighbours across both faces of direction D
+// of the lane's element e0 + le (those past the mesh's last one repeat it).
+template <int D, class UT, class CT>
+__device__ __forceinline__ void strict_line_begin(const StageArgs<UT, CT>& a, int e0, int E, int lane,
+                                                  StrictLine<CT>& w) {
+    const int le = lane >> 4;
+    w.e = e0 + le < E ? e0 + le : -1;
+    w.fp = lane & 15;
+    int ez = e0 / (a.nx * a.ny), ey = (e0 - ez * a.nx * a.ny) / a.nx, ex = e0 - a.nx * (ey + a.ny * ez);
+    int l[kQuad], r[kQuad];
+#pragma unroll
+    for (int q = 0; q < kQuad; ++q) {
+        const Elem n = make_elem(ex, ey, ez, a.nx, a.ny, a.nz, a.wall);
+        l[q] = D == 0 ? n.xl : (D == 1 ? n.yl : n.zl);
+        r[q] = D == 0 ? n.xr : (D == 1 ? n.yr : n.zr);
+        if (e0 + q + 1 < E) {
+            ++ex;
+            if (ex == a.nx) {
+                ex = 0;
+                ++ey;
+                if (ey == a.ny) {
+                    ey = 0;
+                    ++ez;
+                }
+            }
+        }
+    }
+    const bool b0 = le & 1, b1 = le & 2;
+    const int nl = b1 ? (b0 ? l[3] : l[2]) : (b0 ? l[1] : l[0]);
+    const int nr = b1 ? (b0 ? r[3] : r[2]) : (b0 ? r[1] : r[0]);
+    w.wl = D == 1 && nl < 0;
+    w.wr = D == 1 && nr < 0;
+    const CT* tl = a.tr_in + (int64_t)(w.wl ? 0 : nl) * kTraceStride + (2 * D + 1) * 80 + w.fp;
+    const CT* tr = a.tr_in + (int64_t)(w.wr ? 0 : nr) * kTraceStride + (2 * D) * 80 + w.fp;
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+        w.nl[v] = tl[v * 16];
+        w.nr[v] = tr[v * 16];
+    }
+    int base, stride;
+    face_line(D, w.fp, base, stride);
+    const int s0 = swz64(base);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) w.pos[m] = le * kAreaStride + (s0 ^ line_xor<D>(m));
+}
+
+// Jumps (br1_jumps) and corrected derivative along D (lane_gradient_faces) ->
+// the gradient's rows 3 v + D.
+template <int D, bool BLOCK, class UT, class CT>
+__device__ __forceinline__ void strict_line_gradient(const StageArgs<UT, CT>& a, CT* area, StrictLine<CT>& w) {
+    const Ops<CT>& o = dev_ops<CT>();
+    const CT jac = D == 0 ? a.jx : (D == 1 ? a.jy : a.jz);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+        const CT* u = w.u[v];
+        const CT tl = trace4(u, 0, 1, o.eL[0], o.eL[1], o.eL[2], o.eL[3], br1_order(D));
+        const CT tr = trace4(u, 0, 1, o.eR[0], o.eR[1], o.eR[2], o.eR[3], br1_order(D));
+        const CT sign = (v > 0 && v < 4) ? ((CT)-1.0) : ((CT)1.0);
+        CT nl, nr;
+        if constexpr (BLOCK) {
+            const CT in = lane_partner(w.side ? tl : tr);
+            const CT ext = w.wl ? (w.side ? tr : tl) * sign : w.nl[v];
+            nl = w.side ? in : ext;
+            nr = w.side ? ext : in;
+        } else {
+            nl = w.wl ? tl * sign : w.nl[v];
+            nr = w.wr ? tr * sign : w.nr[v];
+        }
+        const CT jl = ((CT)0.5) * (nl + tl) - tl, jr = ((CT)0.5) * (nr + tr) - tr;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            CT d = 0;
+#pragma unroll
+            for (int m = 0; m < 4; ++m) d += o.D[4 * i + m] * u[m];
+            CT g = d * jac;
+            g += jl * o.gL[i] * jac;
+            g += jr * o.gR[i] * jac;
+            if (a.round_q) g = (CT)(float)g;  // Q_REAL round trip (rhs.cu:457-461)
+            area[w.pos[i] + (3 * v + D) * 64] = g;
+        }
+        w.tl[v] = D == 0 ? trace4(u, 0, 1, o.eL[0], o.eL[1], o.eL[2], o.eL[3], fv_order(D)) : tl;
+        w.tr[v] = D == 0 ? trace4(u, 0, 1, o.eR[0], o.eR[1], o.eR[2], o.eR[3], fv_order(D)) : tr;
+        asm volatile("" : "+v"(w.tl[v]), "+v"(w.tr[v])::"memory");  // variable by variable (see lane_gradient_faces)
+    }
+}
+
+// Viscous flux at one end of the line (fv_value) from its state trace and
+// gradient trace -> the element's slot of face 2 D + side.
+template <int D, class UT, class CT>
+__device__ __forceinline__ void strict_end_flux(const StageArgs<UT, CT>& a, int64_t e, bool valid, const CT* st,
+                                                const CT* gt, int side, int fp) {
+    CT f[5];
+    CT mu = a.sutherland ? sutherland(st, a.mu_ref, a.t_ref, a.s_suth) : a.mu;
+    if (a.mu_t) mu = mu + a.mu_t[e];
+    viscous_flux(D, st, gt, mu, f);
+    if (valid)
+        *reinterpret_cast<FvQuad<CT>*>(a.fv + e * kFvStride + (2 * D + side) * 64 + fp * 4) =
+            FvQuad<CT>{{f[1], f[2], f[3], f[4]}};
+}
+template <int D, class UT, class CT>
+__device__ __forceinline__ void strict_line_flux(const StageArgs<UT, CT>& a, const CT* area, const StrictLine<CT>& w) {
+    const Ops<CT>& o = dev_ops<CT>();
+    CT gl[15], gr[15];
+#pragma unroll
+    for (int q = 0; q < 15; ++q) {
+        // what the flux along D reads: the density's gradient, the momenta's
+        // along D, across D of momentum D and on the diagonal, the energy's along D
+        const int v = q / 3, c = q % 3;
+        const bool used = v == 0 || c == D || (v < 4 && (v - 1 == D || v - 1 == c));
+        if (!used) {
+            gl[q] = gr[q] = (CT)0;
+            continue;
+        }
+        CT x[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) x[m] = area[w.pos[m] + q * 64];
+        gl[q] = trace4(x, 0, 1, o.eL[0], o.eL[1], o.eL[2], o.eL[3], fv_order(D));
+        gr[q] = trace4(x, 0, 1, o.eR[0], o.eR[1], o.eR[2], o.eR[3], fv_order(D));
+        asm volatile("" : "+v"(gl[q]), "+v"(gr[q])::"memory");
+    }
+    const bool valid = w.e >= 0;
+    const int64_t e = valid ? w.e : 0;
+    strict_end_flux<D>(a, e, valid, w.tl, gl, 0, w.fp);
+    asm volatile("" ::: "memory");  // one end, then the other
+    strict_end_flux<D>(a, e, valid, w.tr, gr, 1, w.fp);
+}
+
+// BLOCK: the elements of block b, else the N consecutive ones from e0.
+// D, half: this wave's direction (3: none) and half of the pairs along it.
+template <bool BLOCK, class UT, class CT>
+__device__ __forceinline__ void strict_visc_body(const StageArgs<UT, CT>& a, const Block& b, int e0, CT* area, int D,
+                                                 int half) {
+    const int wave = wave_index(), pt = threadIdx.x & 63;
+    const int i = pt & 3, j = (pt >> 2) & 3, k = pt >> 4;
+    const int E = a.nx * a.ny * a.nz;
+    const int64_t NP = (int64_t)E * 64;
+    const bool valid = BLOCK || e0 + wave < E;
+    const int64_t e = BLOCK ? blk_elem(a, b, wave) : (valid ? e0 + wave : E - 1);
+    const CT cf = coef_load<CT>((int)threadIdx.x);
+    UT s0[5];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) s0[v] = a.uin[v * NP + e * 64 + pt];
+    StrictLine<CT> w;
+    if constexpr (BLOCK) {
+        if (D == 0)
+            strict_block_begin<0>(a, b, half, pt, w);
+        else if (D == 1)
+            strict_block_begin<1>(a, b, half, pt, w);
+        else if (D == 2)
+            strict_block_begin<2>(a, b, half, pt, w);
+    } else {
+        if (D == 0)
+            strict_line_begin<0>(a, e0, E, pt, w);
+        else if (D == 1)
+            strict_line_begin<1>(a, e0, E, pt, w);
+        else if (D == 2)
+            strict_line_begin<2>(a, e0, E, pt, w);
+    }
+    {
+        CT* A = area + wave * kAreaStride + swz64(pt);
+#pragma unroll
+        for (int v = 0; v < 5; ++v) A[v * 64] = (CT)s0[v];
+    }
+    coef_store<CT>((int)threadIdx.x, cf);
+    __syncthreads();
+    if (D < 3) {
+#pragma unroll
+        for (int v = 0; v < 5; ++v)
+#pragma unroll
+            for (int m = 0; m < 4; ++m) w.u[v][m] = area[w.pos[m] + v * 64];
+    }
+    __syncthreads();  // the gradients overwrite the states
+    if (D == 0)
+        strict_line_gradient<0, BLOCK>(a, area, w);
+    else if (D == 1)
+        strict_line_gradient<1, BLOCK>(a, area, w);
+    else if (D == 2)
+        strict_line_gradient<2, BLOCK>(a, area, w);
+    __syncthreads();
+    if (D == 0)
+        strict_line_flux<0>(a, area, w);
+    else if (D == 1)
+        strict_line_flux<1>(a, area, w);
+    else if (D == 2)
+        strict_line_flux<2>(a, area, w);
+    CT g[15], st[5], r[5];
+    {
+        const CT* A = area + wave * kAreaStride + swz64(pt);
+#pragma unroll
+        for (int q = 0; q < 15; ++q) g[q] = A[q * 64];
+    }
+#pragma unroll
+    for (int v = 0; v < 5; ++v) st[v] = (CT)a.uin[v * NP + e * 64 + pt];  // again (from L2), not held all along
+    __syncthreads();  // the volume fluxes' lines are staged over the gradients
+    CT mu = a.sutherland ? sutherland(st, a.mu_ref, a.t_ref, a.s_suth) : a.mu;
+    if (a.mu_t) mu = mu + a.mu_t[e];
+    volume_rhs<true>(a, st, g, mu, (const CT*)nullptr, (CT(*)[64])(area + wave * kAreaStride), i, j, k, pt, r);
+    if (valid) {
+#pragma unroll
+        for (int v = 0; v < 5; ++v) a.fv[e * kFvStride + kFvFaces + v * 64 + pt] = r[v];
+    }
+}
+
+template <class UT, class CT>
+__global__ __launch_bounds__(64 * kQuad) void od_visc_line_kernel(StageArgs<UT, CT> a) {
+    __shared__ CT area[kQuad * kAreaStride];
+    // wave -> direction (3: none), turning from work-group to work-group of an
+    // XCD so that the SIMDs get equally many line waves
+    const int D = (wave_index() + ((int)blockIdx.x >> 3)) & 3;
+    strict_visc_body<false>(a, Block{}, kQuad * (int)blockIdx.x, area, D, 0);
+}
+
+// Waves per SIMD asked of the strict block kernels: three work-groups to a CU
+// with f32 compute (78 and 70 VGPRs; held to 64 they spill), two with f64 (124
+// and 128).
+template <class CT>
+constexpr int kMinWavesBlock = sizeof(CT) == 4 ? 6 : 4;
+
+// The same by blocks, for boxes whose update runs on blocks: the traces across
+// internal faces come from the next lane, so the update kernel need not write
+// them.  As fast as by fours (24x26x22 f64 61 us both; 48^3 f32 237 against
+// 234 us, VALU bound).
+template <class UT, class CT>
+__global__ __launch_bounds__(64 * kBlk) __attribute__((amdgpu_waves_per_eu(kMinWavesBlock<CT>))) void od_visc_lines_block_kernel(StageArgs<UT, CT> a) {
+    __shared__ CT area[kBlk * kAreaStride];
+    const int group = (int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
+    const int role = line_role(group), half = role / 3;
+    strict_visc_body<true>(a, make_block<false>(a), 0, area, role < 6 ? role - 3 * half : 3, half);
+}
+
+// ---------------------------------------------------------------------------
+// Strict build, one box: the update kernel on 2x2x2 blocks (wave w owns local
+// element w in the point-wise phases).  Bounds: f32 memory, f64 the chain of
+// the interface fluxes at 16 waves per CU.  Of an element's six faces three face
+// another element of the block: their traces come from the block's LDS states,
+// their flux is evaluated once for both elements (9 wave passes for 8 elements
+// instead of 12), both elements' viscous fluxes are read once, and their traces
+// of the new state are not written: 2309 values moved per element instead of
+// 3061.  Per launch against the two-element tiles: 48^3 f32 211 -> 172 us,
+// 24x26x22 f64 57.8 -> 49 us, 24x20x28 f64 state with f32 fluxes 40.9 -> 34 us.
+// Every value is the expression of update_body.
+// LDS: states in swz64 order; lanes go (pair, side, face point), so a half-wave
+// reads the two elements of a pair, 4, 8 or 16 banks apart as in BlockViscLds.
+// ---------------------------------------------------------------------------
+constexpr int kStateStride = 5 * 64 + 4;  // as kAreaStride
+template <class CT>
+struct FaceBlockLds {
+    CT sJe[kBlk][3][5][16];  // corrections j at the external faces
+    CT sJi[kBlk][3][5][16];  // and at the internal ones
+    CT sU[kBlk * kStateStride];
+};
+
+// Whether a face lane reads the viscous fluxes only after the interface flux:
+// in f64, and beside an f64 state, they cost registers over it (24x26x22 f64:
+// 14 to 70 spilled, 58 us, none and 49 us); all in f32 they fit and their
+// latency is covered (48^3 172 against 181 us).
+template <class UT, class CT>
+constexpr bool kLateFv = sizeof(UT) == 8 || sizeof(CT) == 8;
+template <class CT>
+__device__ __forceinline__ const FvQuad<CT>& fv_quad(const CT* fv, int64_t e, int f, int fp) {
+    return *reinterpret_cast<const FvQuad<CT>*>(fv + e * kFvStride + f * 64 + fp * 4);
+}
+// Element of an external face lane: lane = (pair, side, face point).
+template <int D>
+__device__ __forceinline__ int ext_elem(int half, int lane) {
+    return blk_pair<D>(2 * half + (lane >> 5)) + (((lane >> 4) & 1) << D);
+}
+// The neighbour's trace at an external face (its own at a slip wall, unused).
+template <int D, class UT, class CT>
+__device__ __forceinline__ void ext_face_load(const StageArgs<UT, CT>& a, const Block& b, int half, int lane, CT* far) {
+    const int le = ext_elem<D>(half, lane), side = (lane >> 4) & 1, fp = lane & 15;
+    const int nb = blk_ext_nb(a, b, le, D);
+    const int64_t src = nb < 0 ? blk_elem(a, b, le) : nb;
+    const int rf = D == 0 ? 7 - side : 2 * D + 1 - side;
+#pragma unroll
+    for (int v = 0; v < 5; ++v) far[v] = stream_load(&a.tr_in[src * kTraceStride + rf * 80 + v * 16 + fp]);
+}
+// Trace of local element le at the left or right end of the line of face point fp.
+template <int D, class CT>
+__device__ __forceinline__ void block_trace(const CT* sU, int le, int fp, bool right, CT* t) {
+    int base, stride;
+    face_line(D, fp, base, stride);
+    const int q = swz64(base);
+    const CT* row = sU + le * kStateStride;
+    const Coef4<CT> c = side_coef<CT>(right);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+        CT x[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) x[m] = row[v * 64 + (q ^ line_xor<D>(m))];
+        t[v] = trace4(x, 0, 1, c.c0, c.c1, c.c2, c.c3, face_order(D));
+    }
+}
+// External faces of direction D of half a block: flux_pass, a face point per lane.
+template <int D, class UT, class CT>
+__device__ __forceinline__ void ext_face(const StageArgs<UT, CT>& a, const Block& b, FaceBlockLds<CT>& L, int half,
+                                         int lane, const CT* far) {
+    const int le = ext_elem<D>(half, lane), side = (lane >> 4) & 1, fp = lane & 15;
+    const bool right = side;
+    const int e = blk_elem(a, b, le), nb = blk_ext_nb(a, b, le, D);
+    const bool wall = D == 1 && nb < 0;
+    FvQuad<CT> fo, fn;
+    const auto load_fv = [&] {
+        fo = fv_quad(a.fv, e, 2 * D + side, fp);
+        fn = fv_quad(a.fv, wall ? e : nb, 2 * D + 1 - side, fp);
+    };
+    if constexpr (!kLateFv<UT, CT>) load_fv();
+    CT own[5], Lq[5], Rq[5], fvo[5], fvn[5], fr[5], jv[5];
+    block_trace<D>(L.sU, le, fp, right, own);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+        const CT oth = wall ? own[v] : far[v];
+        Lq[v] = right ? own[v] : oth;
+        Rq[v] = right ? oth : own[v];
+    }
+    interface_flux<D>(a.flux, Lq, Rq, fr);
+    if constexpr (kLateFv<UT, CT>) {
+        asm volatile("" : "+v"(fr[0]), "+v"(fr[1]), "+v"(fr[2]), "+v"(fr[3]), "+v"(fr[4])::"memory");
+        load_fv();
+    }
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+        fvo[v] = v ? fo.c[v - 1] : (CT)0;
+        fvn[v] = v ? fn.c[v - 1] : (CT)0;
+    }
+    face_correction<D, true>(fr, own, fvo, fvn, wall, right, jv);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) L.sJe[le][D][v][fp] = jv[v];
+}
+// Internal faces of direction D: lane = (pair, face point), one flux, each
+// side's correction as flux_pass forms it.
+template <int D, class UT, class CT>
+__device__ __forceinline__ void int_face(const StageArgs<UT, CT>& a, const Block& b, FaceBlockLds<CT>& L, int lane) {
+    const int lL = blk_pair<D>(lane >> 4), lR = lL + (1 << D), fp = lane & 15;
+    FvQuad<CT> fl, fn;
+    const auto load_fv = [&] {
+        fl = fv_quad(a.fv, blk_elem(a, b, lL), 2 * D + 1, fp);
+        fn = fv_quad(a.fv, blk_elem(a, b, lR), 2 * D, fp);
+    };
+    if constexpr (!kLateFv<UT, CT>) load_fv();
+    CT tl[5], tr[5], fvl[5], fvr[5], fr[5], jv[5];
+    block_trace<D>(L.sU, lL, fp, true, tl);
+    block_trace<D>(L.sU, lR, fp, false, tr);
+    interface_flux<D>(a.flux, tl, tr, fr);
+    if constexpr (kLateFv<UT, CT>) {
+        asm volatile("" : "+v"(fr[0]), "+v"(fr[1]), "+v"(fr[2]), "+v"(fr[3]), "+v"(fr[4])::"memory");
+        load_fv();
+    }
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+        fvl[v] = v ? fl.c[v - 1] : (CT)0;
+        fvr[v] = v ? fn.c[v - 1] : (CT)0;
+    }
+    face_correction<D, true>(fr, tl, fvl, fvr, false, true, jv);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) L.sJi[lL][D][v][fp] = jv[v];
+    face_correction<D, true>(fr, tr, fvr, fvl, false, false, jv);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) L.sJi[lR][D][v][fp] = jv[v];
+}
+
+template <class UT, class CT>
+__device__ __forceinline__ void face_block_body(const StageArgs<UT, CT>& a, const Block& b, FaceBlockLds<CT>& L,
+                                                int role) {
+    constexpr bool SAME = std::is_same<UT, CT>::value;
+    const int wave = wave_index(), pt = threadIdx.x & 63;
+    const int i = pt & 3, j = (pt >> 2) & 3, k = pt >> 4;
+    const int64_t NP = (int64_t)a.nx * a.ny * a.nz * 64;
+    const int64_t e = blk_elem(a, b, wave);
+    const int64_t gbase = e * 64 + pt;
+    const CT cf = coef_load<CT>((int)threadIdx.x);
+    UT s0[5];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) s0[v] = a.uin[v * NP + gbase];
+    CT far[5];
+    switch (role) {
+        case 0: ext_face_load<0>(a, b, 0, pt, far); break;
+        case 1: ext_face_load<0>(a, b, 1, pt, far); break;
+        case 2: ext_face_load<1>(a, b, 0, pt, far); break;
+        case 3: ext_face_load<1>(a, b, 1, pt, far); break;
+        case 4: ext_face_load<2>(a, b, 0, pt, far); break;
+        case 5: ext_face_load<2>(a, b, 1, pt, far); break;
+        default: break;
+    }
+    CT* own = L.sU + wave * kStateStride + swz64(pt);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) own[v * 64] = (CT)s0[v];
+    coef_store<CT>((int)threadIdx.x, cf);
+    __syncthreads();
+    // 6 external passes (4 elements x 16 points) and 3 internal ones (4 pairs x
+    // 16 points), 9 over 8 waves
+    switch (role) {
+        case 0:
+            ext_face<0>(a, b, L, 0, pt, far);
+            int_face<2>(a, b, L, pt);
+            break;
+        case 1: ext_face<0>(a, b, L, 1, pt, far); break;
+        case 2: ext_face<1>(a, b, L, 0, pt, far); break;
+        case 3: ext_face<1>(a, b, L, 1, pt, far); break;
+        case 4: ext_face<2>(a, b, L, 0, pt, far); break;
+        case 5: ext_face<2>(a, b, L, 1, pt, far); break;
+        case 6: int_face<0>(a, b, L, pt); break;
+        default: int_face<1>(a, b, L, pt); break;
+    }
+    // the volume RHS and u^n (stage 1: the state), before the barrier's wait
+    UT uprv[5], ucr[5];
+    CT r[5], rts[5];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+        ucr[v] = SAME ? (UT)own[v * 64] : a.uin[v * NP + gbase];
+        r[v] = stream_load(&a.fv[e * kFvStride + kFvFaces + v * 64 + pt]);
+    }
+    if (a.stage1) {
+#pragma unroll
+        for (int v = 0; v < 5; ++v) uprv[v] = ucr[v];
+    } else {
+#pragma unroll
+        for (int v = 0; v < 5; ++v) uprv[v] = stream_load(&a.uprev[v * NP + gbase]);
+    }
+    const StageDt<UT, CT> cdt = stage_dt(a);
+    __syncthreads();
+
+    const CoefTable<CT>& o = coef_lds<CT>();
+    const CT gLi = o.g[i][0], gRi = o.g[i][1];
+    const CT gLj = o.g[j][0], gRj = o.g[j][1];
+    const CT gLk = o.g[k][0], gRk = o.g[k][1];
+    const int fpx = j + 4 * k, fpy = i + 4 * k, fpz = i + 4 * j;
+    const CT* Je = &L.sJe[wave][0][0][0];
+    const CT* Ji = &L.sJi[wave][0][0][0];
+    const int lx = wave & 1, ly = (wave >> 1) & 1, lz = wave >> 2;
+    const CT *Jx0 = lx ? Ji : Je, *Jx1 = lx ? Je : Ji;
+    const CT *Jy0 = (ly ? Ji : Je) + 80, *Jy1 = (ly ? Je : Ji) + 80;
+    const CT *Jz0 = (lz ? Ji : Je) + 160, *Jz1 = (lz ? Je : Ji) + 160;
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+        CT cx = -(Jx0[v * 16 + fpx] * gLi * a.jx) - (Jx1[v * 16 + fpx] * gRi * a.jx);
+        CT cy = -(Jy0[v * 16 + fpy] * gLj * a.jy) - (Jy1[v * 16 + fpy] * gRj * a.jy);
+        CT cz = -(Jz0[v * 16 + fpz] * gLk * a.jz) - (Jz1[v * 16 + fpz] * gRk * a.jz);
+        rts[v] = r[v] + (cx + cy + cz);
+    }
+    if (a.mode == 1) {  // the stage's RHS into dbg, state unchanged
+#pragma unroll
+        for (int v = 0; v < 5; ++v) a.dbg[v * NP + gbase] = rts[v];
+        return;
+    }
+    UT unew[5];
+    rk_stage(a, cdt, uprv, ucr, rts, unew);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+        stream_store(unew[v], &a.uout[v * NP + gbase]);
+        own[v * 64] = (CT)unew[v];
+    }
+    wave_sync();
+
+    // Traces of the new state on the element's external faces (x in both
+    // orders), 16 lanes each; only they are read (the internal ones come from
+    // the blocks' LDS tiles).
+    const int g = pt >> 4, fp = pt & 15, d = g == 3 ? 0 : g;
+    const int tf = 2 * g + blk_bit(wave, d);
+    int base, stride;
+    face_line(d, fp, base, stride);
+    const int q = swz64(base);
+    const int x1 = d == 0 ? line_xor<0>(1) : (d == 1 ? line_xor<1>(1) : line_xor<2>(1));
+    const int x2 = d == 0 ? line_xor<0>(2) : (d == 1 ? line_xor<1>(2) : line_xor<2>(2));
+    const Coef4<CT> c = side_coef<CT>(tf & 1);
+    const int order = trace_face_order(tf);
+    CT* dst = a.tr_out + e * kTraceStride + tf * 80 + fp;
+    const CT* row = L.sU + wave * kStateStride;
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+        const CT x[4] = {row[v * 64 + q], row[v * 64 + (q ^ x1)], row[v * 64 + (q ^ x2)], row[v * 64 + (q ^ x1 ^ x2)]};
+        stream_store(trace4(x, 0, 1, c.c0, c.c1, c.c2, c.c3, order), &dst[v * 16]);
+    }
+}
+
+template <class UT, class CT>
+__global__ __launch_bounds__(64 * kBlk) __attribute__((amdgpu_waves_per_eu(kMinWavesBlock<CT>))) void od_update_face_block_kernel(StageArgs<UT, CT> a) {
+    __shared__ FaceBlockLds<CT> L;
+    const int group = (int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
+    face_block_body(a, make_block<true>(a), L, (wave_index() + (group >> 3)) & 7);
+}
+#endif
+
+#if OD_FAST
+// ---------------------------------------------------------------------------
+// Fast f32 build: the update kernel on blocks of 2x2x2 elements (512 threads; wave w owns local element w = lx + 2 ly +
+// 4 lz in the point-wise phases).  Three of an element's six faces face
+// another element of the block.  Their neighbour traces come from the
+// block's LDS state tiles instead of HBM, and the interface flux of such an
+// internal face is evaluated once for both of its elements.  Every value is
+// formed from the same operands in the same order as in update_body, so each
+// element gets the same bits as in the two-element-tile kernels (which take the
+// last layers of boxes with an odd dimension, and boxes 1 element wide).
+// ---------------------------------------------------------------------------
 // Source of 16-byte chunk `chunk` (0..59) of the external-face traces of
 // local element le, as the LDS prefetch lays them out ([d][5][16]): the
 // neighbour's facing trace (its own at a slip wall, where it is not used).
@@ -1979,7 +2327,7 @@ template <int D, bool VISC>
 __device__ __forceinline__ void blk_int_pass(const StageArgs<float, float>& a, const Block& b, BlockUpdateLds& L,
                                              int lane) {
     const int p = lane >> 4, fp = lane & 15;
-    const int lL = D == 0 ? 2 * p : (D == 1 ? ((p & 1) | ((p >> 1) << 2)) : p);
+    const int lL = blk_pair<D>(p);
     const int lR = lL + (1 << D);
     int base, stride;
     face_line(D, fp, base, stride);
@@ -2195,10 +2543,6 @@ struct BlockViscLds {
     __device__ float* of(int le) { return area + le * kAreaStride; }
 };
 
-// The value of the lane's partner, lane ^ 1.
-__device__ __forceinline__ float lane_partner(float x) {
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xF, 0xF, false));  // quad_perm [1,0,3,2]
-}
 // End trace sum_m q[m] l_m(+-1) in the BR1 order (the right end's coefficients
 // are the left one's backwards).
 __device__ __forceinline__ float line_trace(const float* q, const float* c) {
@@ -2220,7 +2564,7 @@ __device__ __forceinline__ void line_begin(const StageArgs<float, float>& a, con
     w.side = lane & 1;
     w.fp = (lane >> 1) & 15;
     const int p = 2 * half + (lane >> 5);  // pair of elements along D
-    w.le = (D == 0 ? 2 * p : (D == 1 ? ((p & 1) | ((p >> 1) << 2)) : p)) + (w.side << D);
+    w.le = blk_pair<D>(p) + (w.side << D);
     const int nb = blk_ext_nb(a, b, w.le, D);
     const int src = nb >= 0 ? nb : blk_elem(a, b, w.le);  // at a slip wall its own, unused
     const float* t = a.tr_in + (int64_t)src * kTraceStride + (2 * D + 1 - w.side) * 80 + w.fp;
@@ -2366,11 +2710,6 @@ __device__ __forceinline__ void visc_block_body(const StageArgs<float, float>& a
     __syncthreads();  // the volume fluxes' lines are staged over the gradients
     visc_divergence(a, e, st, g, L.of(wave), i, j, k, pt);
 }
-
-// The line waves are waves 0..5 or 2..7 of a work-group in turn, so that the
-// SIMDs of a CU get equally many of them.  Work-groups go round the XCDs, so
-// it is every eighth that turns.
-__device__ __forceinline__ int line_role(int group) { return (wave_index() + ((group >> 3) & 1) * 6) & 7; }
 
 // One box: the update kernel walks the blocks backwards, the visc kernel
 // forwards (make_block).
@@ -2793,6 +3132,23 @@ int launch_trace(const StageArgs<UT, CT>& a, int64_t n_elem, void* stream) {
 }
 
 template <class UT, class CT>
+dim3 block_grid(const StageArgs<UT, CT>& a) {
+    return dim3((unsigned)(a.nx / 2), (unsigned)(a.ny / 2), (unsigned)(a.nz / 2));
+}
+
+#if !OD_FAST
+template <class UT, class CT>
+int launch_strict_block(const StageArgs<UT, CT>& a, int kind, void* stream) {
+    if (a.nx % 2 || a.ny % 2 || a.nz % 2) return 1;  // blocks of 2x2x2 elements tile the box exactly
+    if (kind == 0)
+        hipLaunchKernelGGL((od_visc_lines_block_kernel<UT, CT>), block_grid(a), dim3(64 * kBlk), 0, (hipStream_t)stream, a);
+    else
+        hipLaunchKernelGGL((od_update_face_block_kernel<UT, CT>), block_grid(a), dim3(64 * kBlk), 0, (hipStream_t)stream, a);
+    return check_launch();
+}
+#endif
+
+template <class UT, class CT>
 int launch_visc(const StageArgs<UT, CT>& a, int64_t n_elem, void* stream) {
 #if OD_FAST
     hipLaunchKernelGGL((od_visc_kernel<UT, CT>), grid_of(a), dim3(64 * kEpb), 0, (hipStream_t)stream, a);
@@ -2810,10 +3166,6 @@ int launch_update(const StageArgs<UT, CT>& a, int64_t n_elem, void* stream) {
 }
 
 #if OD_FAST
-inline dim3 block_grid(const StageArgs<float, float>& a) {
-    return dim3((unsigned)(a.nx / 2), (unsigned)(a.ny / 2), (unsigned)(a.nz / 2));
-}
-
 template <bool VISC>
 int launch_update_block(const StageArgs<float, float>& a, void* stream) {
     if (a.nx % 2 || a.ny % 2 || a.nz % 2) return 1;  // blocks of 2x2x2 elements tile the box exactly
@@ -2961,14 +3313,6 @@ int launch_cfl(const UT* u, double* partial, int64_t n_elem, double dx, double d
     return check_launch();
 }
 
-const char* kernel_name(int kind) {
-    switch (kind) {
-        case 0: return "od_visc_kernel";
-        case 1: return "od_update_kernel";
-        case 2: return "od_trace_kernel";
-        default: return "?";
-    }
-}
 #endif
 
 #define OD_INST(UT, CT)                                                                                      \
@@ -2990,6 +3334,10 @@ OD_INST(float, double)
 #endif
 #undef OD_INST
 #if !OD_FAST
+template int launch_strict_block<float, float>(const StageArgs<float, float>&, int, void*);
+template int launch_strict_block<double, float>(const StageArgs<double, float>&, int, void*);
+template int launch_strict_block<double, double>(const StageArgs<double, double>&, int, void*);
+template int launch_strict_block<float, double>(const StageArgs<float, double>&, int, void*);
 template int launch_set_dt<float, float>(StageDt<float, float>*, const StageDt<float, float>*, double*, double, void*);
 template int launch_set_dt<double, float>(StageDt<double, float>*, const StageDt<double, float>*, double*, double, void*);
 template int launch_set_dt<double, double>(StageDt<double, double>*, const StageDt<double, double>*, double*, double, void*);
