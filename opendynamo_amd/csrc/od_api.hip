@@ -143,6 +143,7 @@ template <class UT, class CT>
 od::StageArgs<UT, CT> stage_args(od_ctx* c, int stage, double dt) {
     od::StageArgs<UT, CT> a = make_stage_args<UT, CT>(c->p, c->p.nx, c->p.ny, c->p.nz, c->p.lx, c->p.ly, c->p.lz,
                                                       c->u, c->tr, c->fv, c->dbg, stage, dt);
+    a.ops = c->box_ops;
     a.mu_t = c->mu_t_on ? (const CT*)c->mu_t : nullptr;
     // a captured step (dt 0) reads c * dt from the context's table
     if (dt == kTableDt) a.dt = (const od::StageDt<UT, CT>*)c->dt_table + stage;
@@ -398,16 +399,22 @@ od_status od_create(const od_params* p, int device, od_ctx** out) {
     for (int q = 0; q < 3 && ok; ++q) ok = dmalloc(&c->tr[q], tr_bytes);
     ok = ok && (!p->viscous || dmalloc(&c->fv, fv_bytes));
     // the small arrays share the partial sums' allocation
-    static_assert(sizeof(od::StageDt<double, double>) % sizeof(double) == 0, "table of doubles");
+    static_assert(sizeof(od::StageDt<double, double>) % sizeof(double) == 0 && sizeof(od::BoxOps) % sizeof(double) == 0,
+                  "tables of doubles");
+    const size_t ops_doubles = sizeof(od::BoxOps) / sizeof(double);
     const size_t dt_doubles = 3 * sizeof(od::StageDt<double, double>) / sizeof(double) + 1;
-    ok = ok && dmalloc((void**)&c->sums_partial, ((size_t)5 * E + 8 + od::kCflGroups + dt_doubles) * sizeof(double));
+    ok = ok && dmalloc((void**)&c->sums_partial, ((size_t)5 * E + 8 + od::kCflGroups + dt_doubles + ops_doubles) * sizeof(double));
     if (ok) {
         c->sums_out = c->sums_partial + (size_t)5 * E;
         c->cfl_partial = c->sums_out + 8;
         c->dt_value = c->cfl_partial + od::kCflGroups;
         c->dt_table = c->dt_value + 1;
+        c->box_ops = (od::BoxOps*)(c->dt_value + dt_doubles);
     }
     if (!ok) return cleanup(fail(OD_ERR_NOMEM, "device allocation failed"));
+    const od::BoxOps ops = box_ops(c->ops, p->lx, p->nx, p->ly, p->ny, p->lz, p->nz);
+    if (hipMemcpy(c->box_ops, &ops, sizeof(ops), hipMemcpyHostToDevice) != hipSuccess)
+        return cleanup(fail(OD_ERR_HIP, "copying the box's operators to the device failed"));
     for (int q = 0; q < 3; ++q)
         if (hipHostMalloc(&c->pinned[q], state_bytes, hipHostMallocDefault) != hipSuccess ||
             hipEventCreateWithFlags(&c->slot_done[q], hipEventDisableTiming) != hipSuccess)

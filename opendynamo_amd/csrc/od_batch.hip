@@ -38,6 +38,7 @@ struct od_batch {
     double* sums_out = nullptr;      // 8 doubles
     double* cfl_partial = nullptr;   // od::kCflGroups doubles
     HostOps ops;
+    od::BoxOps* box_ops = nullptr;  // per box: the fast kernels' operators
     std::vector<char> state_set;
     od_schedule sched{0, 1, 0, 0};
     std::vector<double> table_dt;  // the dt values the device table holds
@@ -83,7 +84,10 @@ od::StageArgs<UT, CT> box_args(od_batch* b, int i, int stage, double dt) {
                    (CT*)b->tr[2] + eo * od::kTraceStride};
     void* fv = b->fv ? (void*)((CT*)b->fv + eo * od::fv_stride(fast_kernels(b->p))) : nullptr;
     const od_box& x = b->boxes[i];
-    return make_stage_args<UT, CT>(b->p, x.nx, x.ny, x.nz, x.lx, x.ly, x.lz, u, tr, fv, nullptr, stage, dt);
+    od::StageArgs<UT, CT> a =
+        make_stage_args<UT, CT>(b->p, x.nx, x.ny, x.nz, x.lx, x.ly, x.lz, u, tr, fv, nullptr, stage, dt);
+    a.ops = b->box_ops + i;
+    return a;
 }
 
 // kind: 0 = visc, 1 = update, 2 = trace of u0 into tr[0]
@@ -188,6 +192,7 @@ template <class UT, class CT>
 int batch_launch_t(od_batch* b, int kind, int stage) {
     od::StageArgs<UT, CT> a = make_stage_args<UT, CT>(b->p, 1, 1, 1, 1.0, 1.0, 1.0, b->u, b->tr, b->fv, nullptr,
                                                       stage, 0.0);
+    a.ops = b->box_ops;
     const od_schedule& s = b->sched;
     od::BatchArgs<UT, CT> ba{};
     ba.boxes = (const od::BoxDev<UT, CT>*)b->table;
@@ -227,6 +232,7 @@ int batch_launch_t(od_batch* b, int kind, int stage) {
 int block_launch(od_batch* b, int kind, int stage) {
     od::StageArgs<float, float> a = make_stage_args<float, float>(b->p, 1, 1, 1, 1.0, 1.0, 1.0, b->u, b->tr, b->fv,
                                                                   nullptr, stage, 0.0);
+    a.ops = b->box_ops;
     od::BlockBatch bb{};
     bb.boxes = (const od::BoxDev<float, float>*)b->table;
     bb.n_boxes = (int32_t)b->boxes.size();
@@ -434,12 +440,20 @@ od_status od_batch_create(const od_params* p, const od_box* boxes, int32_t n_box
     ok = ok && (!p->viscous || dmalloc(&b->fv, (size_t)E * od::fv_stride(fast_kernels(*p)) * b->cbytes));
     b->table_bytes = (size_t)n_boxes * sizeof(od::BoxDev<double, double>);
     ok = ok && dmalloc(&b->table, b->table_bytes);
-    ok = ok && dmalloc((void**)&b->sums_partial, ((size_t)5 * max_box + 8 + od::kCflGroups) * sizeof(double));
+    const size_t ops_doubles = (size_t)n_boxes * sizeof(od::BoxOps) / sizeof(double);
+    ok = ok && dmalloc((void**)&b->sums_partial,
+                       ((size_t)5 * max_box + 8 + od::kCflGroups + ops_doubles) * sizeof(double));
     if (ok) {
         b->sums_out = b->sums_partial + (size_t)5 * max_box;
         b->cfl_partial = b->sums_out + 8;
+        b->box_ops = (od::BoxOps*)(b->cfl_partial + od::kCflGroups);
     }
     if (!ok) return cleanup(fail(OD_ERR_NOMEM, "device allocation failed"));
+    std::vector<od::BoxOps> ops;
+    for (int i = 0; i < n_boxes; ++i)
+        ops.push_back(box_ops(b->ops, boxes[i].lx, boxes[i].nx, boxes[i].ly, boxes[i].ny, boxes[i].lz, boxes[i].nz));
+    if (hipMemcpy(b->box_ops, ops.data(), ops.size() * sizeof(ops[0]), hipMemcpyHostToDevice) != hipSuccess)
+        return cleanup(fail(OD_ERR_HIP, "copying the boxes' operators to the device failed"));
     *out = b;
     return OD_OK;
 }

@@ -38,6 +38,7 @@ struct od_ctx {
     hipGraphExec_t graph_k = nullptr;  // kStepsPerGraph RK3 steps
     hipGraphExec_t graph_c = nullptr;  // closure: a refresh of mu_t and one interval's steps
     double* dt_value = nullptr;        // dt on the device, and behind it
+    od::BoxOps* box_ops = nullptr;     // the fast kernels' operators
     void* dt_table = nullptr;          // StageDt[3] that the graphs' kernels read
     double table_dt = 0.0;             // the dt it holds (in stream order), 0: none yet
     void* pinned[3] = {nullptr, nullptr, nullptr};

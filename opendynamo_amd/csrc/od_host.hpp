@@ -90,6 +90,28 @@ template <class CT>
 CT jacobian(double l, int n) {  // jac = 2 / (L / n) in the compute type (rhs.cu:366-369; rk.cu:93-95)
     return ((CT)2.0) / (((CT)l) / ((CT)n));
 }
+inline od::BoxOps box_ops(const HostOps& h, double lx, int nx, double ly, int ny, double lz, int nz) {
+    od::BoxOps o{};
+    const double jac[3] = {jacobian<float>(lx, nx), jacobian<float>(ly, ny), jacobian<float>(lz, nz)};
+    for (int d = 0; d < 3; ++d) {
+        for (int q = 0; q < 16; ++q) o.table[16 * d + q] = (float)(jac[d] * h.D[q]);
+        for (int q = 0; q < 4; ++q) {
+            o.table[48 + 8 * d + 2 * q] = (float)(jac[d] * h.gL[q]);
+            o.table[48 + 8 * d + 2 * q + 1] = (float)(jac[d] * h.gR[q]);
+        }
+        for (int i = 0; i < 2; ++i) {
+            const double* D = h.D + 4 * i;
+            o.line[d][i] = {(float)(jac[d] * 0.25 * ((D[0] + D[3]) - (D[1] + D[2]))),
+                            (float)(jac[d] * 0.25 * (h.gL[i] + h.gR[i])), (float)(jac[d] * 0.5 * (D[0] - D[3])),
+                            (float)(jac[d] * 0.5 * (D[1] - D[2])), (float)(jac[d] * 0.25 * (h.gL[i] - h.gR[i]))};
+        }
+    }
+    for (int q = 0; q < 4; ++q) {
+        o.table[72 + q] = (float)h.eL[q];
+        o.table[76 + q] = (float)h.eR[q];
+    }
+    return o;
+}
 template <class T>
 T stage_dt_coef(int stage, double dt) {  // c * dt in type T from the f32 dt (solver.rs:256)
     return (T)kStage[stage].cm * (T)dt;

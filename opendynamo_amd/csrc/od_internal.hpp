@@ -41,6 +41,17 @@ struct Ops {
     C gR[4];   // g_right'(x_i)
 };
 
+// The operators of one box in the fast build's kernels, with its Jacobians J_d =
+// 2 / h_d in them (formed in f64).
+struct BoxOps {
+    // Corrected derivative along d at points i and 3 - i (see od_kernels.hip)
+    struct EvenOdd {
+        float ps, pb, qa, qb, qp;
+    };
+    float table[80];  // J_d D [3][4][4], J_d {gL, gR} [3][4][2], {eL, eR} [2][4]
+    EvenOdd line[3][2];
+};
+
 // c * dt of one stage in the compute and the state type.  A captured step
 // graph reads it from device memory, so that a new dt leaves the graph valid
 // (capturing and instantiating it again takes milliseconds).
@@ -66,6 +77,7 @@ struct StageArgs {
     CT mu, mu_ref, t_ref, s_suth, bf;
     CT ca, cb, cc;     // blend coefficients in the compute type
     UT ua, ub, uc;     // blend coefficients in the state type
+    const BoxOps* ops;          // fast build: the box's operators (a batch: of box 0)
     const StageDt<UT, CT>* dt;  // cc and uc from here (null: as given above)
 };
 

@@ -613,22 +613,20 @@ constexpr int kFvStride = fv_stride(OD_FAST);
 // point's quad, so the fast f32 build contracts it from registers with DPP
 // quad broadcasts instead of an LDS round trip: the same products summed in
 // the same order, so the results are those of the LDS form bit for bit.
-template <class CT>
-constexpr bool kDppX = OD_FAST && std::is_same<CT, float>::value;
-template <class CT>
-__device__ __forceinline__ CT quad_line(const CT* Dd, CT f) {
-    static_assert(std::is_same<CT, float>::value, "DPP lanes are 32-bit");
-    const int x = __float_as_int(f);
-    const CT b0 = __int_as_float(__builtin_amdgcn_mov_dpp(x, 0x00, 0xF, 0xF, false));  // quad_perm [0,0,0,0]
-    const CT b1 = __int_as_float(__builtin_amdgcn_mov_dpp(x, 0x55, 0xF, 0xF, false));  // [1,1,1,1]
-    const CT b2 = __int_as_float(__builtin_amdgcn_mov_dpp(x, 0xAA, 0xF, 0xF, false));  // [2,2,2,2]
-    const CT b3 = __int_as_float(__builtin_amdgcn_mov_dpp(x, 0xFF, 0xF, 0xF, false));  // [3,3,3,3]
-    CT dd = 0;
-    dd += Dd[0] * b0;
-    dd += Dd[1] * b1;
-    dd += Dd[2] * b2;
-    dd += Dd[3] * b3;
-    return dd;
+// Sum of Dd[m] * (f of lane m of the quad), first a product, then fused in the
+// order of m.  The broadcasts are the multiplies' own DPP operands; left to
+// itself the compiler moves three of the four to a register first.  (s_nop: DPP
+// may read a register two instructions after it was written at the earliest.)
+__device__ __forceinline__ float quad_line(const float* Dd, float f) {
+    float s;
+    asm("s_nop 1\n\t"
+        "v_mul_f32_dpp %0, %1, %2 quad_perm:[0,0,0,0] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %3 quad_perm:[1,1,1,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %4 quad_perm:[2,2,2,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %5 quad_perm:[3,3,3,3] row_mask:0xf bank_mask:0xf"
+        : "=&v"(s)
+        : "v"(f), "v"(Dd[0]), "v"(Dd[1]), "v"(Dd[2]), "v"(Dd[3]));
+    return s;
 }
 // Fast f32 build: the interface correction takes the viscous fluxes of the
 // two sides as their half-difference (F_vL - F_vR) / 2, which the block visc
@@ -660,6 +658,24 @@ struct Coef4 {
 // it needs directly: selecting among 4 wave-uniform scalars costs 3
 // v_cndmask and 2 v_mov per coefficient and lane (one scalar operand per
 // VALU instruction).
+#if OD_FAST
+// Per direction, with the Jacobian in them (BoxOps): an instruction less for
+// every sum along a line, and for every lane's correction slopes.
+struct alignas(16) BoxTable {
+    float D[3][4][4];  // D[d][i][m] = J_d l_m'(x_i)
+    float g[3][4][2];  // J_d {g_left'(x_i), g_right'(x_i)}
+};
+template <class C>
+struct alignas(16) CoefTable : BoxTable {
+    C e[2][4];  // {l_m(-1)}, {l_m(+1)}
+};
+template <class C>
+using Rows = BoxTable;
+// A tile's own copy, and the coefficients of its lines' derivatives.
+struct TileTable : BoxTable {
+    BoxOps::EvenOdd line[3][2];
+};
+#else
 template <class C>
 struct alignas(16) CoefTable {
     C D[4][4];  // D[i][m] = l_m'(x_i)
@@ -667,27 +683,51 @@ struct alignas(16) CoefTable {
     C e[2][4];  // {l_m(-1)}, {l_m(+1)}
 };
 template <class C>
+using Rows = CoefTable<C>;
+struct TileTable {};
+#endif
+template <class C>
 __device__ __forceinline__ CoefTable<C>& coef_lds() {
     __shared__ CoefTable<C> t;
     return t;
 }
-// Threads 0..31 of the work-group copy the table from constant memory: the
+// The first threads of the work-group copy the table from memory: the
 // load is issued first thing (coef_load), the LDS store comes just before the
 // body's first barrier (coef_store), which orders it before every read, so
 // the load's latency hides behind the body's own loads.
 template <class C>
-__device__ __forceinline__ C coef_load(int tid) {
-    static_assert(sizeof(Ops<C>) == 32 * sizeof(C) && sizeof(CoefTable<C>) == 32 * sizeof(C), "table layout");
+constexpr int kCoefs = sizeof(CoefTable<C>) / sizeof(C);
+template <class UT, class C>
+__device__ __forceinline__ C coef_load(const StageArgs<UT, C>& a, int tid) {
+#if OD_FAST
+    static_assert(sizeof(BoxOps::table) == sizeof(CoefTable<C>) && kCoefs<C> <= 128, "table layout");
+    return tid < kCoefs<C> ? a.ops->table[tid] : (C)0;
+#else
+    static_assert(sizeof(Ops<C>) == 32 * sizeof(C) && kCoefs<C> == 32, "table layout");
     // Ops order: D[16], eL[4], eR[4], gL[4], gR[4]; the index stays inside
     // Ops for every thread, whether or not the load is speculated
     const int t = tid & 31;
     const int src = t < 16 ? t : (t < 24 ? 24 + ((t - 16) & 1) * 4 + ((t - 16) >> 1) : t - 8);
     return tid < 32 ? reinterpret_cast<const C*>(&dev_ops<C>())[src] : (C)0;
+#endif
 }
 template <class C>
 __device__ __forceinline__ void coef_store(int tid, C v) {
-    if (tid < 32) reinterpret_cast<C*>(&coef_lds<C>())[tid] = v;
+    if (tid < kCoefs<C>) reinterpret_cast<C*>(&coef_lds<C>())[tid] = v;
 }
+#if OD_FAST
+// The same for a tile's own copy, by its 128 threads.
+template <class UT>
+__device__ __forceinline__ float tile_table_load(const StageArgs<UT, float>& a, int tid) {
+    constexpr int kRows = sizeof(BoxTable) / sizeof(float), kLine = sizeof(BoxOps::line) / sizeof(float);
+    static_assert(kRows + kLine <= 128 && sizeof(TileTable) >= (kRows + kLine) * sizeof(float), "one value a thread");
+    const float* src = tid < kRows ? a.ops->table + tid : &a.ops->line[0][0].ps + (tid - kRows);
+    return tid < kRows + kLine ? *src : 0.f;
+}
+__device__ __forceinline__ void tile_table_store(TileTable& t, int tid, float v) {
+    if (tid < (int)((sizeof(BoxTable) + sizeof(BoxOps::line)) / sizeof(float))) reinterpret_cast<float*>(&t)[tid] = v;
+}
+#endif
 template <class C>
 __device__ __forceinline__ Coef4<C> side_coef(bool right) {
     const C* r = coef_lds<C>().e[right];
@@ -844,8 +884,47 @@ __device__ __forceinline__ void prefetch_issue(const StageArgs<UT, CT>& a, const
     }
 }
 
-// BR1 jump 1/2 (u_nb + u_own) - u_own at every face point of direction D
-// (accumulate_jump, rhs.cu:105-108; wall ghost rhs.cu:111-114), once per face
+#if OD_FAST
+// Corrected derivative along a line, d u / d xi + j_L g_L' + j_R g_R' with the
+// jumps j = (u_nb - u_own) / 2, in even and odd parts (fast f32 build).  The
+// points and operators mirror about the element's centre, D[3-i][m] =
+// -D[i][3-m] and g_R'[i] = -g_L'[3-i], and a constant has no derivative, so with
+//   t = (u0 + u3) - (u1 + u2),  d0 = u0 - u3,  d1 = u1 - u2,
+//   p = w_L - w_R,  q = w_L + w_R,  w = u_nb - u_own = 2 j,
+// the derivative at points i and 3 - i (i = 0, 1) is odd +- even:
+//   even = ps t + pb q,  odd = qa d0 + qb d1 + qp p.
+// 21 operations and the jumps' 2 for the line's four points with the Jacobian in
+// the coefficients (BoxOps); row by row they were 28 and 4.  Differences are
+// formed first, so less cancels than in the rows' sums.  One form for every
+// kernel, explicitly fused: the same bits.  With the Jacobians in the other
+// tables and the DPP operands of quad_line the block visc kernel issues a tenth
+// less: 48^3 132 -> 126 us, 64^3 292 -> 275 us a launch.
+using EvenOdd = BoxOps::EvenOdd;
+__device__ __forceinline__ float line_even(const EvenOdd& c, float t, float q) {
+    return __builtin_fmaf(c.pb, q, c.ps * t);
+}
+__device__ __forceinline__ float line_odd(const EvenOdd& c, float d0, float d1, float p) {
+    return __builtin_fmaf(c.qp, p, __builtin_fmaf(c.qb, d1, c.qa * d0));
+}
+// The coefficients along D of point pair i (wave-uniform: scalar loads).
+__device__ __forceinline__ EvenOdd even_odd(const BoxOps* ops, int D, int i) {
+    const auto* c = (const __attribute__((address_space(4))) float*)&ops->line[D][i];
+    return {c[0], c[1], c[2], c[3], c[4]};
+}
+// Those of a lane at point i of its line, the even part's sign with them.
+__device__ __forceinline__ EvenOdd lane_even_odd(const EvenOdd* line, int i) {
+    const EvenOdd& c = line[i == 1 || i == 2];
+    return {i < 2 ? c.ps : -c.ps, i < 2 ? c.pb : -c.pb, c.qa, c.qb, c.qp};
+}
+// The derivative at a lane's point from the line u[0], u[stride], ...
+__device__ __forceinline__ float lane_derivative(const EvenOdd& c, const float* u, int stride, float wl, float wr) {
+    const float u0 = u[0], u1 = u[stride], u2 = u[2 * stride], u3 = u[3 * stride];
+    return line_odd(c, u0 - u3, u1 - u2, wl - wr) + line_even(c, (u0 + u3) - (u1 + u2), wl + wr);
+}
+#endif
+
+// BR1 jump 1/2 (u_nb + u_own) - u_own (fast build: twice that, u_nb - u_own)
+// at every face point of direction D (accumulate_jump, rhs.cu:105-108; wall ghost rhs.cu:111-114), once per face
 // point instead of once per lane of the normal line.
 template <int D, bool PF, class UT, class CT>
 __device__ __forceinline__ void br1_jumps(const StageArgs<UT, CT>& a, const CT (*sU)[5][64], CT (*sJmp)[6][5][16],
@@ -869,7 +948,7 @@ __device__ __forceinline__ void br1_jumps(const StageArgs<UT, CT>& a, const CT (
         else
             far = !wall ? a.tr_in[nb * kTraceStride + (t.f ^ 1) * 80 + v * 16 + t.fp] : (CT)0;
         CT nbv = !wall ? far : own * sign;
-        sJmp[t.le][t.f][v][t.fp] = ((CT)0.5) * (nbv + own) - own;
+        sJmp[t.le][t.f][v][t.fp] = OD_FAST ? nbv - own : ((CT)0.5) * (nbv + own) - own;
     }
 }
 
@@ -879,13 +958,27 @@ __device__ __forceinline__ void br1_jumps(const StageArgs<UT, CT>& a, const CT (
 template <class UT, class CT>
 __device__ __forceinline__ void lane_gradient_faces(const StageArgs<UT, CT>& a, const CT (*sU)[64], const CT* J0,
                                                     const CT* J1, const CT* J2, const CT* J3, const CT* J4,
-                                                    const CT* J5, int i, int j, int k, CT* g) {
+                                                    const CT* J5, const TileTable& t, int i, int j, int k, CT* g) {
+    const int xb = 4 * j + 16 * k, yb = i + 16 * k, zb = i + 4 * j;
+    const int fpx = j + 4 * k, fpy = i + 4 * k, fpz = i + 4 * j;
+#if OD_FAST
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const EvenOdd c = lane_even_odd(t.line[d], d == 0 ? i : (d == 1 ? j : k));
+        const int base = d == 0 ? xb : (d == 1 ? yb : zb), stride = d == 0 ? 1 : (d == 1 ? 4 : 16);
+        const int fp = d == 0 ? fpx : (d == 1 ? fpy : fpz);
+        const CT *JL = d == 0 ? J0 : (d == 1 ? J2 : J4), *JR = d == 0 ? J1 : (d == 1 ? J3 : J5);
+#pragma unroll
+        for (int v = 0; v < 5; ++v) {
+            g[3 * v + d] = lane_derivative(c, &sU[v][base], stride, JL[v * 16 + fp], JR[v * 16 + fp]);
+            asm volatile("" : "+v"(g[3 * v + d])::"memory");  // one by one, as below
+        }
+    }
+#else
     const CoefTable<CT>& o = coef_lds<CT>();
     const CT* Di = o.D[i];
     const CT* Dj = o.D[j];
     const CT* Dk = o.D[k];
-    const int xb = 4 * j + 16 * k, yb = i + 16 * k, zb = i + 4 * j;
-    const int fpx = j + 4 * k, fpy = i + 4 * k, fpz = i + 4 * j;
     const CT gLi = o.g[i][0], gRi = o.g[i][1];
     const CT gLj = o.g[j][0], gRj = o.g[j][1];
     const CT gLk = o.g[k][0], gRk = o.g[k][1];
@@ -898,12 +991,6 @@ __device__ __forceinline__ void lane_gradient_faces(const StageArgs<UT, CT>& a, 
         for (int m = 0; m < 4; ++m) dxi += Di[m] * sU[v][xb + m];
 #pragma unroll
         for (int m = 0; m < 4; ++m) deta += Dj[m] * sU[v][yb + 4 * m];
-#if OD_FAST
-        // one Jacobian factor per direction
-        CT gx = fma_t(J1[v * 16 + fpx], gRi, fma_t(J0[v * 16 + fpx], gLi, dxi)) * a.jx;
-        CT gy = fma_t(J3[v * 16 + fpy], gRj, fma_t(J2[v * 16 + fpy], gLj, deta)) * a.jy;
-        CT gz = fma_t(J5[v * 16 + fpz], gRk, fma_t(J4[v * 16 + fpz], gLk, dz)) * a.jz;
-#else
         CT gx = dxi * a.jx, gy = deta * a.jy, gz = dz * a.jz;
         gx += J0[v * 16 + fpx] * gLi * a.jx;
         gx += J1[v * 16 + fpx] * gRi * a.jx;
@@ -911,7 +998,6 @@ __device__ __forceinline__ void lane_gradient_faces(const StageArgs<UT, CT>& a, 
         gy += J3[v * 16 + fpy] * gRj * a.jy;
         gz += J4[v * 16 + fpz] * gLk * a.jz;
         gz += J5[v * 16 + fpz] * gRk * a.jz;
-#endif
         if (a.round_q) {  // Q_REAL round trip (rhs.cu:457-461), narrows only when CT is double
             gx = (CT)(float)gx;
             gy = (CT)(float)gy;
@@ -925,13 +1011,14 @@ __device__ __forceinline__ void lane_gradient_faces(const StageArgs<UT, CT>& a, 
         g[3 * v + 1] = gy;
         g[3 * v + 2] = gz;
     }
+#endif
 }
 
 template <class UT, class CT>
 __device__ __forceinline__ void lane_gradient(const StageArgs<UT, CT>& a, const CT (*sU)[64], const CT (*sJmp)[5][16],
-                                              int i, int j, int k, CT* g) {
+                                              const TileTable& t, int i, int j, int k, CT* g) {
     lane_gradient_faces(a, sU, &sJmp[0][0][0], &sJmp[1][0][0], &sJmp[2][0][0], &sJmp[3][0][0], &sJmp[4][0][0],
-                        &sJmp[5][0][0], i, j, k, g);
+                        &sJmp[5][0][0], t, i, j, k, g);
 }
 
 template <bool PF, class UT, class CT>
@@ -1189,7 +1276,7 @@ __device__ __forceinline__ void load_state_tile(const UT* u, int64_t NP, int64_t
 // wave's 256-float LDS staging area.
 template <class UT>
 __device__ __forceinline__ void visc_divergence(const StageArgs<UT, float>& a, int64_t e, const float* st,
-                                                const float* g, float* S, int i, int j, int k, int pt) {
+                                                const float* g, const BoxTable& o, float* S, int i, int j, int k, int pt) {
     const FastVisc f = fast_visc(a, st, g, e);
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -1197,9 +1284,9 @@ __device__ __forceinline__ void visc_divergence(const StageArgs<UT, float>& a, i
         float fvv[4];
         fast_visc_flux(d, f, fvv);
         if (d == 0) {
-            const float* Dx = coef_lds<float>().D[i];
+            const float* Dx = o.D[0][i];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) acc[q] += quad_line(Dx, fvv[q]) * a.jx;
+            for (int q = 0; q < 4; ++q) acc[q] = quad_line(Dx, fvv[q]);
             continue;
         }
         if (d > 1) wave_sync();  // the previous direction's reads are done
@@ -1209,15 +1296,11 @@ __device__ __forceinline__ void visc_divergence(const StageArgs<UT, float>& a, i
         const int idx = d == 1 ? j : k;
         const int base = d == 1 ? i + 16 * k : i + 4 * j;
         const int stride = d == 1 ? 4 : 16;
-        const float jac = d == 1 ? a.jy : a.jz;
-        const float* Dd = coef_lds<float>().D[idx];
+        const float* Dd = o.D[d][idx];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            float dd = 0;
+        for (int q = 0; q < 4; ++q)
 #pragma unroll
-            for (int m = 0; m < 4; ++m) dd += Dd[m] * S[q * 64 + base + m * stride];
-            acc[q] += dd * jac;
-        }
+            for (int m = 0; m < 4; ++m) acc[q] = __builtin_fmaf(Dd[m], S[q * 64 + base + m * stride], acc[q]);
     }
     FvQuad<float>* dst = reinterpret_cast<FvQuad<float>*>(a.fv + e * kFvStride + kFvFaces + pt * 4);
     *dst = FvQuad<float>{{acc[0], acc[1], acc[2], acc[3]}};
@@ -1231,7 +1314,8 @@ __device__ __forceinline__ void visc_divergence(const StageArgs<UT, float>& a, i
 // fast build's Euler fluxes (vdiv: the divergence of the viscous ones).
 template <bool VISC, class UT, class CT>
 __device__ __forceinline__ void volume_rhs(const StageArgs<UT, CT>& a, const CT* st, const CT* g, CT mu,
-                                           const CT* vdiv, CT (*S)[64], int i, int j, int k, int pt, CT* out) {
+                                           const CT* vdiv, const Rows<CT>& o, CT (*S)[64], int i, int j, int k,
+                                           int pt, CT* out) {
     CT rs[5] = {(CT)0, (CT)0, (CT)0, (CT)0, (CT)0};
     ViscPoint<CT> vp;
     if constexpr (VISC) vp = viscous_point(st, g, mu, 7);
@@ -1245,23 +1329,30 @@ __device__ __forceinline__ void volume_rhs(const StageArgs<UT, CT>& a, const CT*
 #pragma unroll
             for (int v = 0; v < 5; ++v) F[v] = F[v] - fvv[v];
         }
-        if constexpr (kDppX<CT>) {
-            if (d == 0) {
-                const CT* Dx = coef_lds<CT>().D[i];
+#if OD_FAST
+        if (d == 0) {
+            const float* Dx = o.D[0][i];
 #pragma unroll
-                for (int v = 0; v < 5; ++v) rs[v] += quad_line(Dx, F[v]) * a.jx;
-                continue;
-            }
+            for (int v = 0; v < 5; ++v) rs[v] = quad_line(Dx, F[v]);
+            continue;
         }
-        if (d > (kDppX<CT> ? 1 : 0)) wave_sync();  // the previous direction's reads are done
+#endif
+        if (d > (OD_FAST ? 1 : 0)) wave_sync();  // the previous direction's reads are done
 #pragma unroll
         for (int v = 0; v < 5; ++v) S[v][pt] = F[v];
         wave_sync();
         const int idx = d == 0 ? i : (d == 1 ? j : k);
         const int base = d == 0 ? 4 * j + 16 * k : (d == 1 ? i + 16 * k : i + 4 * j);
         const int stride = d == 0 ? 1 : (d == 1 ? 4 : 16);
+#if OD_FAST
+        const float* Dd = o.D[d][idx];
+#pragma unroll
+        for (int v = 0; v < 5; ++v)
+#pragma unroll
+            for (int m = 0; m < 4; ++m) rs[v] = __builtin_fmaf(Dd[m], S[v][base + m * stride], rs[v]);
+#else
         const CT jac = d == 0 ? a.jx : (d == 1 ? a.jy : a.jz);
-        const CT* Dd = coef_lds<CT>().D[idx];
+        const CT* Dd = o.D[idx];
 #pragma unroll
         for (int v = 0; v < 5; ++v) {
             CT dd = 0;
@@ -1269,6 +1360,7 @@ __device__ __forceinline__ void volume_rhs(const StageArgs<UT, CT>& a, const CT*
             for (int m = 0; m < 4; ++m) dd += Dd[m] * S[v][base + m * stride];
             rs[v] += dd * jac;
         }
+#endif
     }
 #pragma unroll
     for (int v = 0; v < 5; ++v) {
@@ -1299,6 +1391,14 @@ struct ViscLds {
     CT sJmp[kEpb][6][5][16];
     CT sU[kEpb][5][64];
     CT sG_own[kPF ? 0 : kEpb][15][64];  // zero-length when aliased
+#if OD_FAST
+    TileTable tab;  // of the tile's box: a batch's work-group may have tiles of two boxes
+    __device__ const BoxTable& rows() { return tab; }
+    __device__ const TileTable& tile_table() { return tab; }
+#else
+    __device__ TileTable tile_table() { return {}; }
+    __device__ const CoefTable<CT>& rows() { return coef_lds<CT>(); }
+#endif
     __device__ CT (*sG())[15][64] {
         static_assert(!kPF || (kPfFloats == 15 * 64 && sizeof(sJmp) == kPfFloats * sizeof(float)), "sG aliasing layout");
         if constexpr (kPF) return reinterpret_cast<CT(*)[15][64]>(pf);
@@ -1323,6 +1423,14 @@ struct UpdateLds {
     CT sU[kEpb][5][64];
     CT sJ_own[kPF ? 0 : kEpb][6][5][16];  // zero-length when aliased
     CT sF[kVol ? kEpb : 0][5][64];
+#if OD_FAST
+    TileTable tab;  // of the tile's box: a batch's work-group may have tiles of two boxes
+    __device__ const BoxTable& rows() { return tab; }
+    __device__ const TileTable& tile_table() { return tab; }
+#else
+    __device__ TileTable tile_table() { return {}; }
+    __device__ const CoefTable<CT>& rows() { return coef_lds<CT>(); }
+#endif
     __device__ CT (*sJ())[6][5][16] {
         if constexpr (kPF) return reinterpret_cast<CT(*)[6][5][16]>(pf);
         else return sJ_own;
@@ -1333,7 +1441,7 @@ struct UpdateLds {
 template <class UT, class CT>
 __device__ __forceinline__ void trace_body(const StageArgs<UT, CT>& a, const Tile& tl, CT (*sU)[5][64], int wave,
                                            int pt) {
-    const CT cf = coef_load<CT>((int)threadIdx.x);
+    const CT cf = coef_load(a, (int)threadIdx.x);
     const int64_t NP = (int64_t)a.nx * a.ny * a.nz * 64;
     if (tile_valid(tl, wave)) {
 #pragma unroll
@@ -1352,16 +1460,22 @@ __device__ __forceinline__ void visc_body(const StageArgs<UT, CT>& a, const Tile
     constexpr bool PF = std::is_same<CT, float>::value;
     const int i = pt & 3, j = (pt >> 2) & 3, k = pt >> 4;
     const int64_t NP = (int64_t)a.nx * a.ny * a.nz * 64;
-    const CT cf = coef_load<CT>((int)threadIdx.x);
+    const CT cf = coef_load(a, (int)threadIdx.x);
+#if OD_FAST
+    const float row = tile_table_load(a, wave * 64 + pt);
+#endif
     if constexpr (PF) prefetch_issue<false>(a, tl, L.pf, wave, pt);
     if (tile_valid(tl, wave)) load_state_tile(a.uin, NP, tile_eidx(tl, wave), L.sU[wave], pt);
     coef_store<CT>((int)threadIdx.x, cf);
+#if OD_FAST
+    tile_table_store(L.tab, wave * 64 + pt, row);
+#endif
     if constexpr (PF) __builtin_amdgcn_s_waitcnt(0);  // this wave's LDS copies have landed
     __syncthreads();
     run_br1_jumps<PF>(a, L.sU, L.sJmp, tl, reinterpret_cast<const CT*>(L.pf), wave, pt);
     __syncthreads();
     CT g[15];
-    if (tile_valid(tl, wave)) lane_gradient(a, L.sU[wave], L.sJmp[wave], i, j, k, g);
+    if (tile_valid(tl, wave)) lane_gradient(a, L.sU[wave], L.sJmp[wave], L.tile_table(), i, j, k, g);
     if (tile_valid(tl, wave)) {
         const int64_t e = tile_eidx(tl, wave);
         CT st[5];
@@ -1369,12 +1483,12 @@ __device__ __forceinline__ void visc_body(const StageArgs<UT, CT>& a, const Tile
         for (int v = 0; v < 5; ++v) st[v] = L.sU[wave][v][pt];
         wave_sync();  // without a prefetch the staging area is the jumps just read
 #if OD_FAST
-        visc_divergence(a, e, st, g, L.vol_stage(wave), i, j, k, pt);
+        visc_divergence(a, e, st, g, L.rows(), L.vol_stage(wave), i, j, k, pt);
 #else
         CT r[5];
         CT mu = a.sutherland ? sutherland(st, a.mu_ref, a.t_ref, a.s_suth) : a.mu;
         if (a.mu_t) mu = mu + a.mu_t[e];
-        volume_rhs<true>(a, st, g, mu, (const CT*)nullptr, (CT(*)[64])L.vol_stage(wave), i, j, k, pt, r);
+        volume_rhs<true>(a, st, g, mu, (const CT*)nullptr, L.rows(), (CT(*)[64])L.vol_stage(wave), i, j, k, pt, r);
 #pragma unroll
         for (int v = 0; v < 5; ++v) a.fv[e * kFvStride + kFvFaces + v * 64 + pt] = r[v];
 #endif
@@ -1439,7 +1553,10 @@ __device__ __forceinline__ void update_body(const StageArgs<UT, CT>& a, const Ti
     const bool mine = tile_valid(tl, wave);
     const int64_t NP = (int64_t)a.nx * a.ny * a.nz * 64;
     const int64_t gbase = tile_eidx(tl, wave) * 64 + pt;
-    const CT cf = coef_load<CT>((int)threadIdx.x);
+    const CT cf = coef_load(a, (int)threadIdx.x);
+#if OD_FAST
+    const float row = tile_table_load(a, wave * 64 + pt);
+#endif
     if constexpr (PF) prefetch_issue<true>(a, tl, L.pf, wave, pt);
 
     constexpr bool SAME = std::is_same<UT, CT>::value;  // sU holds the state exactly
@@ -1455,6 +1572,9 @@ __device__ __forceinline__ void update_body(const StageArgs<UT, CT>& a, const Ti
         for (int v = 0; v < 5; ++v) L.sU[wave][v][pt] = (CT)(mine ? a.uin[v * NP + gbase] : (UT)1);
     }
     coef_store<CT>((int)threadIdx.x, cf);
+#if OD_FAST
+    tile_table_store(L.tab, wave * 64 + pt, row);
+#endif
     if constexpr (PF) __builtin_amdgcn_s_waitcnt(0);  // this wave's LDS copies have landed
     __syncthreads();
 
@@ -1475,8 +1595,8 @@ __device__ __forceinline__ void update_body(const StageArgs<UT, CT>& a, const Ti
         CT st[5];
 #pragma unroll
         for (int v = 0; v < 5; ++v) st[v] = L.sU[wave][v][pt];
-        volume_rhs<false>(a, st, (const CT*)nullptr, (CT)0, VISC ? vdiv : (const CT*)nullptr, L.sF[wave], i, j, k, pt,
-                          r);
+        volume_rhs<false>(a, st, (const CT*)nullptr, (CT)0, VISC ? vdiv : (const CT*)nullptr, L.rows(), L.sF[wave], i, j,
+                          k, pt, r);
         wave_sync();
 #pragma unroll
         for (int v = 0; v < 5; ++v) L.sF[wave][v][pt] = r[v];
@@ -1493,12 +1613,11 @@ __device__ __forceinline__ void update_body(const StageArgs<UT, CT>& a, const Ti
 
     // FR correction and stage update (rk.cu:12-25, 63-82).
     const StageDt<UT, CT> cdt = stage_dt(a);
-    const CoefTable<CT>& o = coef_lds<CT>();
+    const Rows<CT>& o = L.rows();
 #if OD_FAST
-    // correction slopes with the Jacobian folded in
-    const CT gLi = o.g[i][0] * a.jx, gRi = o.g[i][1] * a.jx;
-    const CT gLj = o.g[j][0] * a.jy, gRj = o.g[j][1] * a.jy;
-    const CT gLk = o.g[k][0] * a.jz, gRk = o.g[k][1] * a.jz;
+    const CT gLi = o.g[0][i][0], gRi = o.g[0][i][1];
+    const CT gLj = o.g[1][j][0], gRj = o.g[1][j][1];
+    const CT gLk = o.g[2][k][0], gRk = o.g[2][k][1];
 #else
     const CT gLi = o.g[i][0], gRi = o.g[i][1];
     const CT gLj = o.g[j][0], gRj = o.g[j][1];
@@ -1867,7 +1986,7 @@ __device__ __forceinline__ void strict_visc_body(const StageArgs<UT, CT>& a, con
     const int64_t NP = (int64_t)E * 64;
     const bool valid = BLOCK || e0 + wave < E;
     const int64_t e = BLOCK ? blk_elem(a, b, wave) : (valid ? e0 + wave : E - 1);
-    const CT cf = coef_load<CT>((int)threadIdx.x);
+    const CT cf = coef_load(a, (int)threadIdx.x);
     UT s0[5];
 #pragma unroll
     for (int v = 0; v < 5; ++v) s0[v] = a.uin[v * NP + e * 64 + pt];
@@ -1925,7 +2044,7 @@ __device__ __forceinline__ void strict_visc_body(const StageArgs<UT, CT>& a, con
     __syncthreads();  // the volume fluxes' lines are staged over the gradients
     CT mu = a.sutherland ? sutherland(st, a.mu_ref, a.t_ref, a.s_suth) : a.mu;
     if (a.mu_t) mu = mu + a.mu_t[e];
-    volume_rhs<true>(a, st, g, mu, (const CT*)nullptr, (CT(*)[64])(area + wave * kAreaStride), i, j, k, pt, r);
+    volume_rhs<true>(a, st, g, mu, (const CT*)nullptr, coef_lds<CT>(), (CT(*)[64])(area + wave * kAreaStride), i, j, k, pt, r);
     if (valid) {
 #pragma unroll
         for (int v = 0; v < 5; ++v) a.fv[e * kFvStride + kFvFaces + v * 64 + pt] = r[v];
@@ -2099,7 +2218,7 @@ __device__ __forceinline__ void face_block_body(const StageArgs<UT, CT>& a, cons
     const int64_t NP = (int64_t)a.nx * a.ny * a.nz * 64;
     const int64_t e = blk_elem(a, b, wave);
     const int64_t gbase = e * 64 + pt;
-    const CT cf = coef_load<CT>((int)threadIdx.x);
+    const CT cf = coef_load(a, (int)threadIdx.x);
     UT s0[5];
 #pragma unroll
     for (int v = 0; v < 5; ++v) s0[v] = a.uin[v * NP + gbase];
@@ -2369,7 +2488,7 @@ __device__ __forceinline__ void update_block_body(const StageArgs<float, float>&
     const int64_t NP = (int64_t)a.nx * a.ny * a.nz * 64;
     const int64_t e = blk_elem(a, b, wave);
     const int64_t gbase = e * 64 + pt;
-    const float cf = coef_load<float>((int)threadIdx.x);
+    const float cf = coef_load(a, (int)threadIdx.x);
     // the element's three external neighbour traces (60 16-byte LDS-DMA
     // chunks) and its state, both read for the last time in this stage:
     // streaming, like the update kernel's stores
@@ -2384,6 +2503,7 @@ __device__ __forceinline__ void update_block_body(const StageArgs<float, float>&
     __builtin_amdgcn_s_waitcnt(0);  // this wave's LDS copies have landed
     __syncthreads();
 
+    const CoefTable<float>& o = coef_lds<float>();
     // Volume RHS of the wave's element (update_body's fast f32 path).
     float st[5];
 #pragma unroll
@@ -2400,9 +2520,9 @@ __device__ __forceinline__ void update_block_body(const StageArgs<float, float>&
         float F[5];
         euler_flux(d, st, F);
         if (d == 0) {
-            const float* Dx = coef_lds<float>().D[i];
+            const float* Dx = o.D[0][i];
 #pragma unroll
-            for (int v = 0; v < 5; ++v) rs[v] += quad_line(Dx, F[v]) * a.jx;
+            for (int v = 0; v < 5; ++v) rs[v] = quad_line(Dx, F[v]);
             continue;
         }
         if (d > 1) wave_sync();  // the y lines have been read
@@ -2412,15 +2532,11 @@ __device__ __forceinline__ void update_block_body(const StageArgs<float, float>&
         const int idx = d == 1 ? j : k;
         const int base = d == 1 ? i + 16 * k : i + 4 * j;
         const int stride = d == 1 ? 4 : 16;
-        const float jac = d == 1 ? a.jy : a.jz;
-        const float* Dd = coef_lds<float>().D[idx];
+        const float* Dd = o.D[d][idx];
 #pragma unroll
-        for (int v = 0; v < 5; ++v) {
-            float dd = 0;
+        for (int v = 0; v < 5; ++v)
 #pragma unroll
-            for (int m = 0; m < 4; ++m) dd += Dd[m] * L.sF[wave][v][base + m * stride];
-            rs[v] += dd * jac;
-        }
+            for (int m = 0; m < 4; ++m) rs[v] = __builtin_fmaf(Dd[m], L.sF[wave][v][base + m * stride], rs[v]);
     }
     wave_sync();
 #pragma unroll
@@ -2448,10 +2564,9 @@ __device__ __forceinline__ void update_block_body(const StageArgs<float, float>&
     // FR correction and stage update of the wave's element (rk.cu:12-25,
     // 63-82; update_body's fast f32 path).
     const StageDt<float, float> cdt = stage_dt(a);
-    const CoefTable<float>& o = coef_lds<float>();
-    const float gLi = o.g[i][0] * a.jx, gRi = o.g[i][1] * a.jx;
-    const float gLj = o.g[j][0] * a.jy, gRj = o.g[j][1] * a.jy;
-    const float gLk = o.g[k][0] * a.jz, gRk = o.g[k][1] * a.jz;
+    const float gLi = o.g[0][i][0], gRi = o.g[0][i][1];
+    const float gLj = o.g[1][j][0], gRj = o.g[1][j][1];
+    const float gLk = o.g[2][k][0], gRk = o.g[2][k][1];
     const int fpx = j + 4 * k, fpy = i + 4 * k, fpz = i + 4 * j;
     const int lx = wave & 1, ly = (wave >> 1) & 1, lz = wave >> 2;
     const float* Jext = &L.sJe[wave][0][0][0];
@@ -2584,7 +2699,7 @@ __device__ __forceinline__ void line_gradient(const StageArgs<float, float>& a, 
                                               LineWave& w) {
     const Ops<float>& o = dev_ops<float>();
     const bool wall = D == 1 && blk_ext_nb(a, b, w.le, D) < 0;
-    const float jac = D == 0 ? a.jx : (D == 1 ? a.jy : a.jz);
+    const EvenOdd c[2] = {even_odd(a.ops, D, 0), even_odd(a.ops, D, 1)};
 #pragma unroll
     for (int v = 0; v < 5; ++v) {
         const float* u = w.u[v];
@@ -2592,15 +2707,14 @@ __device__ __forceinline__ void line_gradient(const StageArgs<float, float>& a, 
         const float in = lane_partner(w.side ? tl : tr);
         const float own = w.side ? tr : tl;
         const float ext = wall ? ((v > 0 && v < 4) ? -own : own) : w.ext[v];
-        const float nl = w.side ? in : ext, nr = w.side ? ext : in;
-        const float jl = __builtin_fmaf(0.5f, nl + tl, -tl), jr = __builtin_fmaf(0.5f, nr + tr, -tr);
+        const float wl = (w.side ? in : ext) - tl, wr = (w.side ? ext : in) - tr;
+        const float t = (u[0] + u[3]) - (u[1] + u[2]), d0 = u[0] - u[3], d1 = u[1] - u[2];
+        const float p = wl - wr, q = wl + wr;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float d = 0.f;
-#pragma unroll
-            for (int m = 0; m < 4; ++m) d = __builtin_fmaf(o.D[4 * i + m], u[m], d);
-            L.area[w.pos[i] + (3 * v + D) * 64] =
-                __builtin_fmaf(jr, o.gR[i], __builtin_fmaf(jl, o.gL[i], d)) * jac;
+        for (int i = 0; i < 2; ++i) {
+            const float ev = line_even(c[i], t, q), od = line_odd(c[i], d0, d1, p);
+            L.area[w.pos[i] + (3 * v + D) * 64] = od + ev;
+            L.area[w.pos[3 - i] + (3 * v + D) * 64] = od - ev;
         }
         w.tl[v] = tl;
         w.tr[v] = tr;
@@ -2660,7 +2774,7 @@ __device__ __forceinline__ void visc_block_body(const StageArgs<float, float>& a
     const int64_t NP = (int64_t)a.nx * a.ny * a.nz * 64;
     const int64_t e = blk_elem(a, b, wave);
     const int half = role / 3, D = role < 6 ? role - 3 * half : 3;
-    const float cf = coef_load<float>((int)threadIdx.x);
+    const float cf = coef_load(a, (int)threadIdx.x);
     float s0[5];
 #pragma unroll
     for (int v = 0; v < 5; ++v) s0[v] = a.uin[v * NP + e * 64 + pt];
@@ -2708,7 +2822,7 @@ __device__ __forceinline__ void visc_block_body(const StageArgs<float, float>& a
 #pragma unroll
     for (int v = 0; v < 5; ++v) st[v] = a.uin[v * NP + e * 64 + pt];
     __syncthreads();  // the volume fluxes' lines are staged over the gradients
-    visc_divergence(a, e, st, g, L.of(wave), i, j, k, pt);
+    visc_divergence(a, e, st, g, coef_lds<float>(), L.of(wave), i, j, k, pt);
 }
 
 // One box: the update kernel walks the blocks backwards, the visc kernel
@@ -2768,9 +2882,11 @@ __device__ __forceinline__ Elem uni(const Elem& e) {
 // Stage arguments of one box of a batch: the batch's arguments with the
 // box's dimensions, Jacobians, stage coefficients and buffer offsets.
 template <class UT, class CT>
-__device__ __forceinline__ void batch_box_args(const StageArgs<UT, CT>& a, const BoxDev<UT, CT>& bx, int stage,
+__device__ __forceinline__ void batch_box_args(const StageArgs<UT, CT>& a, const BoxDev<UT, CT>* boxes, int box, int stage,
                                                StageArgs<UT, CT>& ab) {
+    const BoxDev<UT, CT>& bx = boxes[box];
     ab = a;
+    ab.ops = a.ops + box;
     ab.nx = uni(bx.nx);
     ab.ny = uni(bx.ny);
     ab.nz = uni(bx.nz);
@@ -2834,7 +2950,7 @@ __device__ __forceinline__ void batch_tile(const StageArgs<UT, CT>& a, const Bat
         }
     }
     const BoxDev<UT, CT>& bx = b.boxes[lo];
-    batch_box_args(a, bx, b.stage, ab);
+    batch_box_args(a, b.boxes, uni(lo), b.stage, ab);
     const int tile_off = uni(bx.tile_off);
     const int lt = tt - tile_off;
     if (uni(bx.shell)) {
@@ -2901,7 +3017,7 @@ __device__ __forceinline__ void batch_block(const StageArgs<float, float>& a, co
         }
         off = uni(bb.boxes[lo].blk_off);
     }
-    batch_box_args(a, bb.boxes[lo], bb.stage, ab);
+    batch_box_args(a, bb.boxes, lo, bb.stage, ab);
     b = core_block(ab, t - off);
 }
 
@@ -2926,11 +3042,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8))) void o
 // One box with an odd dimension: its core on blocks and its shell on tiles in
 // one launch.  A 512-thread work-group takes a block of the core, or as many
 // tiles of the shell as fit its threads and a block's LDS: three in the visc
-// kernel (10.3 KB each), four in the update kernel (9.1 KB).  The blocks come first (the update kernel's backwards,
-// as in the even boxes) and the shell, a small part of the box, fills up the
-// last work-groups' wave; a launch of its own would cost its latency twice a
-// stage.  33x25x37 (AUSM+, 100 steps): 37.4 ms with every element on tiles,
-// 33.6 so (30.0 with the visc kernel's blocks by lines).
+// kernel (10.6 KB each), four in the update kernel (9.4 KB).  The shell, a small
+// part of the box, whose tiles take longest from start to end, comes first in
+// both, so that the blocks cover it (after the blocks it ended the launch alone:
+// 33x25x37 visc 41.5 against 39.2 us, update 43.8 against 43.4 us); a launch of
+// its own would cost its latency twice a stage.  The update kernel walks the
+// blocks backwards, as in the even boxes.  33x25x37 (AUSM+, 100 steps): 37.4 ms
+// with every element on tiles, 29.5 so.
 struct CoreShell {
     int32_t n_blocks, n_tiles;  // blocks of the core, tiles of the shell
 };
@@ -2955,9 +3073,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8))) void o
         BlockUpdateLds block;
         UpdateLds<float, VISC> tile[kShellTiles[1]];
     } L;
-    const int w = (int)blockIdx.x;
+    const int w = (int)(gridDim.x - 1 - blockIdx.x);
     if (w < cs.n_blocks)
-        update_block_body<VISC>(a, core_block(a, cs.n_blocks - 1 - w), L.block);
+        update_block_body<VISC>(a, core_block(a, w), L.block);
     else
         update_body<float, float, VISC>(a, core_shell_tile<kShellTiles[1]>(a, cs, w - cs.n_blocks),
                                         L.tile[threadIdx.x >> 7],
@@ -2968,12 +3086,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8))) void o
         BlockViscLds block;
         ViscLds<float> tile[kShellTiles[0]];
     } L;
-    const int w = (int)blockIdx.x;
-    if (w < cs.n_blocks)
-        visc_block_body(a, core_block(a, w), L.block, line_role(w));
-    else
-        visc_body(a, core_shell_tile<kShellTiles[0]>(a, cs, w - cs.n_blocks),
-                  L.tile[min((int)(threadIdx.x >> 7), kShellTiles[0] - 1)], wave_index() & 1, threadIdx.x & 63);
+    const int shell = (int)gridDim.x - cs.n_blocks, w = (int)blockIdx.x - shell;
+    if (w < 0) {
+        int pt = threadIdx.x & 63;
+        asm volatile("" : "+v"(pt));  // its own: what both forms derive from it is not hoisted and held (6 spills)
+        visc_body(a, core_shell_tile<kShellTiles[0]>(a, cs, w + shell),
+                  L.tile[min((int)(threadIdx.x >> 7), kShellTiles[0] - 1)], wave_index() & 1, pt);
+        return;
+    }
+    visc_block_body(a, core_block(a, w), L.block, line_role(w));
 }
 #endif
 
