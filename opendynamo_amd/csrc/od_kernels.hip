@@ -1543,31 +1543,40 @@ __device__ __forceinline__ void rk_stage(const StageArgs<UT, CT>& a, const Stage
 }
 
 // Full stage for the tile: volume RHS, interface fluxes, FR correction, RK
-// blend, and the face traces of the new state.
-template <class UT, class CT, bool VISC>
+// blend, and the face traces of the new state.  WIDE, for small boxes, whose
+// kernels last as long as one work-group: more waves than elements; the first
+// two own an element in the point-wise phases, and the faces of each direction
+// are another wave's, beside the volume RHS where this kernel forms it, so that
+// no wave does two things in a row that could be done at once.
+template <class CT, bool VISC>
+constexpr int kWideWaves = UpdateLds<CT, VISC>::kVol ? 5 : 3;
+template <class UT, class CT, bool VISC, bool WIDE = false>
 __device__ __forceinline__ void update_body(const StageArgs<UT, CT>& a, const Tile& tl, UpdateLds<CT, VISC>& L,
                                             int wave, int pt) {
     constexpr bool PF = std::is_same<CT, float>::value;
     const CT* pfc = reinterpret_cast<const CT*>(L.pf);
     const int i = pt & 3, j = (pt >> 2) & 3, k = pt >> 4;
-    const bool mine = tile_valid(tl, wave);
+    const bool owner = !WIDE || wave < kEpb;
+    const bool mine = owner && tile_valid(tl, wave);
     const int64_t NP = (int64_t)a.nx * a.ny * a.nz * 64;
     const int64_t gbase = tile_eidx(tl, wave) * 64 + pt;
     const CT cf = coef_load(a, (int)threadIdx.x);
 #if OD_FAST
     const float row = tile_table_load(a, wave * 64 + pt);
 #endif
-    if constexpr (PF) prefetch_issue<true>(a, tl, L.pf, wave, pt);
+    if constexpr (PF) {
+        if (owner) prefetch_issue<true>(a, tl, L.pf, wave, pt);
+    }
 
     constexpr bool SAME = std::is_same<UT, CT>::value;  // sU holds the state exactly
     if constexpr (SAME && PF) {  // f32 state and compute: LDS-DMA
         if (mine) {
             load_state_tile(a.uin, NP, tile_eidx(tl, wave), L.sU[wave], pt);
-        } else {
+        } else if (owner) {
 #pragma unroll
             for (int v = 0; v < 5; ++v) L.sU[wave][v][pt] = (CT)1;
         }
-    } else {
+    } else if (owner) {
 #pragma unroll
         for (int v = 0; v < 5; ++v) L.sU[wave][v][pt] = (CT)(mine ? a.uin[v * NP + gbase] : (UT)1);
     }
@@ -1582,7 +1591,7 @@ __device__ __forceinline__ void update_body(const StageArgs<UT, CT>& a, const Ti
     // the visc kernel's viscous divergence) and kept in LDS during the face
     // passes; else the visc kernel's, read after them.
     constexpr bool VOL = UpdateLds<CT, VISC>::kVol;
-    if constexpr (VOL) {
+    if constexpr (VOL) if (owner) {
         CT vdiv[4] = {(CT)0, (CT)0, (CT)0, (CT)0}, r[5];
         if constexpr (VISC) {
             if (mine) {
@@ -1603,13 +1612,22 @@ __device__ __forceinline__ void update_body(const StageArgs<UT, CT>& a, const Ti
     }
 
     // Interface fluxes at all own faces, direction by direction.
-    if (wave == 0) {
+    if constexpr (WIDE) {
+        const int d = wave - (VOL ? kEpb : 0);
+        if (d == 0)
+            flux_pass<0, VISC, PF>(a, L.sU, L.sJ(), tl, pfc, pt);
+        else if (d == 1)
+            flux_pass<1, VISC, PF>(a, L.sU, L.sJ(), tl, pfc, pt);
+        else if (d == 2)
+            flux_pass<2, VISC, PF>(a, L.sU, L.sJ(), tl, pfc, pt);
+    } else if (wave == 0) {
         flux_pass<0, VISC, PF>(a, L.sU, L.sJ(), tl, pfc, pt);
         flux_pass<2, VISC, PF>(a, L.sU, L.sJ(), tl, pfc, pt);
     } else {
         flux_pass<1, VISC, PF>(a, L.sU, L.sJ(), tl, pfc, pt);
     }
     __syncthreads();
+    if (!owner) return;
 
     // FR correction and stage update (rk.cu:12-25, 63-82).
     const StageDt<UT, CT> cdt = stage_dt(a);
@@ -1707,11 +1725,11 @@ constexpr int kMinWaves = sizeof(CT) == 4 ? 4 : 1;
 template <class UT, class CT>
 constexpr int kMinWavesUpdate = (OD_FAST && sizeof(UT) == 4 && sizeof(CT) == 4) ? 8 : kMinWaves<CT>;
 
-template <class UT, class CT, bool VISC>
-__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(kMinWavesUpdate<UT, CT>))) void od_update_kernel(
+template <class UT, class CT, bool VISC, bool WIDE>
+__global__ __launch_bounds__((64 * (WIDE ? kWideWaves<CT, VISC> : kEpb))) __attribute__((amdgpu_waves_per_eu(kMinWavesUpdate<UT, CT>))) void od_update_kernel(
     StageArgs<UT, CT> a) {
     __shared__ UpdateLds<CT, VISC> L;
-    update_body<UT, CT, VISC>(a, make_tile_reversed(a), L, wave_index(), threadIdx.x & 63);
+    update_body<UT, CT, VISC, WIDE>(a, make_tile_reversed(a), L, wave_index(), threadIdx.x & 63);
 }
 
 // LDS area of one element in the kernels that work by lines: [5][64] or
@@ -3280,9 +3298,24 @@ int launch_visc(const StageArgs<UT, CT>& a, int64_t n_elem, void* stream) {
     return check_launch();
 }
 
+// Largest number of tiles that the wide update kernel takes: its work-groups must
+// all be resident at once, or it loses to the narrow one's finer grain (256 CUs;
+// two work-groups of five waves with f64 compute, more of three).  us a step,
+// narrow and wide: Euler f64 8^3 (256 tiles) 23.5 18.1, 10^3 (500) 30.0 23.5,
+// 12x11x11 (726) 33.0 34.0, 16^3 58 87; Euler f32 8^3 19.9 15.9; f64 8^3 52.5
+// 47.8, 13x12x12 (1008) 77.8 74.4, 15^3 (1800) 103 109; f32 8^3 40.7 38.9, 17^3
+// (2601) 82.4 85.8; fast 1x16x16 (128) 33.6 31.2, 1x39x39 (760) 52.5 52.8.
+template <class CT, bool VISC>
+constexpr int64_t kWideTiles = 256 * (UpdateLds<CT, VISC>::kVol ? 2 : 4);
+
 template <class UT, class CT, bool VISC>
 int launch_update(const StageArgs<UT, CT>& a, int64_t n_elem, void* stream) {
-    hipLaunchKernelGGL((od_update_kernel<UT, CT, VISC>), grid_of(a), dim3(64 * kEpb), 0, (hipStream_t)stream, a);
+    const dim3 g = grid_of(a);
+    if ((int64_t)g.x * g.y * g.z <= kWideTiles<CT, VISC>)
+        hipLaunchKernelGGL((od_update_kernel<UT, CT, VISC, true>), g, dim3(64 * kWideWaves<CT, VISC>), 0,
+                           (hipStream_t)stream, a);
+    else
+        hipLaunchKernelGGL((od_update_kernel<UT, CT, VISC, false>), g, dim3(64 * kEpb), 0, (hipStream_t)stream, a);
     return check_launch();
 }
 
