@@ -2671,9 +2671,12 @@ __device__ __forceinline__ void update_block_body(const StageArgs<float, float>&
 // than their size, so that the partner along x, y, z is 4, 8, 16 banks away,
 // the bit that swz64 keeps fixed over a face of that direction.
 // ---------------------------------------------------------------------------
+template <bool WIDE>
 struct BlockViscLds {
     alignas(16) float area[kBlk * kAreaStride];
+    float own_stage[WIDE ? kBlk : 0][4 * 64];  // staging of the volume fluxes' lines: over the gradients, or its own
     __device__ float* of(int le) { return area + le * kAreaStride; }
+    __device__ float* stage(int le) { return WIDE ? own_stage[le] : of(le); }
 };
 
 // End trace sum_m q[m] l_m(+-1) in the BR1 order (the right end's coefficients
@@ -2713,7 +2716,7 @@ __device__ __forceinline__ void line_begin(const StageArgs<float, float>& a, con
 // Jumps and corrected derivative along D (br1_jumps, lane_gradient_faces) ->
 // the gradient's rows 3 v + D.
 template <int D>
-__device__ __forceinline__ void line_gradient(const StageArgs<float, float>& a, const Block& b, BlockViscLds& L,
+__device__ __forceinline__ void line_gradient(const StageArgs<float, float>& a, const Block& b, float* area,
                                               LineWave& w) {
     const Ops<float>& o = dev_ops<float>();
     const bool wall = D == 1 && blk_ext_nb(a, b, w.le, D) < 0;
@@ -2731,8 +2734,8 @@ __device__ __forceinline__ void line_gradient(const StageArgs<float, float>& a, 
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const float ev = line_even(c[i], t, q), od = line_odd(c[i], d0, d1, p);
-            L.area[w.pos[i] + (3 * v + D) * 64] = od + ev;
-            L.area[w.pos[3 - i] + (3 * v + D) * 64] = od - ev;
+            area[w.pos[i] + (3 * v + D) * 64] = od + ev;
+            area[w.pos[3 - i] + (3 * v + D) * 64] = od - ev;
         }
         w.tl[v] = tl;
         w.tr[v] = tr;
@@ -2745,7 +2748,7 @@ __device__ __forceinline__ void line_gradient(const StageArgs<float, float>& a, 
 // element stores the half-difference (F_vL - F_vR) / 2, all the update kernel
 // reads there.
 template <int D>
-__device__ __forceinline__ void line_flux(const StageArgs<float, float>& a, const Block& b, const BlockViscLds& L,
+__device__ __forceinline__ void line_flux(const StageArgs<float, float>& a, const Block& b, const float* area,
                                           const LineWave& w) {
     const Ops<float>& o = dev_ops<float>();
     float gl[15], gr[15];
@@ -2761,7 +2764,7 @@ __device__ __forceinline__ void line_flux(const StageArgs<float, float>& a, cons
         }
         float x[4];
 #pragma unroll
-        for (int m = 0; m < 4; ++m) x[m] = L.area[w.pos[m] + q * 64];
+        for (int m = 0; m < 4; ++m) x[m] = area[w.pos[m] + q * 64];
         gl[q] = __builtin_fmaf(x[3], o.eL[3], __builtin_fmaf(x[2], o.eL[2], __builtin_fmaf(x[1], o.eL[1], x[0] * o.eL[0])));
         gr[q] = __builtin_fmaf(x[3], o.eR[3], __builtin_fmaf(x[2], o.eR[2], __builtin_fmaf(x[1], o.eR[1], x[0] * o.eR[0])));
         asm volatile("" : "+v"(gl[q]), "+v"(gr[q])::"memory");
@@ -2785,17 +2788,21 @@ __device__ __forceinline__ void line_flux(const StageArgs<float, float>& a, cons
 
 // role: 0..5 the line waves (direction role % 3, half of the pairs role / 3),
 // 6 and 7 none.
-__device__ __forceinline__ void visc_block_body(const StageArgs<float, float>& a, const Block& b, BlockViscLds& L,
-                                                int role) {
+template <bool WIDE = false>
+__device__ __forceinline__ void visc_block_body(const StageArgs<float, float>& a, const Block& b,
+                                                BlockViscLds<WIDE>& L, int role) {
     const int wave = wave_index(), pt = threadIdx.x & 63;
     const int i = pt & 3, j = (pt >> 2) & 3, k = pt >> 4;
     const int64_t NP = (int64_t)a.nx * a.ny * a.nz * 64;
-    const int64_t e = blk_elem(a, b, wave);
+    const bool owner = !WIDE || wave < kBlk;
+    const int64_t e = blk_elem(a, b, wave & (kBlk - 1));
     const int half = role / 3, D = role < 6 ? role - 3 * half : 3;
     const float cf = coef_load(a, (int)threadIdx.x);
     float s0[5];
+    if (owner) {
 #pragma unroll
-    for (int v = 0; v < 5; ++v) s0[v] = a.uin[v * NP + e * 64 + pt];
+        for (int v = 0; v < 5; ++v) s0[v] = a.uin[v * NP + e * 64 + pt];
+    }
     LineWave w;
     if (D == 0)
         line_begin<0>(a, b, half, pt, w);
@@ -2803,7 +2810,7 @@ __device__ __forceinline__ void visc_block_body(const StageArgs<float, float>& a
         line_begin<1>(a, b, half, pt, w);
     else if (D == 2)
         line_begin<2>(a, b, half, pt, w);
-    {
+    if (owner) {
         float* A = L.of(wave) + swz64(pt);
 #pragma unroll
         for (int v = 0; v < 5; ++v) A[v * 64] = s0[v];
@@ -2818,18 +2825,19 @@ __device__ __forceinline__ void visc_block_body(const StageArgs<float, float>& a
     }
     __syncthreads();  // the gradients overwrite the states
     if (D == 0)
-        line_gradient<0>(a, b, L, w);
+        line_gradient<0>(a, b, L.area, w);
     else if (D == 1)
-        line_gradient<1>(a, b, L, w);
+        line_gradient<1>(a, b, L.area, w);
     else if (D == 2)
-        line_gradient<2>(a, b, L, w);
+        line_gradient<2>(a, b, L.area, w);
     __syncthreads();
     if (D == 0)
-        line_flux<0>(a, b, L, w);
+        line_flux<0>(a, b, L.area, w);
     else if (D == 1)
-        line_flux<1>(a, b, L, w);
+        line_flux<1>(a, b, L.area, w);
     else if (D == 2)
-        line_flux<2>(a, b, L, w);
+        line_flux<2>(a, b, L.area, w);
+    if (!owner) return;
     float g[15];
     {
         const float* A = L.of(wave) + swz64(pt);
@@ -2839,8 +2847,8 @@ __device__ __forceinline__ void visc_block_body(const StageArgs<float, float>& a
     float st[5];  // the point's state again (from L2), not held through the line phases
 #pragma unroll
     for (int v = 0; v < 5; ++v) st[v] = a.uin[v * NP + e * 64 + pt];
-    __syncthreads();  // the volume fluxes' lines are staged over the gradients
-    visc_divergence(a, e, st, g, coef_lds<float>(), L.of(wave), i, j, k, pt);
+    if constexpr (!WIDE) __syncthreads();  // the volume fluxes' lines are staged over the gradients
+    visc_divergence(a, e, st, g, coef_lds<float>(), L.stage(wave), i, j, k, pt);
 }
 
 // One box: the update kernel walks the blocks backwards, the visc kernel
@@ -2851,10 +2859,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8))) void o
     __shared__ BlockUpdateLds L;
     update_block_body<VISC>(a, make_block<true>(a), L);
 }
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8))) void od_visc_block_kernel(StageArgs<float, float> a) {
-    __shared__ BlockViscLds L;
+// WIDE, for small boxes, whose kernels last as long as one work-group: the six
+// line waves are waves of their own beside the eight of the elements, so that
+// the fluxes at the lines' ends and the divergence at the points, which both need
+// the gradients, run at once.
+constexpr int kWideBlockWaves = kBlk + 6;
+template <bool WIDE>
+__global__ __launch_bounds__((64 * (WIDE ? kWideBlockWaves : kBlk))) __attribute__((amdgpu_waves_per_eu(WIDE ? 7 : 8))) void od_visc_block_kernel(
+    StageArgs<float, float> a) {
+    __shared__ BlockViscLds<WIDE> L;
     const int group = (int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
-    visc_block_body(a, make_block<false>(a), L, line_role(group));
+    const int role = WIDE ? (wave_index() < kBlk ? 6 : wave_index() - kBlk) : line_role(group);
+    visc_block_body<WIDE>(a, make_block<false>(a), L, role);
 }
 #endif
 
@@ -3053,8 +3069,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8))) void o
     StageArgs<float, float> ab;
     Block b;
     batch_block<false>(a, bb, ab, b);
-    __shared__ BlockViscLds L;
-    visc_block_body(ab, b, L, line_role((int)blockIdx.x));
+    __shared__ BlockViscLds<false> L;
+    visc_block_body<false>(ab, b, L, line_role((int)blockIdx.x));
 }
 
 // One box with an odd dimension: its core on blocks and its shell on tiles in
@@ -3101,7 +3117,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8))) void o
 }
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8))) void od_visc_core_shell_kernel(StageArgs<float, float> a, CoreShell cs) {
     __shared__ union {
-        BlockViscLds block;
+        BlockViscLds<false> block;
         ViscLds<float> tile[kShellTiles[0]];
     } L;
     const int shell = (int)gridDim.x - cs.n_blocks, w = (int)blockIdx.x - shell;
@@ -3112,7 +3128,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8))) void o
                   L.tile[min((int)(threadIdx.x >> 7), kShellTiles[0] - 1)], wave_index() & 1, pt);
         return;
     }
-    visc_block_body(a, core_block(a, w), L.block, line_role(w));
+    visc_block_body<false>(a, core_block(a, w), L.block, line_role(w));
 }
 #endif
 
@@ -3329,9 +3345,18 @@ int launch_update_block(const StageArgs<float, float>& a, void* stream) {
 template int launch_update_block<true>(const StageArgs<float, float>&, void*);
 template int launch_update_block<false>(const StageArgs<float, float>&, void*);
 
+// Largest number of blocks that the wide visc kernel takes: one work-group to
+// each of the 256 CUs.  us a launch, narrow and wide: 4^3 7.9 7.4, 8^3 (64 blocks)
+// 8.4 7.7, 12^3 (216) 9.9 9.3, 14^3 (343) 11.9 12.9, 16^3 (512) 13.6 14.4.  (The
+// update kernel gains 0.1 us of 8 from the like, which is not worth a second form.)
+constexpr int64_t kWideBlocks = 256;
 int launch_visc_block(const StageArgs<float, float>& a, void* stream) {
     if (a.nx % 2 || a.ny % 2 || a.nz % 2) return 1;
-    hipLaunchKernelGGL(od_visc_block_kernel, block_grid(a), dim3(64 * kBlk), 0, (hipStream_t)stream, a);
+    const dim3 g = block_grid(a);
+    if ((int64_t)g.x * g.y * g.z <= kWideBlocks)
+        hipLaunchKernelGGL(od_visc_block_kernel<true>, g, dim3(64 * kWideBlockWaves), 0, (hipStream_t)stream, a);
+    else
+        hipLaunchKernelGGL(od_visc_block_kernel<false>, g, dim3(64 * kBlk), 0, (hipStream_t)stream, a);
     return check_launch();
 }
 namespace {

@@ -64,3 +64,26 @@ def test_wide_and_narrow_form_agree(n, times, types):
         assert np.isfinite(out[0]).all()
         for t in range(times):
             assert out[1][:, t].tobytes() == out[0][:, 0].tobytes()
+
+
+# blocks of the fast build's visc kernel below and above its wide form's limit (256)
+@pytest.mark.parametrize("n, times", [((2, 2, 2), 257), ((8, 8, 8), 5), ((4, 16, 16), 2)],
+                         ids=lambda d: "x".join(map(str, d)) if isinstance(d, tuple) else str(d))
+def test_wide_and_narrow_blocks_agree(n, times):
+    for wall, eddy in ((False, False), (True, True)):
+        print(f"CASE test=wide_blocks n={n} times={times} wall={wall}", flush=True)
+        kw = dict(u_real=4, fast_math=1, flux="slau2", y_wall=wall, mu_ref=2e-3, viscosity_model=1)
+        length = [0.5 * d for d in n]  # powers of two times n: the same Jacobians in both boxes
+        u = smooth_state(*n, *length, seed=sum(n), amp=0.05, dtype=np.float32)
+        a, mu = u.reshape(5, n[2], -1), np.random.default_rng(2).uniform(0.0, 3e-3, (n[2], n[1] * n[0]))
+        out = []
+        for t in (1, times):
+            with od.Solver(od.params(n[0], n[1], n[2] * t, length[0], length[1], length[2] * t, **kw)) as s:
+                s.set_state(np.ascontiguousarray(np.tile(a, (1, t, 1))).ravel())
+                if eddy:
+                    s.set_eddy_viscosity(np.tile(mu, (t, 1)).ravel())
+                s.step(0.003, 3)
+                out.append(s.get_state().reshape(5, t, -1))
+        assert np.isfinite(out[0]).all()
+        for t in range(times):
+            assert out[1][:, t].tobytes() == out[0][:, 0].tobytes()
