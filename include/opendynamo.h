@@ -100,7 +100,9 @@ od_status od_release(od_ctx* ctx, uint64_t ticket);
 
 /* Enqueue n_steps RK3 steps of size dt (the f32 config value widened).
  * Asynchronous; replays of a captured 8-step hipGraph plus a 1-step one
- * (one 1-step replay per step while a closure network is attached). */
+ * (while a closure network is attached, whose refresh starts every interval:
+ * replays of one graph of a refresh and its interval's steps).  A new dt leaves
+ * the graphs valid. */
 od_status od_step(od_ctx* ctx, double dt, uint32_t n_steps);
 od_status od_synchronize(od_ctx* ctx);
 
@@ -289,7 +291,8 @@ od_status od_get_eddy_viscosity(od_ctx* ctx, void* host, size_t n, od_real dtype
 /* out[0] updates, out[1] updates that fell back on the budget check,
  * out[2] element-updates outside the training range, out[3] kinetic energy
  * at the last update, out[4] model dissipation rate at the last update,
- * out[5] 1 if the model is active for the current interval. */
+ * out[5] 1 if the model is active for the current interval.  Waits for the steps
+ * enqueued so far: the budget check runs on the device. */
 od_status od_closure_stats(od_ctx* ctx, double out[6]);
 
 #ifdef __cplusplus

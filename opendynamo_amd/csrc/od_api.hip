@@ -1,7 +1,9 @@
 // C-ABI front end of the HIP library (include/opendynamo.h).
 //
 // Owns the device buffers, the compute stream, an IO stream with three
-// pinned staging slots, and one captured hipGraph per RK3 step.  Replaces the
+// pinned staging slots, and the captured hipGraphs of one and eight RK3 steps
+// and of a closure interval, whose kernels read c * dt from a device table.
+// Replaces the
 // orchestration of drunkseal/opendynamo's src/solver.rs (context, NVRTC
 // module, operators, allocations, launch configs, the RK3 loop with its
 // buffer swap and the async D2H of the IO task).

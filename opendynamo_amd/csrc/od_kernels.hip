@@ -1,28 +1,35 @@
 // gfx950 kernels of the FR P=3 compressible Navier-Stokes RK3 step.
 //
 // Per RK stage (drunkseal/opendynamo: solver.rs:610-738, rhs.cu, rk.cu):
-//   od_visc_kernel    one wave64 per element: BR1-corrected gradient from the
-//                     element's LDS tile and its neighbours' stored face
-//                     traces, gradient face extrapolation, viscous normal flux
-//                     at the element's 6 faces -> fv  (replaces the gradient
-//                     half of compute_rhs_volume_kernel and the viscous half of
-//                     the face kernels)
-//                     In the fast f32 build it also forms the divergence of
-//                     the volume viscous fluxes (-> fv, after the face part)
-//   od_update_kernel  one wave64 per element: gradient again (register only;
-//                     not in the fast f32 build, which takes the volume
-//                     viscous divergence from the visc kernel), volume flux
-//                     divergence, interface fluxes at all 6 own
-//                     faces (SLAU2 / AUSM+ / Rusanov, slip wall), FR
-//                     correction, SSP-RK3 blend, face traces of the new state
-//                     (replaces the rest of the volume kernel, the x/y/wall/z
-//                     face kernels, the j arrays and rk_stage*_kernel)
-// Each face flux is evaluated by both elements that share the face, from the
-// same operands in the same order, so both sides see identical bits and no
-// face array, atomic or second pass is needed.
+//   viscous kernel    BR1-corrected gradient from the element's states and its
+//                     neighbours' face traces, gradient face extrapolation,
+//                     viscous normal flux at the element's 6 faces -> fv
+//                     (replaces the gradient half of compute_rhs_volume_kernel
+//                     and the viscous half of the face kernels), and, since it
+//                     holds the gradient, the volume part that needs it: the
+//                     divergence of the viscous fluxes (fast f32 build) or the
+//                     whole volume RHS (strict build) -> fv, after the face part
+//   update kernel     volume RHS (Euler mode: formed here; fast f32 build: the
+//                     divergence of the Euler fluxes here, plus the stored
+//                     viscous one), interface fluxes at all own faces
+//                     (SLAU2 / AUSM+ / Rusanov, slip wall), FR correction,
+//                     SSP-RK3 blend, face traces of the new state (replaces the
+//                     rest of the volume kernel, the x/y/wall/z face kernels,
+//                     the j arrays and rk_stage*_kernel)
+// Forms of both: tiles of two elements (od_visc_kernel, od_update_kernel), blocks
+// of 2x2x2 (fast: od_*_block_kernel; strict: od_visc_lines_block_kernel,
+// od_update_face_block_kernel), both in one launch for a box with an odd
+// dimension (od_*_core_shell_kernel), four consecutive elements (strict:
+// od_visc_line_kernel), and batches of boxes (od_batch_*).
+// A face flux is evaluated from the same operands in the same order wherever it
+// is formed, once for both elements inside a block, else by both elements that
+// share the face, so both sides see identical bits and no face array, atomic or
+// second pass is needed.
 //
-// Lane = solution point pt = i + 4j + 16k of the element.  Line contractions
-// stage through LDS.  The arithmetic of every quantity (association order,
+// Point-wise phases: lane = solution point pt = i + 4j + 16k of the element; by
+// lines: lane = line of four points (the viscous kernels on blocks and on four
+// elements).  Line contractions of point-wise phases stage through LDS.  The
+// arithmetic of every quantity in the strict build (association order,
 // no contraction: built with -ffp-contract=off) is that of the reference
 // kernel that computes it; comments cite the reference line.
 #include <hip/hip_runtime.h>
@@ -2661,8 +2668,9 @@ __device__ __forceinline__ void update_block_body(const StageArgs<float, float>&
 // gradient 6 to 8 times from LDS and formed the state's face traces twice: its
 // VALU instructions (753 per element's wave) took 78 % of the kernel's time and
 // its LDS reads about as much, at 6 waves to a SIMD.  By lines it is 8 waves
-// (63 VGPRs, 31 KB per work-group) and at 48^3 132 us a launch instead of 195
-// (0.51 GB moved, 82 us at the update kernel's 6.2 TB/s).
+// (64 VGPRs, 31 KB per work-group) and at 48^3 132 us a launch instead of 195
+// (0.51 GB moved, 82 us at the update kernel's 6.2 TB/s; 126 us with the even
+// and odd parts, see line_even).
 // Every value is the same expression as in visc_body.
 //
 // LDS: one area per element, first its state [5][64], then, once every line has
