@@ -1723,10 +1723,10 @@ __global__ __launch_bounds__(128) void od_visc_kernel(StageArgs<UT, CT> a) {
 
 // Occupancy target of the update kernels.  The fast all-f32 single-box kernel
 // and the batch kernel's single-unit form are held to 64 VGPRs (8 waves per
-// SIMD; they need 61 with no spills; their LDS, 9.1 KB per work-group, allows
-// 8).  The strict build (70 VGPRs, 7 waves), f64 states and the persistent batch
-// kernel keep their natural allocation (the 4-wave cap does not bind); f64
-// compute needs 120 VGPRs (4 waves).
+// SIMD; they need 53 to 57 with no spills; their LDS, 9.7 KB per work-group of
+// 128 threads, allows 8).  The strict build (70 VGPRs, 7 waves), f64 states and
+// the persistent batch kernel keep their natural allocation (the 4-wave cap does
+// not bind); f64 compute needs 115 to 122 VGPRs (4 waves).
 template <class CT>
 constexpr int kMinWaves = sizeof(CT) == 4 ? 4 : 1;
 template <class UT, class CT>
@@ -3090,7 +3090,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8))) void o
 // 33x25x37 visc 41.5 against 39.2 us, update 43.8 against 43.4 us); a launch of
 // its own would cost its latency twice a stage.  The update kernel walks the
 // blocks backwards, as in the even boxes.  33x25x37 (AUSM+, 100 steps): 37.4 ms
-// with every element on tiles, 29.5 so.
+// with every element on tiles, 29.0 so.
 struct CoreShell {
     int32_t n_blocks, n_tiles;  // blocks of the core, tiles of the shell
 };
