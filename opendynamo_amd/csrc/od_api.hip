@@ -139,22 +139,20 @@ using namespace od::host;
 
 namespace {
 
-constexpr double kTableDt = 0.0;  // no dt of its own: c * dt from od_ctx::dt_table
-
+// dt null: a captured step, which reads c * dt from the context's table.
 template <class UT, class CT>
-od::StageArgs<UT, CT> stage_args(od_ctx* c, int stage, double dt) {
+od::StageArgs<UT, CT> stage_args(od_ctx* c, int stage, const double* dt) {
     od::StageArgs<UT, CT> a = make_stage_args<UT, CT>(c->p, c->p.nx, c->p.ny, c->p.nz, c->p.lx, c->p.ly, c->p.lz,
-                                                      c->u, c->tr, c->fv, c->dbg, stage, dt);
+                                                      c->u, c->tr, c->fv, c->dbg, stage, dt ? *dt : 0.0);
     a.ops = c->box_ops;
     a.mu_t = c->mu_t_on ? (const CT*)c->mu_t : nullptr;
-    // a captured step (dt 0) reads c * dt from the context's table
-    if (dt == kTableDt) a.dt = (const od::StageDt<UT, CT>*)c->dt_table + stage;
+    if (!dt) a.dt = (const od::StageDt<UT, CT>*)c->dt_table + stage;
     return a;
 }
 
 // kind: 0 = visc, 1 = update, 2 = trace (of u0 into tr[0])
 template <class UT, class CT>
-int launch_kind(od_ctx* c, int kind, int stage, double dt, int mode) {
+int launch_kind(od_ctx* c, int kind, int stage, const double* dt, int mode) {
     od::StageArgs<UT, CT> a = stage_args<UT, CT>(c, stage, dt);
     a.mode = mode;
     if (kind == 2) {
@@ -194,7 +192,7 @@ const char* kernel_name(const od_params& p, int kind) {
     return fast_kernels(p) ? "od_visc_kernel" : "od_visc_line_kernel";
 }
 
-int launch(od_ctx* c, int kind, int stage, double dt, int mode = 0) {
+int launch(od_ctx* c, int kind, int stage, const double* dt, int mode = 0) {
     const bool uf = c->p.u_real == OD_F32, cf = c->p.compute_real == OD_F32;
     if (uf && cf) return launch_kind<float, float>(c, kind, stage, dt, mode);
     if (!uf && !cf) return launch_kind<double, double>(c, kind, stage, dt, mode);
@@ -202,10 +200,10 @@ int launch(od_ctx* c, int kind, int stage, double dt, int mode = 0) {
     return launch_kind<float, double>(c, kind, stage, dt, mode);
 }
 
-od_status enqueue_step(od_ctx* c, double dt) {
+od_status enqueue_step(od_ctx* c) {
     for (int s = 0; s < 3; ++s) {
-        if (c->p.viscous && launch(c, 0, s, dt)) return fail(OD_ERR_HIP, "od_visc_kernel launch failed");
-        if (launch(c, 1, s, dt)) return fail(OD_ERR_HIP, "od_update_kernel launch failed");
+        if (c->p.viscous && launch(c, 0, s, nullptr)) return fail(OD_ERR_HIP, "od_visc_kernel launch failed");
+        if (launch(c, 1, s, nullptr)) return fail(OD_ERR_HIP, "od_update_kernel launch failed");
     }
     return OD_OK;
 }
@@ -221,7 +219,7 @@ od_status capture_steps(od_ctx* c, bool refresh, uint32_t steps, hipGraphExec_t*
     hipGraph_t g = nullptr;
     HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     od_status s = refresh ? od_closure_refresh_internal(c) : OD_OK;
-    for (uint32_t q = 0; q < steps && s == OD_OK; ++q) s = enqueue_step(c, kTableDt);
+    for (uint32_t q = 0; q < steps && s == OD_OK; ++q) s = enqueue_step(c);
     hipError_t e = hipStreamEndCapture(c->stream, &g);
     if (s != OD_OK) {
         if (g) (void)hipGraphDestroy(g);
@@ -251,14 +249,12 @@ int write_dt(od_ctx* c, double dt) {
 // The dt of the steps enqueued from here on, written in stream order (steps
 // already enqueued keep theirs).
 od_status set_dt(od_ctx* c, double dt) {
-    if (c->table_dt == dt) return OD_OK;
+    if (c->table_set && c->table_dt == dt) return OD_OK;
     const bool uf = c->p.u_real == OD_F32, cf = c->p.compute_real == OD_F32;
     const int rc = uf ? (cf ? write_dt<float, float>(c, dt) : write_dt<float, double>(c, dt))
                       : (cf ? write_dt<double, float>(c, dt) : write_dt<double, double>(c, dt));
-    if (rc) {
-        c->table_dt = 0.0;
-        return fail(OD_ERR_HIP, "od_set_dt_kernel launch failed");
-    }
+    c->table_set = rc == 0;
+    if (rc) return fail(OD_ERR_HIP, "od_set_dt_kernel launch failed");
     c->table_dt = dt;
     return OD_OK;
 }
@@ -469,7 +465,8 @@ od_status od_set_state(od_ctx* c, const void* host, size_t n, od_real dtype) {
         src = tmp.data();
     }
     HIP_TRY(hipMemcpyAsync(c->u[0], src, n * c->ubytes, hipMemcpyHostToDevice, c->stream));
-    if (launch(c, 2, 0, 0.0)) return fail(OD_ERR_HIP, "od_trace_kernel launch failed");
+    const double no_dt = 0.0;
+    if (launch(c, 2, 0, &no_dt)) return fail(OD_ERR_HIP, "od_trace_kernel launch failed");
     HIP_TRY(hipStreamSynchronize(c->stream));
     c->state_set = true;
     return OD_OK;
@@ -582,8 +579,9 @@ od_status od_rhs(od_ctx* c, void* host_out, size_t n) {
         c->device_bytes += (size_t)5 * c->NP * c->cbytes;
     }
     // stage-1 operands: uin = u0, tr_in = tr[0]; mode 1 writes the corrected RHS
-    if (c->p.viscous && launch(c, 0, 0, 1.0)) return fail(OD_ERR_HIP, "od_visc_kernel launch failed");
-    if (launch(c, 1, 0, 1.0, 1)) return fail(OD_ERR_HIP, "od_update_kernel launch failed");
+    const double dt = 1.0;  // not used in this mode
+    if (c->p.viscous && launch(c, 0, 0, &dt)) return fail(OD_ERR_HIP, "od_visc_kernel launch failed");
+    if (launch(c, 1, 0, &dt, 1)) return fail(OD_ERR_HIP, "od_update_kernel launch failed");
     HIP_TRY(hipMemcpyAsync(host_out, c->dbg, n * c->cbytes, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     return OD_OK;
@@ -665,7 +663,7 @@ od_status od_time_kernels(od_ctx* c, double dt, uint32_t n_steps, double out_ms[
                 od_status st = rec(kind);
                 if (st != OD_OK) return st;
                 HIP_TRY(hipEventRecord(ev[ev.size() - 2], c->stream));
-                if (launch(c, kind, s, dt)) return fail(OD_ERR_HIP, "kernel launch failed");
+                if (launch(c, kind, s, &dt)) return fail(OD_ERR_HIP, "kernel launch failed");
                 HIP_TRY(hipEventRecord(ev.back(), c->stream));
             }
     HIP_TRY(hipStreamSynchronize(c->stream));

@@ -40,7 +40,8 @@ struct od_ctx {
     double* dt_value = nullptr;        // dt on the device, and behind it
     od::BoxOps* box_ops = nullptr;     // the fast kernels' operators
     void* dt_table = nullptr;          // StageDt[3] that the graphs' kernels read
-    double table_dt = 0.0;             // the dt it holds (in stream order), 0: none yet
+    bool table_set = false;            // whether it has been written (no dt of its own says so: every dt may be asked for)
+    double table_dt = 0.0;             // the dt it holds (in stream order)
     void* pinned[3] = {nullptr, nullptr, nullptr};
     hipEvent_t slot_done[3] = {nullptr, nullptr, nullptr};
     // Device copies of the snapshots (allocated at the first snapshot): the
