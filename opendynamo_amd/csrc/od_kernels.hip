@@ -86,16 +86,25 @@ __device__ __forceinline__ C sq(C x) {
 
 // A denominator that several quotients share.  In the strict build its
 // reciprocal is formed once, in f64 (v_rcp_f64 to 24 bits, then the cubic
-// iteration y (1 + e + e^2), e = 1 - b y: within 2^-52 of 1 / b), and each
-// quotient is the correctly rounded a / b in three or four more instructions:
-//   f32  a y in f64, rounded to f32.  The quotient of two 24-bit numbers lies
-//        2^-49 of itself or more from the middle between two f32 numbers, a y
-//        within 2^-51.5 of it, so the rounding is that of a / b.
+// iteration y (1 + e + e^2), e = 1 - b y), and each quotient is the correctly
+// rounded a / b in three or four more instructions:
+//   f32  q = a y in f64, its last three bits cleared, rounded to f32.  A quotient
+//        of two 24-bit numbers in [2^e, 2^(e+1)) that is not itself the middle
+//        between two f32 numbers lies 2^(e-48) or more from it.  Where the
+//        quotient is subnormal it can be the middle, which has few bits; a y a
+//        hair beside it would then round the wrong way.  So y is 2^-51 of itself
+//        too large (the 1 in e is 1 + 2^-51): with y and q each rounded to within
+//        2^-53 of themselves q exceeds the quotient by 1 to 3 2^-52 of it, less
+//        than the 2^(e-49) that clearing takes off, and is a middle again exactly
+//        where the quotient is one.
 //   f64  q = a y, then one correction with the residual a - b q, exact in an
 //        FMA (Markstein, IBM J. Res. Dev. 34, 1990: the last steps of the
-//        compiler's own a / b).  v_div_fixup gives zeros, infinities and NaN
-//        their IEEE results; |a| between 0 and 2^-969 may be off by one unit
-//        in the last place.
+//        compiler's own a / b; his theorem asks for y rounded correctly, which
+//        one b in 700,000 misses: 10^7 quotients by 37,000 such b, those nearest
+//        the middle between two numbers, all came out right).  v_div_fixup gives
+//        zeros, infinities and NaN their IEEE results; |a| between 0 and 2^-969
+//        may be off by one unit in the last place, and b below 2^-1022 or above
+//        2^1021, whose reciprocal is not a normal number, is not covered.
 // A division takes 46 (f32) and 65 (f64) cycles of a SIMD, a quotient 14 and
 // 20, a reciprocal 37; a point has about 90 quotients by some ten
 // denominators, which were nearly half of the strict kernels' instructions.
@@ -105,12 +114,14 @@ struct Recip {
     double y;
 };
 template <class C>
+constexpr double kRecipOne = sizeof(C) == 8 ? 1.0 : 1.0 + 0x1p-51;
+template <class C>
 __device__ __forceinline__ Recip<C> recip(C b) {
 #if OD_FAST
     return {b, 0.0};  // quot takes v_rcp_f32 as dv does
 #else
     const double d = (double)b, y0 = __builtin_amdgcn_rcp(d);
-    const double e = __builtin_fma(-d, y0, 1.0);
+    const double e = __builtin_fma(-d, y0, kRecipOne<C>);
     const double y = __builtin_fma(__builtin_fma(e, e, e), y0, y0);
     if constexpr (sizeof(C) == 8) return {b, y};
     return {b, e == e ? y : y0};  // b zero or infinite: y0 is infinite or zero, and e NaN
@@ -125,7 +136,7 @@ __device__ __forceinline__ C quot(C a, Recip<C> r) {
         const double q = a * r.y;
         return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-r.b, q, a), r.y, q), r.b, a);
     }
-    return (C)((double)a * r.y);
+    return (C)__longlong_as_double(__double_as_longlong((double)a * r.y) & ~7LL);
 #endif
 }
 
@@ -352,7 +363,7 @@ __device__ __forceinline__ C sound_speed(C p, Recip<C> ir) {
     }
 #endif
     // by max(1e-7, rho): rho's reciprocal, or that of the constant
-    const Recip<C> im = rho >= (C)1e-7 ? ir : Recip<C>{(C)1e-7, 1.0 / (double)(C)1e-7};
+    const Recip<C> im = rho >= (C)1e-7 ? ir : Recip<C>{(C)1e-7, kRecipOne<C> / (double)(C)1e-7};
     return sq(fmax(((C)0.0), quot(((C)1.4) * p, im)));
 }
 
