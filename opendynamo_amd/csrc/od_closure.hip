@@ -16,7 +16,6 @@
 #include <algorithm>
 #include <cmath>
 #include <cstddef>
-#include <cstdlib>
 #include <cstring>
 #include <memory>
 #include <mutex>
@@ -25,6 +24,7 @@
 #include <vector>
 
 #include "od_ctx.hpp"
+#include "od_order.hpp"
 
 using namespace od::host;
 
@@ -834,26 +834,6 @@ struct EpochSlot {
     }
 };
 
-// x mod d for d <= n without a 64-bit division: q = the high half of x times
-// floor((2^64 - 1) / d) is floor(x / d) or one less.  An epoch's shuffle takes
-// one modulus per sample, with the same n - 1 divisors every time.
-struct ModTable {
-    uint64_t* inv = nullptr;
-    ModTable() = default;
-    ModTable(const ModTable&) = delete;
-    ModTable& operator=(const ModTable&) = delete;
-    ~ModTable() { std::free(inv); }
-    void fill(size_t n) {
-        inv = (uint64_t*)std::malloc((n + 1) * sizeof(uint64_t));
-        for (size_t d = 1; inv && d <= n; ++d) inv[d] = ~(uint64_t)0 / d;
-    }
-    size_t mod(uint64_t x, size_t d) const {
-        if (!inv) return (size_t)(x % d);
-        const uint64_t r = x - (uint64_t)(((unsigned __int128)x * inv[d]) >> 64) * d;
-        return (size_t)(r >= d ? r - d : r);
-    }
-};
-
 // Gradient of the mean squared error over n gathered samples; grad and the
 // sum of squared errors in m->grad (device).  With `adam` the parameters take
 // their step in the same launch as the sum over the groups.
@@ -1191,7 +1171,6 @@ od_status od_mlp_train(od_mlp* m, const float* x, const float* t, size_t n, uint
     const size_t n_batches = (n + batch - 1) / batch;
     DevBuf dx, dt;
     EpochSlot slot[2];
-    ModTable mod;
     HIP_TRY(hipMalloc(&dx.p, n * NF * sizeof(float)));
     HIP_TRY(hipMalloc(&dt.p, n * sizeof(float)));
     for (EpochSlot& q : slot) {
@@ -1203,8 +1182,7 @@ od_status od_mlp_train(od_mlp* m, const float* x, const float* t, size_t n, uint
     }
     HIP_TRY(hipMemcpyAsync(dx.p, x, n * NF * sizeof(float), hipMemcpyHostToDevice, m->stream));
     HIP_TRY(hipMemcpyAsync(dt.p, t, n * sizeof(float), hipMemcpyHostToDevice, m->stream));
-    if (epochs > 1) mod.fill(n);
-    std::mt19937_64 rng(seed);
+    od::SampleOrder order(n, seed, epochs > 1);
     // waits for the epoch in slot q and takes its loss
     auto finish = [&](EpochSlot& q) -> od_status {
         if (!q.busy) return OD_OK;
@@ -1218,11 +1196,8 @@ od_status od_mlp_train(od_mlp* m, const float* x, const float* t, size_t n, uint
     auto run_epoch = [&](EpochSlot& q, uint32_t ep) -> od_status {
         od_status s = finish(q);
         if (s != OD_OK) return s;
-        int* perm = q.host_idx;
-        for (size_t k = 0; k < n; ++k) perm[k] = (int)k;
-        for (size_t k = n - 1; k > 0; --k)  // Fisher-Yates with the seeded generator
-            std::swap(perm[k], perm[mod.mod(rng(), k + 1)]);
-        HIP_TRY(hipMemcpyAsync(q.idx, perm, n * sizeof(int), hipMemcpyHostToDevice, m->stream));
+        order.next(q.host_idx);
+        HIP_TRY(hipMemcpyAsync(q.idx, q.host_idx, n * sizeof(int), hipMemcpyHostToDevice, m->stream));
         for (size_t b0 = 0, k = 0; b0 < n; b0 += batch, ++k) {
             const uint64_t at = m->adam_t + 1;
             const Adam ad{m->params,
