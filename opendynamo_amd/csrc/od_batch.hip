@@ -67,7 +67,7 @@ bool f32_compute(const od_batch* b) { return b->p.compute_real == OD_F32; }
 // all even, else the box less its last layer along each odd dimension, whose
 // elements (the shell) run on two-element tiles.  Blocks and tiles give the
 // same bits for every face, so every box still equals the same box run alone.
-bool core_box(const od_batch* b, const od_box& x) { return box_form(b->p, x.nx, x.ny, x.nz) != BoxForm::tiles; }
+bool core_box(const od_batch* b, const od_box& x) { return block_core(b->p, x.nx, x.ny, x.nz); }
 int64_t tile_count(const od_batch* b, const od_box& x, int orient) {
     return core_box(b, x) ? od::shell_tiles(x.nx, x.ny, x.nz) : box_tiles(x, orient);
 }
@@ -104,7 +104,7 @@ int box_launch_t(od_batch* b, int i, int kind, int stage, double dt) {
         return od::launch_trace<UT, CT>(a, E, b->stream);
     }
     if constexpr (sizeof(UT) == 4 && sizeof(CT) == 4) {
-        if (core_box(b, b->boxes[i]))  // as od_step runs this box alone
+        if (core_box(b, b->boxes[i]))  // not tiles, which read the traces of the core's internal faces too
             return launch_block_form(a, b->p.viscous != 0, kind, b->stream);
     }
     if constexpr (sizeof(CT) == 4) {

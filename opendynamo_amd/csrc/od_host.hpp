@@ -46,15 +46,30 @@ od::Ops<C> cast_ops(const HostOps& h) {
 // Whether a context's kernels are the fast build's: f32 compute with fast_math.
 inline bool fast_kernels(const od_params& p) { return p.fast_math && p.compute_real == OD_F32; }
 
-// The kernels a box runs on when it is stepped by itself: fast f32 boxes at
-// least 2 elements wide in each direction on 2x2x2-element blocks, with the
-// last layer along each odd dimension on two-element tiles in the same launch;
-// all others on tiles.
+// Whether the kernels on 2x2x2-element blocks take a box's core: fast f32, at
+// least 2 elements wide in each direction.
+inline bool block_core(const od_params& p, int nx, int ny, int nz) {
+    return p.fast_math && p.u_real == OD_F32 && p.compute_real == OD_F32 && nx >= 2 && ny >= 2 && nz >= 2;
+}
+// The kernels of a box that is a context of its own: boxes with a block core on
+// blocks, with the last layer along each odd dimension on two-element tiles in
+// the same launch; all others, and small boxes with an odd dimension, on tiles.
+// Those are over with their longest work-group, which a block and a tile of the
+// shell in one launch make longer than a tile is, above all beside the update
+// kernel's wide form (512 tiles).  us a step, tiles against core and shell:
+//   viscous  3^3 (18 tiles) 30.3 39.0, 9^3 (405) 38.5 43.9, 3x16x16 (512) 38.9
+//            44.3, 8x17x8 (544) 46.0 44.4, 16x5x16 (640) 44.3 45.9, 11^3 (726)
+//            47.4 47.6, 12x13x12 (936) 52.2 50.2, 13^3 (1183) 55.2 56.8, 15^3
+//            (1800) 69 62
+//   Euler    3^3 13.1 18.8, 9^3 15.9 20.2, 11^3 20.3 21.1, 13^3 22.9 24.7, 30x3x30
+//            (1350) 24.9 25.2, 33x3x33 (1683) 27.2 26.3, 15^3 26.9 26.3, 16x16x17
+//            (2176) 31.2 32.4, 17^3 (2601) 35.2 33.4
 enum class BoxForm { tiles, blocks, core_shell };
 inline BoxForm box_form(const od_params& p, int nx, int ny, int nz) {
-    if (!p.fast_math || p.u_real != OD_F32 || p.compute_real != OD_F32 || nx < 2 || ny < 2 || nz < 2)
-        return BoxForm::tiles;
-    return nx % 2 || ny % 2 || nz % 2 ? BoxForm::core_shell : BoxForm::blocks;
+    if (!block_core(p, nx, ny, nz)) return BoxForm::tiles;
+    if (nx % 2 == 0 && ny % 2 == 0 && nz % 2 == 0) return BoxForm::blocks;
+    const int64_t tiles = (int64_t)((nx + 1) / 2) * ny * nz;
+    return tiles <= (p.viscous ? 512 : 1500) ? BoxForm::tiles : BoxForm::core_shell;
 }
 // Whether a strict viscous box runs on 2x2x2-element blocks when it is a context
 // of its own (a batch's boxes all run on tiles): even dimensions, and two and a
@@ -68,7 +83,7 @@ inline bool strict_blocks(const od_params& p) {
     return !fast_kernels(p) && p.viscous && p.nx % 2 == 0 && p.ny % 2 == 0 && p.nz % 2 == 0 &&
            (int64_t)p.nx * p.ny * p.nz >= 8 * kStrictBlocks;
 }
-// Launch of kind 0 visc, 1 update of a box whose form is not tiles.
+// Launch of kind 0 visc, 1 update of a box with a block core: blocks, or core and shell.
 int launch_block_form(const od::StageArgs<float, float>& a, bool viscous, int kind, hipStream_t stream);
 
 inline bool real_ok(int r) { return r == OD_F32 || r == OD_F64; }
