@@ -45,6 +45,8 @@ struct od_batch {
     int table_orient = -1;
     int64_t n_tiles[3] = {0, 0, 0};  // tiles (boxes on tiles, shells of the others), per orientation
     int64_t n_blocks = 0;            // 2x2x2-element blocks of the boxes' cores
+    bool small_odd = false;          // some box has a block core, but runs on tiles by itself
+    bool core_faces_stale = false;   // tr[0] lacks those boxes' internal faces of the core (see before_steps)
     hipGraphExec_t graph = nullptr;
     int cu_count = 0;
     size_t device_bytes = 0;
@@ -104,7 +106,8 @@ int box_launch_t(od_batch* b, int i, int kind, int stage, double dt) {
         return od::launch_trace<UT, CT>(a, E, b->stream);
     }
     if constexpr (sizeof(UT) == 4 && sizeof(CT) == 4) {
-        if (core_box(b, b->boxes[i]))  // not tiles, which read the traces of the core's internal faces too
+        const od_box& x = b->boxes[i];
+        if (box_form(b->p, x.nx, x.ny, x.nz) != BoxForm::tiles)  // as od_step runs this box alone
             return launch_block_form(a, b->p.viscous != 0, kind, b->stream);
     }
     if constexpr (sizeof(CT) == 4) {
@@ -335,7 +338,11 @@ od_status check_schedule(const od_schedule* s) {
     return OD_OK;
 }
 
+od_status before_steps(od_batch* b, bool per_box);
+
 od_status time_graph(od_batch* b, uint32_t n_steps, double* ms) {
+    od_status st = before_steps(b, b->sched.order == 2);
+    if (st != OD_OK) return st;
     hipEvent_t e0, e1;
     HIP_TRY(hipEventCreate(&e0));
     HIP_TRY(hipEventCreate(&e1));
@@ -355,6 +362,19 @@ od_status time_graph(od_batch* b, uint32_t n_steps, double* ms) {
 od_status retrace_all(od_batch* b) {
     for (size_t i = 0; i < b->boxes.size(); ++i)
         if (box_launch(b, (int)i, 2, 0, 0.0)) return fail(OD_ERR_HIP, "od_trace_kernel launch failed");
+    b->core_faces_stale = false;
+    return OD_OK;
+}
+
+// Before steps on the batch's stream.  Box by box (schedule order 2, per-box
+// timing) a small box with an odd dimension runs on tiles, which read the traces
+// of every face of tr[0]; batched steps leave its core's internal faces out of
+// it (the block kernels form those from the state), so after batched steps they
+// are formed again from u0 first, with the arithmetic of the update kernels'
+// trace stores.
+od_status before_steps(od_batch* b, bool per_box) {
+    if (per_box && b->core_faces_stale) return retrace_all(b);
+    if (!per_box && b->small_odd) b->core_faces_stale = true;
     return OD_OK;
 }
 
@@ -420,7 +440,9 @@ od_status od_batch_create(const od_params* p, const od_box* boxes, int32_t n_box
     for (int o = 0; o < 3; ++o)
         for (int i = 0; i < n_boxes; ++i) b->n_tiles[o] += tile_count(b, boxes[i], o);
     for (int i = 0; i < n_boxes; ++i) {
-        b->n_blocks += block_count(b, boxes[i]);
+        const od_box& x = boxes[i];
+        b->n_blocks += block_count(b, x);
+        b->small_odd = b->small_odd || (core_box(b, x) && box_form(b->p, x.nx, x.ny, x.nz) == BoxForm::tiles);
     }
     if (b->n_blocks * 512 > (int64_t)0xffffffff)
         return cleanup(fail(OD_ERR_INVALID, "batch too large for one launch grid"));
@@ -532,7 +554,9 @@ od_status od_batch_step(od_batch* b, const double* dt, uint32_t n_steps) {
     if (s == OD_OK) s = ready(b, "od_batch_step");
     if (s != OD_OK) return s;
     HIP_TRY(hipSetDevice(b->device));
-    if ((s = ensure_table(b, dt)) != OD_OK || (s = ensure_graph(b)) != OD_OK) return s;
+    if ((s = ensure_table(b, dt)) != OD_OK || (s = ensure_graph(b)) != OD_OK ||
+        (s = before_steps(b, b->sched.order == 2)) != OD_OK)
+        return s;
     for (uint32_t q = 0; q < n_steps; ++q) HIP_TRY(hipGraphLaunch(b->graph, b->stream));
     return OD_OK;
 }
@@ -653,6 +677,7 @@ od_status od_batch_autotune(od_batch* b, const double* dt, uint32_t steps_per_tr
             (st = ensure_graph(b)) != OD_OK)
             return done(st);
         double ms = 0.0;
+        if ((st = before_steps(b, c.order == 2)) != OD_OK) return done(st);
         if (hipGraphLaunch(b->graph, b->stream) != hipSuccess)
             return done(fail(OD_ERR_HIP, "od_batch_autotune: graph launch failed"));
         if ((st = time_graph(b, steps_per_trial, &ms)) != OD_OK) return done(st);
@@ -687,6 +712,7 @@ od_status od_batch_time_steps(od_batch* b, const double* dt, uint32_t n_steps, i
         if ((st = ensure_table(b, dt)) != OD_OK || (st = ensure_graph(b)) != OD_OK) return st;
         return time_graph(b, n_steps, ms_total);
     }
+    if ((st = before_steps(b, true)) != OD_OK) return st;
     hipEvent_t e0, e1;
     HIP_TRY(hipEventCreate(&e0));
     HIP_TRY(hipEventCreate(&e1));

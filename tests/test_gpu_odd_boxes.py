@@ -67,3 +67,33 @@ def test_tiles_equal_core_and_shell(n, times, viscous):
                 assert np.isfinite(a).all()
                 wrong = np.count_nonzero(repeated(a, n, times).view(np.uint32) != b.view(np.uint32))
                 assert wrong == 0, wrong
+
+
+def test_boxes_of_a_batch_switch_between_their_forms():
+    """Box by box a small odd box runs on tiles, in batched steps its core on blocks,
+    which leave out the core's internal traces; larger odd boxes and even ones keep
+    their form.  Every box follows the box run alone, however the steps are made."""
+    print("CASE test=odd_boxes_batch", flush=True)
+    kw = dict(u_real=od.OD_F32, y_wall=True, viscosity_model=1, mu_ref=2e-3, fast_math=1)
+    boxes = [(3, 3, 3, 1.5, 1.5, 1.5), (5, 19, 9, 2.5, 9.5, 4.5), (4, 4, 2, 2.0, 2.0, 1.0), (1, 5, 3, 0.5, 2.5, 1.5),
+             (2, 5, 4, 1.0, 2.5, 2.0)]
+    inits = [smooth_state(*x, seed=q, amp=0.04, dtype=np.float32) for q, x in enumerate(boxes)]
+    plan = [(0, 2), (2, 1), (1, 1), (2, 2), (0, 1), (0, 1), (2, 1)]
+    with od.Batch(od.params(1, 1, 1, 1.0, 1.0, 1.0, **kw), boxes) as b:
+        for q, u in enumerate(inits):
+            b.set_state(q, u)
+        for order, n in plan:
+            b.set_schedule(order=order)
+            b.step(0.003, n)
+        b.set_schedule(order=0)
+        b.time_steps(0.003, 2)
+        b.time_steps(0.003, 1, per_box=True)
+        b.step(0.003, 1)
+        got = [b.get_state(q) for q in range(len(boxes))]
+    for q, x in enumerate(boxes):
+        with od.Solver(od.params(*x, **kw)) as s:
+            s.set_state(inits[q])
+            s.step(0.003, sum(n for _, n in plan) + 4)
+            want = s.get_state()
+        assert np.isfinite(want).all()
+        assert np.array_equal(got[q].view(np.uint32), want.view(np.uint32)), x
