@@ -734,16 +734,21 @@ __device__ __forceinline__ void coef_store(int tid, C v) {
     if (tid < kCoefs<C>) reinterpret_cast<C*>(&coef_lds<C>())[tid] = v;
 }
 #if OD_FAST
-// The same for a tile's own copy, by its 128 threads.
-template <class UT>
+// The same for a tile's own copy, by its 128 threads: the visc kernel's with the
+// coefficients of the lines' derivatives (TileTable), the update kernel's, which
+// takes none, without (BoxTable).
+template <class Table>
+constexpr int kTableValues = (sizeof(BoxTable) + (std::is_same<Table, TileTable>::value ? sizeof(BoxOps::line) : 0)) / sizeof(float);
+template <class Table, class UT>
 __device__ __forceinline__ float tile_table_load(const StageArgs<UT, float>& a, int tid) {
-    constexpr int kRows = sizeof(BoxTable) / sizeof(float), kLine = sizeof(BoxOps::line) / sizeof(float);
-    static_assert(kRows + kLine <= 128 && sizeof(TileTable) >= (kRows + kLine) * sizeof(float), "one value a thread");
+    constexpr int kRows = kTableValues<BoxTable>, kAll = kTableValues<Table>;
+    static_assert(kAll <= 128 && sizeof(Table) >= kAll * sizeof(float), "one value a thread");
     const float* src = tid < kRows ? a.ops->table + tid : &a.ops->line[0][0].ps + (tid - kRows);
-    return tid < kRows + kLine ? *src : 0.f;
+    return tid < kAll ? *src : 0.f;
 }
-__device__ __forceinline__ void tile_table_store(TileTable& t, int tid, float v) {
-    if (tid < (int)((sizeof(BoxTable) + sizeof(BoxOps::line)) / sizeof(float))) reinterpret_cast<float*>(&t)[tid] = v;
+template <class Table>
+__device__ __forceinline__ void tile_table_store(Table& t, int tid, float v) {
+    if (tid < kTableValues<Table>) reinterpret_cast<float*>(&t)[tid] = v;
 }
 #endif
 template <class C>
@@ -1442,11 +1447,9 @@ struct UpdateLds {
     CT sJ_own[kPF ? 0 : kEpb][6][5][16];  // zero-length when aliased
     CT sF[kVol ? kEpb : 0][5][64];
 #if OD_FAST
-    TileTable tab;  // of the tile's box: a batch's work-group may have tiles of two boxes
+    BoxTable tab;  // of the tile's box: a batch's work-group may have tiles of two boxes
     __device__ const BoxTable& rows() { return tab; }
-    __device__ const TileTable& tile_table() { return tab; }
 #else
-    __device__ TileTable tile_table() { return {}; }
     __device__ const CoefTable<CT>& rows() { return coef_lds<CT>(); }
 #endif
     __device__ CT (*sJ())[6][5][16] {
@@ -1480,7 +1483,7 @@ __device__ __forceinline__ void visc_body(const StageArgs<UT, CT>& a, const Tile
     const int64_t NP = (int64_t)a.nx * a.ny * a.nz * 64;
     const CT cf = coef_load(a, (int)threadIdx.x);
 #if OD_FAST
-    const float row = tile_table_load(a, wave * 64 + pt);
+    const float row = tile_table_load<TileTable>(a, wave * 64 + pt);
 #endif
     if constexpr (PF) prefetch_issue<false>(a, tl, L.pf, wave, pt);
     if (tile_valid(tl, wave)) load_state_tile(a.uin, NP, tile_eidx(tl, wave), L.sU[wave], pt);
@@ -1580,7 +1583,7 @@ __device__ __forceinline__ void update_body(const StageArgs<UT, CT>& a, const Ti
     const int64_t gbase = tile_eidx(tl, wave) * 64 + pt;
     const CT cf = coef_load(a, (int)threadIdx.x);
 #if OD_FAST
-    const float row = tile_table_load(a, wave * 64 + pt);
+    const float row = tile_table_load<BoxTable>(a, wave * 64 + pt);
 #endif
     if constexpr (PF) {
         if (owner) prefetch_issue<true>(a, tl, L.pf, wave, pt);
@@ -1734,7 +1737,7 @@ __global__ __launch_bounds__(128) void od_visc_kernel(StageArgs<UT, CT> a) {
 
 // Occupancy target of the update kernels.  The fast all-f32 single-box kernel
 // and the batch kernel's single-unit form are held to 64 VGPRs (8 waves per
-// SIMD; they need 53 to 57 with no spills; their LDS, 9.7 KB per work-group of
+// SIMD; they need 53 to 57 with no spills; their LDS, 9.6 KB per work-group of
 // 128 threads, allows 8).  The strict build (70 VGPRs, 7 waves), f64 states and
 // the persistent batch kernel keep their natural allocation (the 4-wave cap does
 // not bind); f64 compute needs 115 to 122 VGPRs (4 waves).
@@ -3095,7 +3098,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8))) void o
 // One box with an odd dimension: its core on blocks and its shell on tiles in
 // one launch.  A 512-thread work-group takes a block of the core, or as many
 // tiles of the shell as fit its threads and a block's LDS: three in the visc
-// kernel (10.6 KB each), four in the update kernel (9.4 KB).  The shell, a small
+// kernel (10.6 KB each), four in the update kernel (9.2 KB).  The shell, a small
 // part of the box, whose tiles take longest from start to end, comes first in
 // both, so that the blocks cover it (after the blocks it ended the launch alone:
 // 33x25x37 visc 41.5 against 39.2 us, update 43.8 against 43.4 us); a launch of
