@@ -40,9 +40,12 @@ def test_form_of_an_odd_box(n, viscous, on_tiles):
     assert update_kernel(p) == ("od_update_kernel" if on_tiles else "od_update_core_shell_kernel")
 
 
-# boxes of 18, 45 and 10 tiles; as many times as gives core and shell
+# every combination of odd directions, as many times as gives core and shell; shells
+# with every remainder of a work-group's three and four tiles
 @pytest.mark.parametrize("n,times", [((3, 3, 3), (11, 1, 11)), ((3, 5, 3), (11, 1, 9)), ((2, 3, 2), (17, 1, 31)),
-                                     ((4, 5, 2), (15, 1, 11)), ((1, 3, 1), (33, 1, 35)), ((1, 2, 5), (33, 1, 11))],
+                                     ((4, 5, 2), (15, 1, 11)), ((1, 3, 1), (33, 1, 35)), ((1, 2, 5), (33, 1, 11)),
+                                     ((3, 2, 2), (21, 1, 13)), ((2, 2, 3), (31, 1, 11)), ((3, 3, 2), (21, 1, 13)),
+                                     ((2, 3, 3), (21, 1, 11))],
                          ids=lambda d: "x".join(map(str, d)))
 @pytest.mark.parametrize("viscous", [True, False])
 def test_tiles_equal_core_and_shell(n, times, viscous):
