@@ -1568,10 +1568,12 @@ __device__ __forceinline__ void rk_stage(const StageArgs<UT, CT>& a, const Stage
 // kernels last as long as one work-group: more waves than elements; the first
 // two own an element in the point-wise phases, and the faces of each direction
 // are another wave's, beside the volume RHS where this kernel forms it, so that
-// no wave does two things in a row that could be done at once.
+// no wave does two things in a row that could be done at once.  HOLD: a state of
+// another type than the fluxes' stays in registers (see kHoldTiles; in the strict
+// build it would cost them a wave per SIMD).
 template <class CT, bool VISC>
 constexpr int kWideWaves = UpdateLds<CT, VISC>::kVol ? 5 : 3;
-template <class UT, class CT, bool VISC, bool WIDE = false>
+template <class UT, class CT, bool VISC, bool WIDE = false, bool HOLD = false>
 __device__ __forceinline__ void update_body(const StageArgs<UT, CT>& a, const Tile& tl, UpdateLds<CT, VISC>& L,
                                             int wave, int pt) {
     constexpr bool PF = std::is_same<CT, float>::value;
@@ -1590,6 +1592,8 @@ __device__ __forceinline__ void update_body(const StageArgs<UT, CT>& a, const Ti
     }
 
     constexpr bool SAME = std::is_same<UT, CT>::value;  // sU holds the state exactly
+    static_assert(!(SAME && HOLD), "sU holds it");
+    UT held[HOLD ? 5 : 1];
     if constexpr (SAME && PF) {  // f32 state and compute: LDS-DMA
         if (mine) {
             load_state_tile(a.uin, NP, tile_eidx(tl, wave), L.sU[wave], pt);
@@ -1599,7 +1603,11 @@ __device__ __forceinline__ void update_body(const StageArgs<UT, CT>& a, const Ti
         }
     } else if (owner) {
 #pragma unroll
-        for (int v = 0; v < 5; ++v) L.sU[wave][v][pt] = (CT)(mine ? a.uin[v * NP + gbase] : (UT)1);
+        for (int v = 0; v < 5; ++v) {
+            const UT x = mine ? a.uin[v * NP + gbase] : (UT)1;
+            if constexpr (HOLD) held[v] = x;
+            L.sU[wave][v][pt] = (CT)x;
+        }
     }
     coef_store<CT>((int)threadIdx.x, cf);
 #if OD_FAST
@@ -1667,10 +1675,11 @@ __device__ __forceinline__ void update_body(const StageArgs<UT, CT>& a, const Ti
     CT r[5];
 #pragma unroll
     for (int v = 0; v < 5; ++v) {
-        // the state in its own type: from LDS, or again from L2 (held in f64
-        // from the start it cost the f32 fluxes a wave per SIMD)
+        // the state in its own type: from LDS, held, or again from L2
         if constexpr (SAME)
             ucr[v] = (UT)L.sU[wave][v][pt];
+        else if constexpr (HOLD)
+            ucr[v] = held[v];
         else
             ucr[v] = mine ? a.uin[v * NP + gbase] : (UT)1;
         if constexpr (VOL)
@@ -1746,11 +1755,11 @@ constexpr int kMinWaves = sizeof(CT) == 4 ? 4 : 1;
 template <class UT, class CT>
 constexpr int kMinWavesUpdate = (OD_FAST && sizeof(UT) == 4 && sizeof(CT) == 4) ? 8 : kMinWaves<CT>;
 
-template <class UT, class CT, bool VISC, bool WIDE>
+template <class UT, class CT, bool VISC, bool WIDE, bool HOLD>
 __global__ __launch_bounds__((64 * (WIDE ? kWideWaves<CT, VISC> : kEpb))) __attribute__((amdgpu_waves_per_eu(kMinWavesUpdate<UT, CT>))) void od_update_kernel(
     StageArgs<UT, CT> a) {
     __shared__ UpdateLds<CT, VISC> L;
-    update_body<UT, CT, VISC, WIDE>(a, make_tile_reversed(a), L, wave_index(), threadIdx.x & 63);
+    update_body<UT, CT, VISC, WIDE, HOLD>(a, make_tile_reversed(a), L, wave_index(), threadIdx.x & 63);
 }
 
 // LDS area of one element in the kernels that work by lines: [5][64] or
@@ -3346,14 +3355,32 @@ int launch_visc(const StageArgs<UT, CT>& a, int64_t n_elem, void* stream) {
 template <class CT, bool VISC>
 constexpr int64_t kWideTiles = 256 * (UpdateLds<CT, VISC>::kVol ? 2 : 4);
 
+// Tiles above which the fast kernel with an f64 state holds that state in registers
+// from its first load instead of loading it again for the blend.  Held it takes 70
+// to 72 VGPRs, 7 waves per SIMD; loaded again 64, 8 waves, at which 4096 tiles are
+// resident at once: up to there the second load is the smaller cost, above it the
+// state's traffic counts.  us a step, loaded again and held: Euler 20^3 (4000 tiles)
+// 61 69, 20x20x21 (4200) 73.7 71.8, 40^3 408 377; viscous 2x48x48 (2304) 84 88, 21^3
+// (4851) 145 140, 40^3 784 747.
+constexpr int64_t kHoldTiles = 4096;
+
 template <class UT, class CT, bool VISC>
 int launch_update(const StageArgs<UT, CT>& a, int64_t n_elem, void* stream) {
     const dim3 g = grid_of(a);
-    if ((int64_t)g.x * g.y * g.z <= kWideTiles<CT, VISC>)
-        hipLaunchKernelGGL((od_update_kernel<UT, CT, VISC, true>), g, dim3(64 * kWideWaves<CT, VISC>), 0,
+    const int64_t tiles = (int64_t)g.x * g.y * g.z;
+    if (tiles <= kWideTiles<CT, VISC>) {
+        hipLaunchKernelGGL((od_update_kernel<UT, CT, VISC, true, false>), g, dim3(64 * kWideWaves<CT, VISC>), 0,
                            (hipStream_t)stream, a);
-    else
-        hipLaunchKernelGGL((od_update_kernel<UT, CT, VISC, false>), g, dim3(64 * kEpb), 0, (hipStream_t)stream, a);
+        return check_launch();
+    }
+    if constexpr (OD_FAST && !std::is_same<UT, CT>::value) {
+        if (tiles > kHoldTiles) {
+            hipLaunchKernelGGL((od_update_kernel<UT, CT, VISC, false, true>), g, dim3(64 * kEpb), 0,
+                               (hipStream_t)stream, a);
+            return check_launch();
+        }
+    }
+    hipLaunchKernelGGL((od_update_kernel<UT, CT, VISC, false, false>), g, dim3(64 * kEpb), 0, (hipStream_t)stream, a);
     return check_launch();
 }
 
