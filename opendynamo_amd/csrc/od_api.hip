@@ -118,19 +118,17 @@ int launch_block_form(const od::StageArgs<float, float>& a, bool viscous, int ki
                    : od::fastmath::launch_update_core_shell<false>(a, stream);
 }
 
-od_status cfl_dt_of_state(const void* u, int u_real, int64_t E, double dx, double dy, double dz, double cfl,
-                          double* partial, hipStream_t stream, double* dt_out) {
+od_status enqueue_cfl(const void* u, int u_real, int64_t E, double dx, double dy, double dz, double* partial,
+                      hipStream_t stream) {
     const int rc = u_real == OD_F32 ? od::launch_cfl<float>((const float*)u, partial, E, dx, dy, dz, stream)
                                     : od::launch_cfl<double>((const double*)u, partial, E, dx, dy, dz, stream);
-    if (rc) return fail(OD_ERR_HIP, "od_cfl_kernel launch failed");
-    double h[od::kCflGroups];
-    const int groups = od::cfl_groups(E);
-    HIP_TRY(hipMemcpyAsync(h, partial, groups * sizeof(double), hipMemcpyDeviceToHost, stream));
-    HIP_TRY(hipStreamSynchronize(stream));
+    return rc ? fail(OD_ERR_HIP, "od_cfl_kernel launch failed") : OD_OK;
+}
+
+double cfl_dt(const double* partial, int groups, double cfl) {
     double lam = 0.0;
-    for (int q = 0; q < groups; ++q) lam = std::fmax(lam, h[q]);
-    *dt_out = (double)(float)(cfl / (7.0 * lam));
-    return OD_OK;
+    for (int q = 0; q < groups; ++q) lam = std::fmax(lam, partial[q]);
+    return (double)(float)(cfl / (7.0 * lam));
 }
 
 }  // namespace od::host
@@ -607,8 +605,15 @@ od_status od_cfl_dt(od_ctx* c, double cfl, double* dt_out) {
     if (!c || !dt_out) return fail(OD_ERR_INVALID, "od_cfl_dt: null argument");
     if (!(cfl > 0.0)) return fail(OD_ERR_INVALID, "od_cfl_dt: cfl must be positive");
     HIP_TRY(hipSetDevice(c->device));
-    return cfl_dt_of_state(c->u[0], c->p.u_real, c->E, c->p.lx / c->p.nx, c->p.ly / c->p.ny, c->p.lz / c->p.nz, cfl,
-                           c->cfl_partial, c->stream, dt_out);
+    od_status s = enqueue_cfl(c->u[0], c->p.u_real, c->E, c->p.lx / c->p.nx, c->p.ly / c->p.ny, c->p.lz / c->p.nz,
+                              c->cfl_partial, c->stream);
+    if (s != OD_OK) return s;
+    double h[od::kCflGroups];
+    const int groups = od::cfl_groups(c->E);
+    HIP_TRY(hipMemcpyAsync(h, c->cfl_partial, groups * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    *dt_out = cfl_dt(h, groups, cfl);
+    return OD_OK;
 }
 
 od_status od_time_steps(od_ctx* c, double dt, uint32_t n_steps, double* ms_total) {

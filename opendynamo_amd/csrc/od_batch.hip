@@ -36,7 +36,7 @@ struct od_batch {
     size_t table_bytes = 0;
     double* sums_partial = nullptr;  // [5][largest box], then (one allocation):
     double* sums_out = nullptr;      // 8 doubles
-    double* cfl_partial = nullptr;   // od::kCflGroups doubles
+    double* cfl_partial = nullptr;   // od::cfl_groups doubles of each box
     HostOps ops;
     od::BoxOps* box_ops = nullptr;  // per box: the fast kernels' operators
     std::vector<char> state_set;
@@ -462,13 +462,15 @@ od_status od_batch_create(const od_params* p, const od_box* boxes, int32_t n_box
     ok = ok && (!p->viscous || dmalloc(&b->fv, (size_t)E * od::fv_stride(fast_kernels(*p)) * b->cbytes));
     b->table_bytes = (size_t)n_boxes * sizeof(od::BoxDev<double, double>);
     ok = ok && dmalloc(&b->table, b->table_bytes);
+    size_t cfl_doubles = 0;
+    for (int i = 0; i < n_boxes; ++i) cfl_doubles += od::cfl_groups((int64_t)boxes[i].nx * boxes[i].ny * boxes[i].nz);
     const size_t ops_doubles = (size_t)n_boxes * sizeof(od::BoxOps) / sizeof(double);
     ok = ok && dmalloc((void**)&b->sums_partial,
-                       ((size_t)5 * max_box + 8 + od::kCflGroups + ops_doubles) * sizeof(double));
+                       ((size_t)5 * max_box + 8 + cfl_doubles + ops_doubles) * sizeof(double));
     if (ok) {
         b->sums_out = b->sums_partial + (size_t)5 * max_box;
         b->cfl_partial = b->sums_out + 8;
-        b->box_ops = (od::BoxOps*)(b->cfl_partial + od::kCflGroups);
+        b->box_ops = (od::BoxOps*)(b->cfl_partial + cfl_doubles);
     }
     if (!ok) return cleanup(fail(OD_ERR_NOMEM, "device allocation failed"));
     std::vector<od::BoxOps> ops;
@@ -572,13 +574,21 @@ od_status od_batch_cfl_dt(od_batch* b, double cfl, double* dt_out) {
     if (!b || !dt_out) return fail(OD_ERR_INVALID, "od_batch_cfl_dt: null argument");
     if (!(cfl > 0.0)) return fail(OD_ERR_INVALID, "od_batch_cfl_dt: cfl must be positive");
     HIP_TRY(hipSetDevice(b->device));
+    // every box's launch, then one copy and one wait for all of them
+    std::vector<int> first(b->boxes.size() + 1, 0);
     for (size_t i = 0; i < b->boxes.size(); ++i) {
         const od_box& x = b->boxes[i];
+        const int64_t E = (int64_t)x.nx * x.ny * x.nz;
         const unsigned char* u = (const unsigned char*)b->u[0] + (size_t)320 * b->e_off[i] * b->ubytes;
-        od_status s = cfl_dt_of_state(u, b->p.u_real, (int64_t)x.nx * x.ny * x.nz, x.lx / x.nx, x.ly / x.ny,
-                                      x.lz / x.nz, cfl, b->cfl_partial, b->stream, dt_out + i);
+        od_status s = enqueue_cfl(u, b->p.u_real, E, x.lx / x.nx, x.ly / x.ny, x.lz / x.nz, b->cfl_partial + first[i],
+                                  b->stream);
         if (s != OD_OK) return s;
+        first[i + 1] = first[i] + od::cfl_groups(E);
     }
+    std::vector<double> h(first.back());
+    HIP_TRY(hipMemcpyAsync(h.data(), b->cfl_partial, h.size() * sizeof(double), hipMemcpyDeviceToHost, b->stream));
+    HIP_TRY(hipStreamSynchronize(b->stream));
+    for (size_t i = 0; i < b->boxes.size(); ++i) dt_out[i] = cfl_dt(h.data() + first[i], first[i + 1] - first[i], cfl);
     return OD_OK;
 }
 

@@ -179,10 +179,11 @@ od::StageArgs<UT, CT> make_stage_args(const od_params& p, int nx, int ny, int nz
     return a;
 }
 
-// dt = cfl / ((2P+1) max_points sum_d (|u_d| + c) / dx_d), rounded to f32, of a
-// state [5][64 E] on the device; partial: od::kCflGroups doubles there.  Waits
-// for the stream.
-od_status cfl_dt_of_state(const void* u, int u_real, int64_t E, double dx, double dy, double dz, double cfl,
-                          double* partial, hipStream_t stream, double* dt_out);
+// dt = cfl / ((2P+1) max_points sum_d (|u_d| + c) / dx_d), rounded to f32: the
+// launch for a state [5][64 E] on the device, which leaves the maxima of
+// od::cfl_groups(E) groups in partial, and the dt from those, on the host.
+od_status enqueue_cfl(const void* u, int u_real, int64_t E, double dx, double dy, double dz, double* partial,
+                      hipStream_t stream);
+double cfl_dt(const double* partial, int groups, double cfl);
 
 }  // namespace od::host
