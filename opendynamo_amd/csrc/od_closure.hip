@@ -517,7 +517,8 @@ constexpr int kPartialRow = (NPARAM + 1 + 31) / 32 * 32;  // floats; rows start 
 // tiles of the (gathered) batch -> partial[gw][NPARAM + 1] (last entry: sum of
 // the squared errors).  Loss = mean over the batch of (C - t)^2.  At most 1024
 // groups (four to a CU: all resident), each with the next tile's inputs on the
-// way while it works on this one's.
+// way while it works on this one's.  At the 128 VGPRs that four waves per SIMD
+// leave it, 60 registers are spilled (236 bytes a lane).
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void od_mlp_grad_kernel(
     DevNet net, Scaling sc, const float* __restrict__ x, const float* __restrict__ tgt, const int* __restrict__ idx,
     int64_t n, int tiles_per_group, float* __restrict__ partial) {

@@ -105,8 +105,9 @@ __device__ __forceinline__ C sq(C x) {
 //        zeros, infinities and NaN their IEEE results; |a| between 0 and 2^-969
 //        may be off by one unit in the last place, and b below 2^-1022 or above
 //        2^1021, whose reciprocal is not a normal number, is not covered.
-// A division takes 46 (f32) and 65 (f64) cycles of a SIMD, a quotient 14 and
-// 20, a reciprocal 37; a point has about 90 quotients by some ten
+// A division takes 46 (f32) and 65 (f64) cycles of a SIMD, a quotient 14 (f32,
+// without the clearing, one instruction more: 48^3 visc 1267 -> 1320 instructions a
+// wave, 235 -> 245 us) and 20, a reciprocal 37; a point has about 90 quotients by some ten
 // denominators, which were nearly half of the strict kernels' instructions.
 template <class C>
 struct Recip {
@@ -1746,7 +1747,7 @@ __global__ __launch_bounds__(128) void od_visc_kernel(StageArgs<UT, CT> a) {
 
 // Occupancy target of the update kernels.  The fast all-f32 single-box kernel
 // and the batch kernel's single-unit form are held to 64 VGPRs (8 waves per
-// SIMD; they need 53 to 57 with no spills; their LDS, 9.6 KB per work-group of
+// SIMD; they need 51 to 59 with no spills; their LDS, 9.6 KB per work-group of
 // 128 threads, allows 8).  The strict build (70 VGPRs, 7 waves), f64 states and
 // the persistent batch kernel keep their natural allocation (the 4-wave cap does
 // not bind); f64 compute needs 115 to 122 VGPRs (4 waves).
